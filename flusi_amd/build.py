@@ -18,8 +18,8 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(ROOT, "_build")
 LIB = os.path.join(HERE, "libflusi_hip.so")
-SOURCES = ["passes.hip", "tiles_wave.hip", "zstep.hip", "xrhs_wave.hip", "fields.hip", "adjoint.hip", "solver.hip",
-           "host_params.cpp", "h5bind.cc"]
+SOURCES = ["zstep.hip:0", "zstep.hip:1", "zstep.hip:2", "zstep.hip:3", "passes.hip", "tiles_wave.hip", "xrhs_wave.hip",
+           "fields.hip", "adjoint.hip", "solver.hip", "host_params.cpp", "h5bind.cc"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("FLUSI_OFFLOAD_ARCH", "gfx950")
 FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
@@ -29,7 +29,8 @@ FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
 
 
 def _compile(src: str) -> str:
-    obj = os.path.join(BUILD, os.path.splitext(src)[0] + ".o")
+    src, _, part = src.partition(":")  # "file:n": part n of a source split for compile time
+    obj = os.path.join(BUILD, os.path.splitext(src)[0] + part + ".o")
     if src.endswith(".cc"):  # host-only C++ (dlopen of the HDF5 layer), no device pass
         cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-c", os.path.join(CSRC, src), "-o", obj]
         r = subprocess.run(cmd, capture_output=True, text=True)
@@ -39,6 +40,8 @@ def _compile(src: str) -> str:
     cmd = [HIPCC, *FLAGS]
     if src.endswith(".cpp"):
         cmd += ["-x", "hip"]
+    if part:
+        cmd += [f"-DFLUSI_PART={part}"]
     cmd += ["-c", os.path.join(CSRC, src), "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
@@ -46,7 +49,7 @@ def _compile(src: str) -> str:
     return obj
 
 
-def build(force: bool = True, jobs: int = 4) -> str:
+def build(force: bool = True, jobs: int = 8) -> str:
     """Compile every HIP source and link the shared library; returns its path."""
     if shutil.which(HIPCC) is None and not os.path.exists(HIPCC):
         raise RuntimeError(f"hipcc not found at {HIPCC}")

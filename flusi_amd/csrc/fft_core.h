@@ -61,6 +61,31 @@ template <typename T> __device__ __forceinline__ void gst(gptr<cplx<T>> p, cplx<
 template <typename T> __device__ __forceinline__ cplx<T> twv(const cplx<T>* __restrict__ p, int i) { return p[i]; }
 template <typename T> __device__ __forceinline__ cplx<T> twv(gptr<const cplx<T>> p, int i) { return gld<T>(p + i); }
 
+// ------------------------------------------------------------ buffer access
+// Complex elements through a buffer descriptor: 32-bit byte offsets from a
+// wave-uniform base, and an offset at or beyond the descriptor's size reads
+// zero and stores nothing.  A structural zero (a mode outside the dealiased
+// region, a line beyond the tile axis) is therefore the offset kOob instead
+// of a branch or a select, costs no memory traffic, and leaves every access
+// of a pass unconditional.  A field (at most 2^30 + padding bytes: 512^3 FP64)
+// stays below kOob; the hosts check it (buffer_bytes).
+using brsrc = __amdgpu_buffer_rsrc_t;
+constexpr unsigned kOob = 0x80000000u;
+__device__ __forceinline__ brsrc make_brsrc(const void* p, unsigned bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
+}
+using bword2 = unsigned __attribute__((ext_vector_type(2)));
+using bword4 = unsigned __attribute__((ext_vector_type(4)));
+// AUX: 2 = non-temporal, 0 = ordinary caching
+template <typename T, int AUX = 2> __device__ __forceinline__ cplx<T> bld(brsrc r, unsigned off) {
+  if constexpr (sizeof(T) == 4) return __builtin_bit_cast(cplx<T>, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, AUX));
+  else return __builtin_bit_cast(cplx<T>, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, AUX));
+}
+template <typename T, int AUX = 2> __device__ __forceinline__ void bst(brsrc r, unsigned off, cplx<T> v) {
+  if constexpr (sizeof(T) == 4) __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(bword2, v), r, off, 0, AUX);
+  else __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(bword4, v), r, off, 0, AUX);
+}
+
 // ---------------------------------------------------------------- LDS padding
 template <typename T> struct Pad { static constexpr int PS = (sizeof(T) == 4) ? 4 : 3; };
 template <typename T> __host__ __device__ constexpr int lp(int a) { return a + (a >> Pad<T>::PS); }

@@ -24,6 +24,27 @@ struct Batch {
 };
 __host__ __device__ __forceinline__ int batch_n(const Batch& b) { return b.nmem > 1 ? b.nmem : 1; }
 
+// Dealiased ("pruned") passes.  With dealiasing every stepper writes zero to
+// the modes outside the ellipsoid (kx/Kx)^2 + (ky/Ky)^2 + (kz/Kz)^2 < 1,
+// K = 2/3 (n/2 - 1) (vis.f90:23-53): 15 % of the half spectrum is left, its
+// (kx, ky) shadow is 35 %, its kx range 2/3.  The pruned passes move and
+// transform only what those modes need and what they produce.  Their Q layout
+// is compact: row position p holds ky = p - ym0, nyp positions a row.
+struct Prune {
+  int ym0;                 // largest |ky| of the region
+  int nyp;                 // Q row length: 2 ym0 + 1 rounded up to whole 128-byte lines
+  int nkx;                 // kx = 0..nkx-1 hold the region
+  const int16_t* ylim;     // per kx (nkx): largest |ky|
+  const int16_t* zlim;     // per (kx, p) (nkx x nyp): largest |kz|, -1 outside
+};
+// the passes' use of the region
+enum PruneMode {
+  PR_NONE = 0,
+  PR_ZINV = 1,   // state rows inside the region -> compact Q rows
+  PR_YINV = 2,   // compact Q rows -> P, kx < nkx
+  PR_YFWD = 3,   // P, kx < nkx -> the compact Q rows' region (whole 128-byte lines of it)
+};
+
 enum TileOp { OP_COPY = 0, OP_DERIV = 1, OP_DERIV_MINUS = 2 };
 
 // One job reads its operands once and writes one or two transforms of them.
@@ -48,6 +69,11 @@ struct TilePassArgs {
   double scale;        // applied to every stored value
   const void* tw;      // L twiddles exp(-2 pi i m / L), element type of the pass
   int pf;              // block passes: load the next job's operand while the current one is transformed
+  unsigned ibytes, obytes;  // bytes of one input / output field (buffer descriptors)
+  int prune;           // PruneMode
+  Prune pr;
+  const uint32_t* tiles;  // PR_ZINV: (c << 16 | first line / TL) per workgroup, ntiles of them
+  int ntiles;
   Batch bat;           // grid z: member
 };
 
@@ -66,7 +92,9 @@ struct XPassArgs {
   int nf;              // fields for XM_INV / XM_FWD
   int nlines;          // ny*nz
   int nx, ny, nxh;
-  long prow;           // row stride of the spectral (P-layout) side, >= nxh
+  long prow;           // row stride of the spectral (P-layout) side
+  int kin, kout;       // spectral entries read (the others are zero) and written per line
+  unsigned fbytes;     // bytes of one P field (buffer descriptor)
   const double* kx;    // nxh wavenumbers
   double kx_scale;     // kx = kx_scale * k
   int wpe;             // one-wave-per-line RHS pass: register budget for 3 waves per SIMD (3) or none (0)
@@ -145,6 +173,13 @@ struct ZStepArgs {
   double* energy_partial;  // per block Parseval partial sum (final stages only)
   int wave;              // 1: transform each z line inside one wavefront (nz = 64..512)
   int eu;                // block kernel, nz >= 256: epilogue positions scheduled together (0 = all)
+  // prune & 1: the state operands are zero outside the dealiased region and
+  // are not read there; prune & 2: the result is, too - Q is compact and only
+  // the region (its whole 128-byte lines) is transformed and written
+  int prune;
+  Prune pr;
+  const uint32_t* tiles;  // prune & 2: (kx << 16 | first line / TL) per workgroup, ntiles of them
+  int ntiles;
   Batch bat;             // grid z: member
 };
 
@@ -165,6 +200,9 @@ int x_rhs_wave_blocks(int nx, int nlines);
 // mask value of the line is nonzero, else 0 (xrhs_wave.hip)
 template <typename T>
 void launch_mask_flags(const void* mask, uint8_t* flag, int nx, int ny, int y0, int y1, int z0, int z1, hipStream_t s);
+// lines per workgroup of the pruned z passes: the tile lists are built for them
+int tile_lines(bool fp64);                                  // z inverse
+int zstep_tile_lines(int nz, bool fp64, bool wave);
 // energy partial sums one z-step launch writes per member (the block kernel
 // or, wave = true, the in-wave kernel)
 int zstep_blocks(int nz, int ny, int nxh, bool fp64, bool wave);

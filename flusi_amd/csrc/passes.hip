@@ -44,11 +44,16 @@ __global__ __launch_bounds__(NT) void tile_pass_k(TilePassArgs a) {
   constexpr int LSP = line_stride<T>(L);
   constexpr int NB0 = TL * (L / R0), PER0 = (NB0 + NT - 1) / NT;
   constexpr int NBL = TL * (L / RL), PERL = (NBL + NT - 1) / NT;
+  constexpr unsigned ES = sizeof(cplx<T>);
   extern __shared__ char smem_raw[];
   cplx<T>* buf = reinterpret_cast<cplx<T>*>(smem_raw);
   const int tid = threadIdx.x;
-  const int b0 = blockIdx.x * TL;
-  const long c = blockIdx.y;
+  int b0 = blockIdx.x * TL, c = blockIdx.y;
+  if (a.tiles) {  // the tiles that meet the dealiased region
+    const uint32_t t = ((gptr<const uint32_t>)a.tiles)[blockIdx.x];
+    b0 = (int)(t & 0xffffu) * TL;
+    c = (int)(t >> 16);
+  }
   const long moff = (long)blockIdx.z * a.bat.mstride;  // batch member's slab
   // global-address-space views of the arguments (see gptr)
   const gptr<const cplx<T>> tw = (gptr<const cplx<T>>)mshift(a.tw, moff);
@@ -57,7 +62,7 @@ __global__ __launch_bounds__(NT) void tile_pass_k(TilePassArgs a) {
   cplx<T> r0[PER0][R0], r1[PER0][R0];
   // operand `which` (0: in0, prefetched; 1: in1, read when its job starts)
   auto load = [&](int jb, int which) {
-    const gptr<const cplx<T>> in = (gptr<const cplx<T>>)mshift(which ? a.jobs[jb].in1 : a.jobs[jb].in0, moff);
+    const brsrc in = make_brsrc(mshift(which ? a.jobs[jb].in1 : a.jobs[jb].in0, moff), a.ibytes);
 #pragma unroll
     for (int p = 0; p < PER0; ++p) {
       const int beta = tid + p * NT;
@@ -65,14 +70,34 @@ __global__ __launch_bounds__(NT) void tile_pass_k(TilePassArgs a) {
         int bb, j;
         if (CONTIG_IN) { bb = beta / (L / R0); j = beta - bb * (L / R0); }
         else { bb = beta % TL; j = beta / TL; }
-        const bool ok = b0 + bb < a.nb;
-        // the contiguous side has unit stride (checked on the host)
-        const long base = CONTIG_IN ? c * a.sin.c + (long)(b0 + bb) * a.sin.b + j
-                                    : c * a.sin.c + (long)(b0 + bb) + (long)j * a.sin.a;
-        const long step = CONTIG_IN ? (long)(L / R0) : (long)(L / R0) * a.sin.a;
+        // contiguous side (unit stride, checked on the host): the line's row,
+        // the largest |wave number| it holds and the element shifts of its
+        // halves (see tile_wave_k)
+        const int b = b0 + bb;
+        int lim = b < a.nb ? L : -1, row = b;
+        unsigned lo = 0, hi = 0;
+        if (CONTIG_IN && a.prune == PR_ZINV) {
+          lim = ((gptr<const int16_t>)a.pr.zlim)[c * a.pr.nyp + b];
+          row = b - a.pr.ym0;
+          if (row < 0) row += a.nb;
+        } else if (CONTIG_IN && a.prune == PR_YINV) {
+          lim = b < a.nb ? ((gptr<const int16_t>)a.pr.ylim)[b] : -1;
+          lo = a.pr.ym0;
+          hi = (unsigned)(a.pr.ym0 - L);
+        }
+        const unsigned base = CONTIG_IN ? (unsigned)c * (unsigned)a.sin.c + (unsigned)row * (unsigned)a.sin.b
+                                        : (unsigned)c * (unsigned)a.sin.c + (unsigned)b;
 #pragma unroll
         for (int q = 0; q < R0; ++q) {
-          const cplx<T> x = ok ? gld<T>(in + base + q * step) : mk<T>(T(0), T(0));
+          const int aa = j + q * (L / R0);
+          unsigned off;
+          if (CONTIG_IN) {
+            const bool up = aa >= L / 2;
+            off = (up ? L - aa : aa) <= lim ? (base + aa + (up ? hi : lo)) * ES : kOob;
+          } else {
+            off = lim >= 0 ? (base + (unsigned)aa * (unsigned)a.sin.a) * ES : kOob;
+          }
+          const cplx<T> x = bld<T, 0>(in, off);
           if (which) r1[p][q] = x;
           else r0[p][q] = x;
         }
@@ -87,7 +112,7 @@ __global__ __launch_bounds__(NT) void tile_pass_k(TilePassArgs a) {
     if (a.jobs[jb].in1) load(jb, 1);
     for (int o = 0; o < nout; ++o) {
       const int op = o ? a.jobs[jb].op2 : a.jobs[jb].op;
-      const gptr<cplx<T>> out = (gptr<cplx<T>>)mshift(o ? a.jobs[jb].out2 : a.jobs[jb].out, moff);
+      const brsrc out = make_brsrc(mshift(o ? a.jobs[jb].out2 : a.jobs[jb].out, moff), a.obytes);
       // FP32 at L >= 384: a copy of the thread index per transform, so that
       // the LDS addresses and twiddles are recomputed in each iteration of
       // the job loop instead of being kept live (spilled) across it
@@ -141,13 +166,29 @@ __global__ __launch_bounds__(NT) void tile_pass_k(TilePassArgs a) {
 #pragma unroll
           for (int q = 0; q < RL; ++q) w[q] = buf[bb * LSP + lp<T>(j + q * (L / RL))];
           twiddle_bfly<T, L, RL, S, NSL>(w, j, tw);
+          const int b = b0 + bb;
           // segment-side stores may cover the row padding (zeros; see nb_store)
-          if (b0 + bb < (CONTIG_IN && a.nb_store > a.nb ? a.nb_store : a.nb)) {
-            const long base = !CONTIG_IN ? c * a.sout.c + (long)(b0 + bb) * a.sout.b + j
-                                         : c * a.sout.c + (long)(b0 + bb) + (long)j * a.sout.a;
-            const long step = !CONTIG_IN ? (long)(L / RL) : (long)(L / RL) * a.sout.a;
+          const bool ok = b < (CONTIG_IN && a.nb_store > a.nb ? a.nb_store : a.nb);
+          const unsigned base = !CONTIG_IN ? (unsigned)c * (unsigned)a.sout.c + (unsigned)b * (unsigned)a.sout.b
+                                           : (unsigned)c * (unsigned)a.sout.c + (unsigned)b;
+          int plo = 0, phi = 0;  // PR_YFWD: compact positions written (see tile_wave_k)
+          if (!CONTIG_IN && a.prune == PR_YFWD) {
+            constexpr int SEG = 128 / ES;
+            const int ym = ok ? ((gptr<const int16_t>)a.pr.ylim)[b] : -1;
+            plo = (a.pr.ym0 - ym) & ~(SEG - 1);
+            phi = ok ? min(a.pr.nyp, ((a.pr.ym0 + ym) | (SEG - 1)) + 1) : 0;
+          }
 #pragma unroll
-            for (int q = 0; q < RL; ++q) gst<T>(out + base + q * step, mk<T>(w[q].x * sc, w[q].y * sc));
+          for (int q = 0; q < RL; ++q) {
+            const int aa = j + q * (L / RL);
+            unsigned off;
+            if (!CONTIG_IN && a.prune == PR_YFWD) {
+              const int pp = a.pr.ym0 + (aa < L / 2 ? aa : aa - L);
+              off = pp >= plo && pp < phi ? (base + (unsigned)pp) * ES : kOob;
+            } else {
+              off = ok ? (base + (CONTIG_IN ? (unsigned)aa * (unsigned)a.sout.a : (unsigned)aa)) * ES : kOob;
+            }
+            bst<T, 0>(out, off, mk<T>(w[q].x * sc, w[q].y * sc));
           }
         }
       }
@@ -163,7 +204,7 @@ static void run_tile_pf(const TilePassArgs& a, hipStream_t s) {
   const size_t smem = sizeof(cplx<T>) * TL * line_stride<T>(L);
   static bool init = false;
   if (!init) { set_smem(tile_pass_k<T, L, TL, NT, S, CI, PF>, smem); init = true; }
-  dim3 grid((a.nb + TL - 1) / TL, a.nc, batch_n(a.bat));
+  const dim3 grid = a.tiles ? dim3(a.ntiles, 1, batch_n(a.bat)) : dim3((a.nb + TL - 1) / TL, a.nc, batch_n(a.bat));
   hipLaunchKernelGGL((tile_pass_k<T, L, TL, NT, S, CI, PF>), grid, dim3(NT), smem, s, a);
 }
 template <typename T, int L, int S, bool CI>
@@ -199,6 +240,7 @@ void launch_tile_pass(const TilePassArgs& a, int L, int dir, bool ci, hipStream_
   const bool unit = ci ? (a.sin.a == 1 && a.sout.b == 1) : (a.sin.b == 1 && a.sout.a == 1);
   if (!unit) throw std::runtime_error("tile pass: the contiguous axes must have unit stride");
   if (a.njobs < 1 || a.njobs > 6) throw std::runtime_error("tile pass: 1..6 jobs");
+  if (a.ibytes >= kOob || a.obytes >= kOob) throw std::runtime_error("tile pass: field too large for 32-bit offsets");
   switch (L) {
     case 16: run_tile_dir<T, 16>(a, dir, ci, s); break;
     case 24: run_tile_dir<T, 24>(a, dir, ci, s); break;
@@ -266,7 +308,7 @@ __global__ __launch_bounds__(NT) void x_pass_k(XPassArgs a) {
         const int line = e / nxh, k = e - line * nxh;
         const int gl = l0 + line;
         cplx<T> v = mk<T>(T(0), T(0));
-        if (gl < a.nlines) v = gld<T>(in + f * a.fstride_in + (long)gl * a.prow + k);
+        if (gl < a.nlines && k < a.kin) v = gld<T>(in + f * a.fstride_in + (long)gl * a.prow + k);
         L_(f, line)[lp<T>(k)] = v;
       }
     __syncthreads();
@@ -500,8 +542,8 @@ __global__ __launch_bounds__(NT) void x_pass_k(XPassArgs a) {
       const cplx<T> zm = L_(f, line)[lp<T>(k2 == M ? 0 : k2)];
       const cplx<T> s1 = add(zk, conj_(zm)), d1 = sub(zk, conj_(zm));
       const gptr<cplx<T>> o = out + f * a.fstride_out + (long)gl * a.prow;
-      gst<T>(o + k, scl(sub(s1, ik_<T>(T(1), cmul(wa, d1))), half));
-      if (k2 != k) {
+      if (k < a.kout) gst<T>(o + k, scl(sub(s1, ik_<T>(T(1), cmul(wa, d1))), half));
+      if (k2 != k && k2 < a.kout) {
         const cplx<T> s2 = add(zm, conj_(zk)), d2 = sub(zm, conj_(zk));
         gst<T>(o + k2, scl(sub(s2, ik_<T>(T(1), cmul(wb, d2))), half));
       }

@@ -293,8 +293,19 @@ class Solver : public SolverBase {
   bool zwave = false;          // z-forward step pass with in-wave line transforms
   int zeu = 0;                 // block z step, nz >= 256: epilogue positions scheduled together (0 = all)
   double* fw_d = nullptr;     // Fourier wing radius table
+  // dealiased region (Prune) and the tiles of the z passes that meet it, per
+  // lines a tile (8, 16)
+  Prune pr{};
+  bool prune_ok = false;      // the grid's compact Q rows fit (FLUSI_PRUNE=0: off)
+  bool prune_any_size = false;  // FLUSI_PRUNE=1: also below the size where it pays (prunes())
+  uint32_t* ptiles[2] = {nullptr, nullptr};
+  int nptiles[2] = {0, 0};
+  long prowc = 0;             // P row stride of the passes pruned on both sides
+  // zero outside the dealiased region: the state, the two registers
+  bool uk_pruned = false, reg_pruned[2] = {false, false};
   bool xwave = false;       // right-hand-side x pass with one wavefront per line
   double* zpart = nullptr; int nzblocks = 0;
+  int nzpart = 0;           // partial sums the last z step wrote
   double* dpart = nullptr; int ndblocks = 0;
   double* noalloc_scratch = nullptr;  // device address of `scratch` on this context's GPU
   double* red = nullptr;    // small results
@@ -408,6 +419,7 @@ class Solver : public SolverBase {
     HIPCHECK(hipMemcpy(tab, h.data(), ntab * sizeof(double), hipMemcpyHostToDevice));
     kx_d = tab; ky_d = kx_d + nxh; kz_d = ky_d + ny; kxt2_d = kz_d + nz; kyt2_d = kxt2_d + nxh; kzt2_d = kyt2_d + ny;
     if (fft_ok) {
+      setup_prune();
       tw_z = make_tw(nz, nz); tw_y = make_tw(ny, ny); tw_M = make_tw(nx / 2, nx / 2); tw_N = make_tw(nxh, nx);
       if (const char* e = getenv("FLUSI_TILE_WAVE")) twave = atoi(e) != 0;
       if (const char* e = getenv("FLUSI_ZWAVE")) zwave = atoi(e) != 0;
@@ -438,6 +450,61 @@ class Solver : public SolverBase {
     kinds = (int*)dalloc(sizeof(int) * k.size());
     HIPCHECK(hipMemcpy(kinds, k.data(), sizeof(int) * k.size(), hipMemcpyHostToDevice));
     HIPCHECK(hipStreamSynchronize(stream));
+  }
+
+  // The dealiased region's tables, from the predicate the steppers evaluate
+  // (kxt2 + kyt2) + kzt2 < 1 in FP64; each term grows with |k|, so the region
+  // is an interval of every axis.
+  void setup_prune() {
+    const int seg = 128 / (int)sizeof(C);
+    auto last = [](int n, auto&& inside) { int m = -1; while (m + 1 < n && inside(m + 1)) ++m; return m; };
+    pr.nkx = 1 + last(nx / 2, [&](int k) { return (kxt2_h[k] + kyt2_h[0]) + kzt2_h[0] < 1.0; });
+    pr.ym0 = last(ny / 2, [&](int k) { return (kxt2_h[0] + kyt2_h[k]) + kzt2_h[0] < 1.0; });
+    pr.nyp = (2 * pr.ym0 + 1 + seg - 1) / seg * seg;
+    prowc = (pr.nkx + seg - 1) / seg * seg;
+    prune_ok = pr.nyp <= ny && prowc <= prow;
+    if (const char* e = getenv("FLUSI_PRUNE")) {
+      prune_ok = prune_ok && atoi(e) != 0;
+      prune_any_size = prune_ok;
+    }
+    std::vector<int16_t> yl(pr.nkx), zl((size_t)pr.nkx * pr.nyp, -1);
+    std::vector<uint32_t> tl[2];
+    for (int kx = 0; kx < pr.nkx; ++kx) {
+      yl[kx] = (int16_t)last(ny / 2, [&](int k) { return (kxt2_h[kx] + kyt2_h[k]) + kzt2_h[0] < 1.0; });
+      int zm = nz / 2;  // shrinks as |ky| grows
+      for (int ky = 0; ky <= yl[kx]; ++ky) {
+        while (!((kxt2_h[kx] + kyt2_h[ky]) + kzt2_h[zm] < 1.0)) --zm;
+        int16_t* row = zl.data() + (size_t)kx * pr.nyp + pr.ym0;
+        row[ky] = row[-ky] = (int16_t)zm;
+      }
+      // Tiles of 8 and of 16 lines.  Where two 8-line tiles share 128-byte
+      // lines (FP32) they sit 8 entries apart: workgroups are dealt
+      // round-robin to the 8 XCDs, so the pair runs on one XCD.
+      for (int v = 0; v < 2; ++v) {
+        const int TL = 8 << v, t0 = (pr.ym0 - yl[kx]) / TL, t1 = (pr.ym0 + yl[kx]) / TL;
+        std::vector<int> order;
+        if (v == 0 && seg == 16) {
+          for (int g = t0 / 2; g <= t1 / 2; g += 8)
+            for (int half = 0; half < 2; ++half)
+              for (int i = g; i < g + 8 && i <= t1 / 2; ++i) order.push_back(2 * i + half);
+        } else {
+          for (int t = t0; t <= t1; ++t) order.push_back(t);
+        }
+        for (int t : order)
+          if (t >= t0 && t <= t1) tl[v].push_back((uint32_t)kx << 16 | (uint32_t)t);
+      }
+    }
+    // (fixed sizes per grid: batch members' buffers keep one layout)
+    int16_t* y = (int16_t*)dalloc(sizeof(int16_t) * yl.size());
+    int16_t* z = (int16_t*)dalloc(sizeof(int16_t) * zl.size());
+    HIPCHECK(hipMemcpy(y, yl.data(), sizeof(int16_t) * yl.size(), hipMemcpyHostToDevice));
+    HIPCHECK(hipMemcpy(z, zl.data(), sizeof(int16_t) * zl.size(), hipMemcpyHostToDevice));
+    pr.ylim = y; pr.zlim = z;
+    for (int v = 0; v < 2; ++v) {
+      nptiles[v] = (int)tl[v].size();
+      ptiles[v] = (uint32_t*)dalloc(sizeof(uint32_t) * tl[v].size());
+      HIPCHECK(hipMemcpy(ptiles[v], tl[v].data(), sizeof(uint32_t) * tl[v].size(), hipMemcpyHostToDevice));
+    }
   }
 
   void* make_tw(int n, int period) {
@@ -492,37 +559,53 @@ class Solver : public SolverBase {
   }
   C* cfp(int f) { return reinterpret_cast<C*>(P) + (long)f * pc; }  // field f of P
 
-  void zinv(const TileJob* jobs, int nj) {  // S -> Q
+  // Pruned passes (in: the input is zero outside the dealiased region) read
+  // and write only what that region needs (see Prune).
+  unsigned sbytes() const { return (unsigned)(nc * sizeof(C)); }
+  unsigned pbytes() const { return (unsigned)(pc * sizeof(C)); }
+  long p_row = 0;  // P row stride of the current right-hand side (prow or prowc)
+  void zinv(const TileJob* jobs, int nj, bool in) {  // S -> Q
     TilePassArgs a{};
     for (int j = 0; j < nj; ++j) a.jobs[j] = jobs[j];
     a.njobs = nj; a.nb = ny; a.nc = nxh;
     a.sin = Strides{1, nz, (long)ny * nz};
     a.sout = Strides{ny, 1, (long)nz * ny};
+    if (in) {
+      const int v = tile_lines(FP64) == 16;
+      a.prune = PR_ZINV; a.pr = pr; a.tiles = ptiles[v]; a.ntiles = nptiles[v];
+      a.sout = Strides{pr.nyp, 1, (long)nz * pr.nyp};
+    }
+    a.ibytes = sbytes(); a.obytes = sbytes();
     a.kscale = ksz; a.scale = 1.0; a.tw = tw_z;
     timed(TM_ZINV, [&] { tile(a, nz, +1, true); });
     kcheck("zinv");
   }
-  void yinv(const TileJob* jobs, int nj) {  // Q -> P
+  // Q -> P with rows of p_row entries
+  void yinv(const TileJob* jobs, int nj, bool in) {
     TilePassArgs a{};
     for (int j = 0; j < nj; ++j) a.jobs[j] = jobs[j];
-    a.njobs = nj; a.nb = nxh; a.nc = nz;
+    a.njobs = nj; a.nb = in ? pr.nkx : nxh; a.nc = nz;
     // the last tile column stores whole 128-byte segments (zeros beyond nxh):
     // a store of the lone Nyquist value alone is a partial-line write that the
     // memory side turns into a read-modify-write (YINV at 512^3: 5.41 -> 4.70 ms
     // per RK4 step)
-    a.nb_store = (int)std::min<long>(prow, (nxh + 15) / 16 * 16);
-    a.sin = Strides{1, (long)nz * ny, ny};
-    a.sout = Strides{prow, 1, (long)ny * prow};
+    a.nb_store = (int)std::min<long>(p_row, (a.nb + 15) / 16 * 16);
+    a.sin = in ? Strides{1, (long)nz * pr.nyp, pr.nyp} : Strides{1, (long)nz * ny, ny};
+    a.sout = Strides{p_row, 1, (long)ny * p_row};
+    if (in) { a.prune = PR_YINV; a.pr = pr; }
+    a.ibytes = sbytes(); a.obytes = pbytes();
     a.kscale = ksy; a.scale = 1.0; a.tw = tw_y;
     timed(TM_YINV, [&] { tile(a, ny, +1, true); });
     kcheck("yinv");
   }
-  void yfwd(int nf) {  // P -> Q
+  void yfwd(int nf, bool out) {  // P -> Q
     TilePassArgs a{};
     for (int j = 0; j < nf; ++j) a.jobs[j] = TileJob{cfp(j), nullptr, cf(Q, j), OP_COPY, nullptr, 0};
-    a.njobs = nf; a.nb = nxh; a.nc = nz;
-    a.sin = Strides{prow, 1, (long)ny * prow};
-    a.sout = Strides{1, (long)nz * ny, ny};
+    a.njobs = nf; a.nb = out ? pr.nkx : nxh; a.nc = nz;
+    a.sin = Strides{p_row, 1, (long)ny * p_row};
+    a.sout = out ? Strides{1, (long)nz * pr.nyp, pr.nyp} : Strides{1, (long)nz * ny, ny};
+    if (out) { a.prune = PR_YFWD; a.pr = pr; }
+    a.ibytes = pbytes(); a.obytes = sbytes();
     a.kscale = ksy; a.scale = 1.0; a.tw = tw_y;
     timed(TM_YFWD, [&] { tile(a, ny, -1, false); });
     kcheck("yfwd");
@@ -533,13 +616,15 @@ class Solver : public SolverBase {
     a.njobs = nf; a.nb = ny; a.nc = nxh;
     a.sin = Strides{ny, 1, (long)nz * ny};
     a.sout = Strides{1, nz, (long)ny * nz};
+    a.ibytes = sbytes(); a.obytes = sbytes();
     a.kscale = ksz; a.scale = 1.0 / (double(nx) * double(ny) * double(nz)); a.tw = tw_z;
     timed(TM_ZSTEP, [&] { tile(a, nz, -1, false); });
     kcheck("zfwd");
   }
   XPassArgs xargs() {
     XPassArgs a{};
-    a.nlines = ny * nz; a.nx = nx; a.ny = ny; a.nz = nz; a.nxh = nxh; a.prow = prow;
+    a.nlines = ny * nz; a.nx = nx; a.ny = ny; a.nz = nz; a.nxh = nxh; a.prow = p_row;
+    a.kin = nxh; a.kout = nxh; a.fbytes = pbytes();
     a.kx = kx_d; a.kx_scale = 2.0 * PI / p.xl; a.twM = tw_M; a.twN = tw_N;
     a.npts = npts; a.wpe = xwpe;
     a.bat = bat;
@@ -548,13 +633,13 @@ class Solver : public SolverBase {
   // the five fields of the z-inverse pass and the six of the y-inverse pass:
   // Q: 0 U_x, 1 U_y, 2 U_z, 3 D_x = F_z^-1(i kz u_x), 4 D_y = F_z^-1(i kz u_y)
   // P: 0 V_x, 1 V_y, 2 V_z, 3 w_x, 4 dz u_x, 5 dy u_x
-  void inv_uw(const void* u_in) {
+  void inv_uw(const void* u_in, bool in) {
     const C* u = reinterpret_cast<const C*>(u_in);
     // each operand is read once: u_x gives U_x and D_x, u_y gives U_y and D_y
     TileJob zj[3] = {{u, nullptr, cf(Q, 0), OP_COPY, cf(Q, 3), OP_DERIV},
                      {u + nc, nullptr, cf(Q, 1), OP_COPY, cf(Q, 4), OP_DERIV},
                      {u + 2 * nc, nullptr, cf(Q, 2), OP_COPY, nullptr, 0}};
-    zinv(zj, 3);
+    zinv(zj, 3, in);
     // (U_z, D_y) give V_z and w_x; U_x gives V_x and dy u_x.  The two-operand
     // job goes first: both its reads start with the kernel, the later jobs'
     // reads are prefetched behind the transforms
@@ -562,7 +647,7 @@ class Solver : public SolverBase {
                      {cf(Q, 0), nullptr, cfp(0), OP_COPY, cfp(5), OP_DERIV},
                      {cf(Q, 1), nullptr, cfp(1), OP_COPY, nullptr, 0},
                      {cf(Q, 3), nullptr, cfp(4), OP_COPY, nullptr, 0}};
-    yinv(yj, 4);
+    yinv(yj, 4, in);
   }
 
   int sponge_code() const {
@@ -573,12 +658,17 @@ class Solver : public SolverBase {
   }
 
   // rhs.f90:2-115 up to the forward transform: mask, inverse passes, x pass,
-  // and the reduction of max|u|^2 and sum chi (u - us) into red[0..3]
-  void pre_rhs(const void* u_in, double t, bool with_mask = true) {
+  // and the reduction of max|u|^2 and sum chi (u - us) into red[0..3].  in:
+  // u_in is zero outside the dealiased region; out: only the result's modes
+  // inside it are used (post_rhs with prune & 2).
+  void pre_rhs(const void* u_in, double t, bool with_mask = true, bool in = false, bool out = false) {
     if (with_mask && p.iMoving == 1 && p.iPenalization == 1) create_mask(t);
     if (p.eps < 1.0e-11) throw FlusiError(77363800, "Value of eps is very small, maybe even zero.");
-    inv_uw(u_in);
+    p_row = in && out ? prowc : prow;
+    inv_uw(u_in, in);
     XPassArgs a = xargs();
+    if (in) a.kin = pr.nkx;
+    if (out) a.kout = (int)std::min<long>(prowc, nxh);
     a.in = P; a.out = P; a.fstride_in = pc; a.fstride_out = pc; a.nf = 6;
     a.mask = mask; a.us = us; a.eps_inv = 1.0 / p.eps;
     a.mflag = mflag_valid ? mflag : nullptr; a.mzero = mzero;
@@ -623,7 +713,13 @@ class Solver : public SolverBase {
     return z;
   }
   void post_rhs(ZStepArgs& z) {
-    yfwd(z.sponge ? 6 : 3);
+    if (z.prune) z.pr = pr;
+    if (z.prune & 2) {
+      const int v = zstep_tile_lines(nz, FP64, zwave) == 16;
+      z.tiles = ptiles[v]; z.ntiles = nptiles[v];
+    }
+    yfwd(z.sponge ? 6 : 3, (z.prune & 2) != 0);
+    nzpart = z.tiles ? z.ntiles : zstep_blocks(nz, ny, nxh, FP64, zwave);
     const bool fin = z.mode == SM_EULER || z.mode == SM_AB2 || z.mode == SM_RK2_2 || z.mode == SM_RK4_4;
     if (fin) {
       // set_mean_flow (fluid_time_step.f90:1066-1090) with the time of the step start
@@ -680,7 +776,7 @@ class Solver : public SolverBase {
   // for every member after the step)
   void record_ekin(bool force = false) {
     if (out_dir.empty() || (ens_step && !force)) return;
-    launch_reduce_rows(zpart, zstep_blocks(nz, ny, nxh, FP64, zwave), 1, kinds + 4, rmid, red + 8, stream);
+    launch_reduce_rows(zpart, nzpart, 1, kinds + 4, rmid, red + 8, stream);
     double e = 0.0;
     HIPCHECK(hipMemcpyAsync(&e, red + 8, sizeof(double), hipMemcpyDeviceToHost, stream));
     HIPCHECK(hipStreamSynchronize(stream));
@@ -692,7 +788,7 @@ class Solver : public SolverBase {
   // NaN or Inf anywhere makes it non-finite)
   void check_nan() override {
     need_fft();
-    launch_reduce_rows(zpart, zstep_blocks(nz, ny, nxh, FP64, zwave), 1, kinds + 4, rmid, red + 10, stream);
+    launch_reduce_rows(zpart, nzpart, 1, kinds + 4, rmid, red + 10, stream);
     kcheck("checknan");
     double e = 0.0;
     HIPCHECK(hipMemcpyAsync(&e, red + 10, sizeof(double), hipMemcpyDeviceToHost, stream));
@@ -807,16 +903,26 @@ class Solver : public SolverBase {
     need_fft();
     if (!fields_initialized) throw FlusiError(900004, "fields not initialised (call flusi_init_fields)");
     const std::string& m = p.method;
+    // Pruning.  AB2's and RK4's results (with dealiasing; RK4 dealiases
+    // always) are zero outside the region, so that a step from such a state
+    // is pruned on both sides.  RK2's first stage leaves such a state, which
+    // its second stage adds an undealiased right-hand side to
+    // (fluid_time_step.f90:594-597): the first stage prunes its result, the
+    // second its input.
+    const bool dea = prunes();
+    const bool in = dea && state_pruned();
     if (m == "AB2") {
+      const int both = in ? 3 : 0;
+      if (in) prune_reg(n0);
       if (it == 0) {  // fluid_time_step.f90:675-748 euler_startup
-        pre_rhs(uk, time);
+        pre_rhs(uk, time, true, in, in);
         dt1 = adjust_dt(time);
         if (dt1 != dt0) vis_dt = dt1;
         ZStepArgs z = zargs(SM_EULER);
-        z.u = uk; z.r0 = reg[n0]; z.dt = dt1; z.vis_dt_new = vis_dt;
+        z.u = uk; z.r0 = reg[n0]; z.dt = dt1; z.vis_dt_new = vis_dt; z.prune = both;
         post_rhs(z);
       } else {        // :752-832 adamsbashforth
-        pre_rhs(uk, time);
+        pre_rhs(uk, time, true, in, in);
         double d = adjust_dt(time);
         if (d > p.tmax - time) d = p.tmax - time;
         dt1 = d;
@@ -824,37 +930,74 @@ class Solver : public SolverBase {
         z.b10 = dt1 / dt0 * (0.5 * dt1 + dt0);
         z.b11 = -0.5 * dt1 * dt1 / dt0;
         if (dt1 != dt0) vis_dt = dt1;
-        z.u = uk; z.r0 = reg[n0]; z.r1 = reg[n1]; z.dt = dt1; z.vis_dt_new = vis_dt;
+        z.u = uk; z.r0 = reg[n0]; z.r1 = reg[n1]; z.dt = dt1; z.vis_dt_new = vis_dt; z.prune = both;
         post_rhs(z);
       }
+      set_state_pruned(dea);
+      if (dea) set_reg_pruned(n0);
     } else if (m == "RK2") {  // :519-598
-      pre_rhs(uk, time);
+      pre_rhs(uk, time, true, in, dea);
       dt1 = adjust_dt(time);
       const double old = vis_dt;
       if (dt1 != dt0) vis_dt = dt1;
+      if (dea) prune_reg(0);
+      set_state_pruned(false);
       ZStepArgs z = zargs(SM_RK2_1);
-      z.u = uk; z.r0 = reg[0]; z.dt = dt1; z.vis_dt_old = old; z.vis_dt_new = vis_dt;
+      z.u = uk; z.r0 = reg[0]; z.dt = dt1; z.vis_dt_old = old; z.vis_dt_new = vis_dt; z.prune = dea ? 2 : 0;
       post_rhs(z);
-      pre_rhs(uk, time);
+      pre_rhs(uk, time, true, dea);
       ZStepArgs z2 = zargs(SM_RK2_2);
-      z2.u = uk; z2.r0 = reg[0]; z2.dt = dt1;
+      z2.u = uk; z2.r0 = reg[0]; z2.dt = dt1; z2.prune = dea ? 1 : 0;
       post_rhs(z2);
     } else if (m == "RK4") {  // :602-671 (explicit diffusion, accumulator register)
-      pre_rhs(uk, time);
+      if (in) { prune_reg(0); prune_reg(1); }
+      pre_rhs(uk, time, true, in, in);
       dt1 = adjust_dt(time);
       const int modes[4] = {SM_RK4_1, SM_RK4_2, SM_RK4_3, SM_RK4_4};
       const double ts[4] = {time, time + 0.5 * dt1, time + 0.5 * dt1, time + dt1};
+      if (!in) { set_reg_pruned(0, false); set_reg_pruned(1, false); }
       for (int s = 0; s < 4; ++s) {
-        if (s > 0) pre_rhs(reg[0], ts[s]);
+        if (s > 0) pre_rhs(reg[0], ts[s], true, in, in);
         ZStepArgs z = zargs(modes[s]);
         z.u = uk; z.udiff = (s == 0) ? uk : reg[0]; z.ustage = reg[0]; z.acc = reg[1]; z.dt = dt1;
+        z.prune = in ? 3 : 0;
         post_rhs(z);
       }
+      set_state_pruned(dea);
     } else {
       throw FlusiError(10001, "Error! iTimeMethodFluid unknown. Abort.");
     }
     record_ekin();
     std::swap(n0, n1);  // time_step.f90:72
+  }
+
+  // what the buffers hold outside the dealiased region, for every member of
+  // the batch being launched
+  template <typename F> void members(F&& f) {
+    if (batch_n(bat) > 1) for (Solver<T>* m : batch) f(*m);
+    else f(*this);
+  }
+  // Whether steps are pruned: RK4 dealiases always, AB2 and RK2 with iDealias.
+  // The smallest grids are bound by their launches and the latency of each
+  // pass, which the region's tables add a load to (us per step, full/pruned:
+  // 32^3 FP64 AB2 51.5/52.4, RK2 102/109, FP32 RK2 111/123; 48^3 AB2 81/73,
+  // RK2 158/160, FP32 AB2 69/68, RK2 133/147; 64^3 AB2 57/51, RK2 107/101,
+  // FP32 51/49, 99/97): AB2 and RK4 gain from 48^3 on, RK2, pruned on one
+  // side of each right-hand side, from 64^3.
+  bool prunes() const {
+    if (!prune_ok || !(p.method == "RK4" || p.iDealias == 1)) return false;
+    return prune_any_size || npts >= (p.method == "RK2" ? 1L << 18 : 100000L);
+  }
+  bool state_pruned() { bool b = true; members([&](Solver<T>& m) { b = b && m.uk_pruned; }); return b; }
+  void set_state_pruned(bool v) { members([&](Solver<T>& m) { m.uk_pruned = v; }); }
+  void set_reg_pruned(int r, bool v = true) { members([&](Solver<T>& m) { m.reg_pruned[r] = v; }); }
+  // a register about to be written only inside the region: clear what an
+  // earlier use left outside it
+  void prune_reg(int r) {
+    members([&](Solver<T>& m) {
+      if (!m.reg_pruned[r]) { launch_zero(m.reg[r], state_bytes(), stream); kcheck("clear register"); }
+      m.reg_pruned[r] = true;
+    });
   }
 
   void cal_nlk(double t, double* nlk, double* u) override {
@@ -886,6 +1029,7 @@ class Solver : public SolverBase {
   struct AdjointState {
     int K = 0, every = 0;
     std::vector<double> theta, tn;  // controls and the step times t_0..t_K
+    std::vector<char> ckp, segp;    // whether those states are zero outside the dealiased region
     void* ck = nullptr;             // states at steps 0, every, 2 every, ...
     void* seg = nullptr;            // states of one segment
     void* st[3] = {nullptr, nullptr, nullptr};  // stage states u_2, u_3, u_4
@@ -1008,13 +1152,16 @@ class Solver : public SolverBase {
     adj.tn.assign(K + 1, 0.0);
     adj.tn[0] = time;
     copy_state(state_at(adj.ck, 0), uk);
+    adj.ckp.assign(K / every + 1, 0);
+    adj.segp.assign(every + 1, 0);
+    adj.ckp[0] = uk_pruned;
     double J = 0.0;
     for (int n = 1; n <= K; ++n) {
       step_plain();
       adj.tn[n] = time;
-      ifft_fields(uk, 3, pf(0));
+      ifft_fields(uk, 3, pf(0), uk_pruned);
       J += lift_now() / K;  // the last stage left the mask at t_n
-      if (n % every == 0) copy_state(state_at(adj.ck, n / every), uk);
+      if (n % every == 0) { copy_state(state_at(adj.ck, n / every), uk); adj.ckp[n / every] = uk_pruned; }
     }
     adj.J = J;
     adj.have_forward = true;
@@ -1187,11 +1334,12 @@ class Solver : public SolverBase {
     insect.update(t);
   }
   // W = N_u(u_s)^T lam at time t_s; grad += <phi, dg/dtheta>
-  void adjoint_rhs(const void* u_s, double t_s, const void* lam, void* W) {
+  // (in: u_s is zero outside the dealiased region)
+  void adjoint_rhs(const void* u_s, double t_s, const void* lam, void* W, bool in) {
     const SpecGeom g = sgeom();
     const double N = double(nx) * double(ny) * double(nz);
     create_mask(t_s);
-    inv_uw_phys(u_s);  // pf(0..2) u, pf(3..5) w
+    inv_uw_phys(u_s, in);  // pf(0..2) u, pf(3..5) w
     launch_adj_pre<T>(g, p.nu, 1.0 / N, lam, W, adj.mw, stream);
     void* phi = adj.ph;
     void* aw = (char*)adj.ph + 3 * sizeof(T) * npts;
@@ -1205,12 +1353,12 @@ class Solver : public SolverBase {
     kcheck("adjoint rhs");
   }
   // ub += dJ/du at step n (its state u_n), grad += dJ/dtheta there
-  void objective_terms(int n, const void* u_n) {
+  void objective_terms(int n, const void* u_n, bool in) {
     const double dV = p.dx() * p.dy() * p.dz();
     const double N = double(nx) * double(ny) * double(nz);
     const double s = dV / (p.eps * adj.K);
     create_mask(adj.tn[n]);
-    ifft_fields(u_n, 3, pf(0));
+    ifft_fields(u_n, 3, pf(0), in);
     theta_terms(adj.tn[n], nullptr, s);
     void* src = adj.ph;
     launch_ez_mask<T>(npts, s, mask, src, stream);
@@ -1219,15 +1367,19 @@ class Solver : public SolverBase {
     kcheck("objective terms");
   }
   // stage states u_2, u_3, u_4 of the step from u_n at t_n
-  void stage_states(const void* u_n, double t_n) {
+  void stage_states(const void* u_n, double t_n, bool in) {
     copy_state(uk, u_n);
+    uk_pruned = in;
+    if (in) { prune_reg(0); prune_reg(1); }
+    else reg_pruned[0] = reg_pruned[1] = false;
     const double dt = p.dt_fixed;
     const int modes[3] = {SM_RK4_1, SM_RK4_2, SM_RK4_3};
     const double ts[3] = {t_n, t_n + 0.5 * dt, t_n + 0.5 * dt};
     for (int s = 0; s < 3; ++s) {
-      pre_rhs(s == 0 ? uk : reg[0], ts[s]);
+      pre_rhs(s == 0 ? uk : reg[0], ts[s], true, in, in);
       ZStepArgs z = zargs(modes[s]);
       z.u = uk; z.udiff = (s == 0) ? uk : reg[0]; z.ustage = reg[0]; z.acc = reg[1]; z.dt = dt;
+      z.prune = in ? 3 : 0;
       post_rhs(z);
       copy_state(adj.st[s], reg[0]);
     }
@@ -1245,38 +1397,43 @@ class Solver : public SolverBase {
       const int n0 = sg * E, n1 = std::min(K, n0 + E);
       // the segment's states u_{n0} .. u_{n1}
       copy_state(uk, state_at(a.ck, sg));
+      uk_pruned = a.ckp[sg];
       time = a.tn[n0]; it = n0; dt1 = dt;
       copy_state(state_at(a.seg, 0), uk);
+      a.segp[0] = uk_pruned;
       for (int n = n0; n < n1; ++n) {
         step_plain();
         copy_state(state_at(a.seg, n + 1 - n0), uk);
+        a.segp[n + 1 - n0] = uk_pruned;
       }
       for (int n = n1 - 1; n >= n0; --n) {
-        objective_terms(n + 1, state_at(a.seg, n + 1 - n0));
+        objective_terms(n + 1, state_at(a.seg, n + 1 - n0), a.segp[n + 1 - n0]);
         const void* u_n = state_at(a.seg, n - n0);
-        stage_states(u_n, a.tn[n]);
+        const bool in = a.segp[n - n0];  // then the stage states are zero outside the region, too
+        stage_states(u_n, a.tn[n], in);
         const double t = a.tn[n];
         // stage 4 (u_4 at t + dt)
         launch_axpby<T>(ns, dt / 6.0, a.ub, 0.0, nullptr, a.kb, stream);
-        adjoint_rhs(a.st[2], t + dt, a.kb, a.wv);
+        adjoint_rhs(a.st[2], t + dt, a.kb, a.wv, in);
         launch_axpby<T>(ns, 1.0, a.ub, 1.0, a.wv, a.un, stream);
         // stage 3 (u_3 at t + dt/2)
         launch_axpby<T>(ns, dt / 3.0, a.ub, dt, a.wv, a.kb, stream);
-        adjoint_rhs(a.st[1], t + 0.5 * dt, a.kb, a.wv);
+        adjoint_rhs(a.st[1], t + 0.5 * dt, a.kb, a.wv, in);
         launch_axpby<T>(ns, 1.0, a.un, 1.0, a.wv, a.un, stream);
         // stage 2 (u_2 at t + dt/2)
         launch_axpby<T>(ns, dt / 3.0, a.ub, 0.5 * dt, a.wv, a.kb, stream);
-        adjoint_rhs(a.st[0], t + 0.5 * dt, a.kb, a.wv);
+        adjoint_rhs(a.st[0], t + 0.5 * dt, a.kb, a.wv, in);
         launch_axpby<T>(ns, 1.0, a.un, 1.0, a.wv, a.un, stream);
         // stage 1 (u_n at t)
         launch_axpby<T>(ns, dt / 6.0, a.ub, 0.5 * dt, a.wv, a.kb, stream);
-        adjoint_rhs(u_n, t, a.kb, a.wv);
+        adjoint_rhs(u_n, t, a.kb, a.wv, in);
         launch_axpby<T>(ns, 1.0, a.un, 1.0, a.wv, a.ub, stream);
       }
     }
     HIPCHECK(hipMemcpyAsync(grad_out, a.gacc, sizeof(double) * ncon, hipMemcpyDeviceToHost, stream));
     // the solver is left at the initial state
     copy_state(uk, state_at(a.ck, 0));
+    uk_pruned = a.ckp[0];
     time = a.tn[0]; it = 0;
     create_mask(time);
     HIPCHECK(hipStreamSynchronize(stream));
@@ -1610,6 +1767,7 @@ class Solver : public SolverBase {
 
   void set_uk(const double* h) override {
     need_fft();
+ uk_pruned = false;
  copy_real_in(h, uk, 6 * nc); fields_initialized = true; }
   void get_uk(double* h) override {
     need_fft();
@@ -1618,36 +1776,42 @@ class Solver : public SolverBase {
   void ensure_phys() { if (!phys) phys = dalloc(7 * sizeof(T) * npts); }
   T* pf(int f) { return reinterpret_cast<T*>(phys) + (long)f * npts; }
 
-  void inv_uw_phys(const void* u_in) {
-    inv_uw(u_in);
+  // in: u_in is zero outside the dealiased region
+  void inv_uw_phys(const void* u_in, bool in) {
+    p_row = prow;
+    inv_uw(u_in, in);
     ensure_phys();
     XPassArgs a = xargs();
+    if (in) a.kin = pr.nkx;
     a.in = P; a.out = phys; a.fstride_in = pc; a.fstride_out = npts; a.nf = 6;
     timed(TM_X, [&] { launch_x_pass<T>(a, XM_INV_UW, stream); });
     kcheck("x inverse uw");
   }
   // 1 or 3 spectral S-layout fields -> physical
-  void ifft_fields(const void* src, int nf, void* dst) {
+  void ifft_fields(const void* src, int nf, void* dst, bool in = false) {
+    p_row = prow;
     const C* s = reinterpret_cast<const C*>(src);
     TileJob zj[3], yj[3];
     for (int f = 0; f < nf; ++f) {
       zj[f] = TileJob{s + (long)f * nc, nullptr, cf(Q, f), OP_COPY, nullptr, 0};
       yj[f] = TileJob{cf(Q, f), nullptr, cfp(f), OP_COPY, nullptr, 0};
     }
-    zinv(zj, nf);
-    yinv(yj, nf);
+    zinv(zj, nf, in);
+    yinv(yj, nf, in);
     XPassArgs a = xargs();
+    if (in) a.kin = pr.nkx;
     a.in = P; a.out = dst; a.fstride_in = pc; a.fstride_out = npts; a.nf = nf;
     timed(TM_X, [&] { launch_x_pass<T>(a, XM_INV, stream); });
     kcheck("x inverse");
   }
   // 1 or 3 physical fields -> S-layout spectral (times 1/N)
   void fft_fields(const void* src, int nf, void* dst) {
+    p_row = prow;
     XPassArgs a = xargs();
     a.in = src; a.out = P; a.fstride_in = npts; a.fstride_out = pc; a.nf = nf;
     timed(TM_X, [&] { launch_x_pass<T>(a, XM_FWD, stream); });
     kcheck("x forward");
-    yfwd(nf);
+    yfwd(nf, false);
     zfwd_plain(nf, dst);
   }
 
@@ -1662,7 +1826,7 @@ class Solver : public SolverBase {
     post_rhs(z);
     ensure_phys();
     ifft_fields(P, 1, pf(6));
-    ifft_fields(uk, 3, pf(0));
+    ifft_fields(uk, 3, pf(0), uk_pruned);
     launch_pressure_phys<T>(npts, pf(0), pf(6), stream);
     kcheck("pressure");
     copy_real_out(pf(6), out, npts);
@@ -1795,6 +1959,7 @@ class Solver : public SolverBase {
       throw FlusiError(77776, "ERROR! read_runtime_backup(): Resolution mismatch");
     std::vector<double> f(npts);
     void* dst[3] = {uk, reg[0], reg[1]};
+    uk_pruned = reg_pruned[0] = reg_pruned[1] = false;
     const char* names[3][3] = {{"ux", "uy", "uz"}, {"nlkx0", "nlky0", "nlkz0"}, {"nlkx1", "nlky1", "nlkz1"}};
     for (int g = 0; g < 3; ++g)
       for (int c = 0; c < 3; ++c) {
@@ -1829,7 +1994,7 @@ class Solver : public SolverBase {
 
   void get_u(double* u, bool vort) override {
     need_fft();
-    inv_uw_phys(uk);
+    inv_uw_phys(uk, uk_pruned);
     copy_real_out(vort ? (void*)pf(3) : (void*)pf(0), u, 3 * npts);
   }
 
@@ -1860,8 +2025,11 @@ class Solver : public SolverBase {
       launch_zero(uk, 3 * cs, stream);
       launch_zero(reg[0], 3 * cs, stream);
       launch_zero(reg[1], 3 * cs, stream);
+      uk_pruned = prune_ok;  // of the initial fields, a mean flow or none stays inside the region
+      reg_pruned[0] = reg_pruned[1] = true;
     }
     if (p.inicond == "VortexRing") {
+      uk_pruned = false;
       // init_fields_fsi.f90:381-435 (core radius 0.82*Size unless core_a is given)
       const double r00 = p.length;
       const double a = p.core_a > 0.0 ? p.core_a : 0.82 * r00;
@@ -2045,7 +2213,7 @@ class Solver : public SolverBase {
     if (p.iPenalization == 1) {  // drag.f90:53: nothing to do without penalisation
       ensure_phys();
       if (u_host) copy_real_in(u_host, pf(0), 3 * npts);
-      else { need_fft(); ifft_fields(uk, 3, pf(0)); }
+      else { need_fft(); ifft_fields(uk, 3, pf(0), uk_pruned); }
       drag_assemble(t, diag_sums(pf(0), nullptr, nullptr), o, true);
     }
     if (out) std::memcpy(out, o, sizeof(o));
@@ -2057,14 +2225,14 @@ class Solver : public SolverBase {
     if (!fields_initialized) throw FlusiError(900004, "fields not initialised (call flusi_init_fields)");
     const bool ins = is_insect;
     if (ins) append("kinematics.t", insect.kinematics_row(t), kin_header());
-    inv_uw_phys(uk);
+    inv_uw_phys(uk, uk_pruned);
     const bool forces = p.compute_forces == 1 && p.iPenalization == 1;
     if (p.compute_forces == 1 && p.iMoving == 1) create_mask(t);
     // divergence (basic_operators.f90:707-734) -> physical
     void* dk = reg_scratch();
     launch_divergence<T>(geom, kx_d, ky_d, kz_d, uk, dk, stream);
     kcheck("divergence");
-    ifft_fields(dk, 1, pf(6));
+    ifft_fields(dk, 1, pf(6), uk_pruned);
     const std::vector<double> r = diag_sums(pf(0), pf(3), pf(6));
     std::vector<C> m0(3);
     for (int c = 0; c < 3; ++c)
@@ -2226,9 +2394,9 @@ class Ensemble : public EnsembleBase {
       for (size_t k = 1; k < g.idx.size(); ++k) {
         Solver<T>& m = S(g.idx[k]);
         const void* a[] = {L.uk, L.reg[0], L.reg[1], L.Q, L.P, L.mask, L.us, L.color, L.tab, L.tw_z, L.tw_y, L.tw_M,
-                           L.tw_N, L.xpart, L.zpart, L.dpart, L.red, L.rmid, L.kinds};
+                           L.tw_N, L.xpart, L.zpart, L.dpart, L.red, L.rmid, L.kinds, L.pr.zlim, L.ptiles[1]};
         const void* b[] = {m.uk, m.reg[0], m.reg[1], m.Q, m.P, m.mask, m.us, m.color, m.tab, m.tw_z, m.tw_y, m.tw_M,
-                           m.tw_N, m.xpart, m.zpart, m.dpart, m.red, m.rmid, m.kinds};
+                           m.tw_N, m.xpart, m.zpart, m.dpart, m.red, m.rmid, m.kinds, m.pr.zlim, m.ptiles[1]};
         for (size_t j = 0; j < sizeof(a) / sizeof(a[0]); ++j)
           if ((const char*)b[j] - (const char*)a[j] != (long)(k * g.stride))
             throw FlusiError(900014, "ensemble: member buffers do not follow the batch layout");
@@ -2440,10 +2608,14 @@ class Ensemble : public EnsembleBase {
     if (mode != 1 && mode != 2) throw FlusiError(900019, "ensemble: mode must be 0, 1 or 2");
     int k = 0;
     if (mode == 2) {
-      // the captured step assumes an established integrating factor
+      // the captured step assumes an established integrating factor, and RK4
+      // (pruned) a state that is zero outside the dealiased region
       for (; k < nsteps; ++k) {
         bool fresh = false;
-        for (flusi_ctx* c : ctxs) fresh = fresh || c->s->it == 0;
+        for (flusi_ctx* c : ctxs) {
+          const Solver<T>& m = *static_cast<const Solver<T>*>(c->s.get());
+          fresh = fresh || m.it == 0 || (m.prunes() && m.p.method == "RK4" && !m.uk_pruned);
+        }
         if (!fresh) break;
         batched_step();
       }

@@ -47,23 +47,29 @@ __device__ __forceinline__ cplx<T> apply_op(int op, double kscale, int aa, cplx<
   return x;
 }
 
-// SF: every store of the grid lands on a row below the store bound (the host
-// checks it), so that the stores need no guard.  Loads and stores then carry
-// no branch, and the wait for the next job's prefetched operands does not
-// have to cover the current job's stores (with a guard, the compiler cannot
-// count the stores in flight and waits for all of them).
-template <typename T, int L, int S, bool CONTIG_IN, bool SF>
+// Loads and stores go through buffer descriptors (see make_brsrc): a line
+// beyond the tile axis and a position outside the dealiased region are
+// out-of-range offsets, so that no access carries a branch and the wait for
+// the next job's prefetched operands does not have to cover the current job's
+// stores (with a guard, the compiler cannot count the stores in flight and
+// waits for all of them).
+template <typename T, int L, int S, bool CONTIG_IN>
 __global__ __launch_bounds__((TWShape<T, L>::NT)) void tile_wave_k(TilePassArgs a) {
   using Sh = TWShape<T, L>;
   constexpr int TL = Sh::TL, NT = Sh::NT, LS = Sh::LS, K = Sh::K;
   constexpr int G = TWPlan<L>::G;
+  constexpr unsigned ES = sizeof(cplx<T>);
   extern __shared__ char smem_raw[];
   cplx<T>* tile = reinterpret_cast<cplx<T>*>(smem_raw);
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int line = wv * TWPlan<L>::LPW + lane / G, l = lane % G;
   cplx<T>* ln = tile + line * LS;
-  const int b0 = blockIdx.x * TL;
-  const long c = blockIdx.y;
+  int b0 = blockIdx.x * TL, c = blockIdx.y;
+  if (a.tiles) {  // the tiles that meet the dealiased region
+    const uint32_t t = ((gptr<const uint32_t>)a.tiles)[blockIdx.x];
+    b0 = (int)(t & 0xffffu) * TL;
+    c = (int)(t >> 16);
+  }
   const int nbs = a.nb_store > a.nb ? a.nb_store : a.nb;  // lines >= nb hold zeros
   const long moff = (long)blockIdx.z * a.bat.mstride;  // batch member's slab
   const T sc = (T)a.scale;
@@ -79,30 +85,50 @@ __global__ __launch_bounds__((TWShape<T, L>::NT)) void tile_wave_k(TilePassArgs 
     tw = (gptr<const cplx<T>>)mshift(a.tw, moff);
   }
 
+  // This lane's line on the contiguous side: the byte offset of its position
+  // 0, the shift of its upper half (positions L/2.., the negative wave
+  // numbers) and what it holds.  Reading (CONTIG_IN): positions of |wave
+  // number| <= lim.  Writing (PR_YFWD): compact positions [plo, phi).
+  const int b = b0 + line;
+  const bool lok = b < a.nb;
+  int lim = lok ? L : -1, row = b;
+  unsigned lo = 0, hi = 0;  // element shifts of the lower and the upper half
+  int plo = 0, phi = 0;
+  if (CONTIG_IN && a.prune == PR_ZINV) {
+    lim = ((gptr<const int16_t>)a.pr.zlim)[c * a.pr.nyp + b];
+    row = b - a.pr.ym0;
+    if (row < 0) row += a.nb;
+  } else if (CONTIG_IN && a.prune == PR_YINV) {
+    lim = lok ? ((gptr<const int16_t>)a.pr.ylim)[b] : -1;
+    lo = a.pr.ym0;
+    hi = (unsigned)(a.pr.ym0 - L);
+  } else if (!CONTIG_IN && a.prune == PR_YFWD) {
+    constexpr int SEG = 128 / ES;
+    const int ym = lok ? ((gptr<const int16_t>)a.pr.ylim)[b] : -1;
+    plo = (a.pr.ym0 - ym) & ~(SEG - 1);
+    phi = lok ? min(a.pr.nyp, ((a.pr.ym0 + ym) | (SEG - 1)) + 1) : 0;
+  }
+
   // operands: CONTIG_IN - the lane's 8 positions of its own line;
   // otherwise - the thread's K tile elements (bb = e % TL, a = e / TL)
-  // (lines beyond nb read line nb - 1, unused: zeros are taken where the
-  // operands are consumed, so that neither the loads nor a select right
-  // after them needs a branch or a wait)
   cplx<T> r0[8], r1[8];
   auto load = [&](int jb, int which) {
-    // global-address-space views (see gptr): the prefetched loads then do
-    // not hold up the transform's LDS waits
-    const gptr<const cplx<T>> in = (gptr<const cplx<T>>)mshift(which ? a.jobs[jb].in1 : a.jobs[jb].in0, moff);
+    const brsrc in = make_brsrc(mshift(which ? a.jobs[jb].in1 : a.jobs[jb].in0, moff), a.ibytes);
     if (CONTIG_IN) {
-      const bool ok = b0 + line < a.nb;
-      const long base = c * a.sin.c + (long)(ok ? b0 + line : a.nb - 1) * a.sin.b + l;
+      const unsigned base = (unsigned)c * (unsigned)a.sin.c + (unsigned)row * (unsigned)a.sin.b + l;
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
-        const cplx<T> x = lds<T>(in + base + q * G);
+        const int w = q < 4 ? l + q * G : L - l - q * G;  // |wave number|
+        const unsigned off = w <= lim ? (base + (q < 4 ? lo : hi) + q * G) * ES : kOob;
+        const cplx<T> x = bld<T>(in, off);
         if (which) r1[q] = x; else r0[q] = x;
       }
     } else {
 #pragma unroll
       for (int k = 0; k < K; ++k) {
         const int e = tid + k * NT, bb = e % TL, aa = e / TL;
-        const bool ok = b0 + bb < a.nb;
-        const cplx<T> x = lds<T>(in + c * a.sin.c + (long)(ok ? b0 + bb : a.nb - 1) + (long)aa * a.sin.a);
+        const unsigned off = (unsigned)c * (unsigned)a.sin.c + (unsigned)(b0 + bb) + (unsigned)aa * (unsigned)a.sin.a;
+        const cplx<T> x = bld<T>(in, b0 + bb < a.nb ? off * ES : kOob);
         if (which) r1[k] = x; else r0[k] = x;
       }
     }
@@ -120,16 +146,12 @@ __global__ __launch_bounds__((TWShape<T, L>::NT)) void tile_wave_k(TilePassArgs 
     const int nout = a.jobs[jb].out2 ? 2 : 1;
     for (int o = 0; o < nout; ++o) {
       const int op = o ? a.jobs[jb].op2 : a.jobs[jb].op;
-      const gptr<cplx<T>> out = (gptr<cplx<T>>)mshift(o ? a.jobs[jb].out2 : a.jobs[jb].out, moff);
+      const brsrc out = make_brsrc(mshift(o ? a.jobs[jb].out2 : a.jobs[jb].out, moff), a.obytes);
       const bool pf = (o == nout - 1) && (jb + 1 < a.njobs);
       cplx<T> v[8];
       if (CONTIG_IN) {
 #pragma unroll
         for (int q = 0; q < 8; ++q) v[q] = apply_op<T, L>(op, a.kscale, l + q * G, r0[q], r1[q]);
-        if (b0 + line >= a.nb) {
-#pragma unroll
-          for (int q = 0; q < 8; ++q) v[q] = mk<T>(T(0), T(0));
-        }
         if (pf) load_job(jb + 1);
         twfft<T, L, S>(v, tw, ln, l);
         // turn the tile: natural order into the line's row, then 128-byte
@@ -141,15 +163,15 @@ __global__ __launch_bounds__((TWShape<T, L>::NT)) void tile_wave_k(TilePassArgs 
         for (int k = 0; k < K; ++k) {
           const int e = tid + k * NT, bb = e % TL, aa = e / TL;
           const cplx<T> x = tile[bb * LS + lp<T>(aa)];
-          if (SF || b0 + bb < nbs) sts<T>(out + c * a.sout.c + (long)(b0 + bb) + (long)aa * a.sout.a, mk<T>(x.x * sc, x.y * sc));
+          const unsigned off = (unsigned)c * (unsigned)a.sout.c + (unsigned)(b0 + bb) + (unsigned)aa * (unsigned)a.sout.a;
+          bst<T>(out, b0 + bb < nbs ? off * ES : kOob, mk<T>(x.x * sc, x.y * sc));
         }
         __syncthreads();
       } else {
 #pragma unroll
         for (int k = 0; k < K; ++k) {
           const int e = tid + k * NT, bb = e % TL, aa = e / TL;
-          const cplx<T> x = apply_op<T, L>(op, a.kscale, aa, r0[k], r1[k]);
-          tile[bb * LS + lp<T>(aa)] = b0 + bb < a.nb ? x : mk<T>(T(0), T(0));
+          tile[bb * LS + lp<T>(aa)] = apply_op<T, L>(op, a.kscale, aa, r0[k], r1[k]);
         }
         __syncthreads();
         if (pf) load_job(jb + 1);
@@ -157,10 +179,18 @@ __global__ __launch_bounds__((TWShape<T, L>::NT)) void tile_wave_k(TilePassArgs 
         for (int q = 0; q < 8; ++q) v[q] = ln[lp<T>(l + q * G)];
         wave_sync();
         twfft<T, L, S>(v, tw, ln, l);
-        if (SF || b0 + line < a.nb) {
-          const long base = c * a.sout.c + (long)(b0 + line) * a.sout.b + l;
+        const unsigned base = (unsigned)c * (unsigned)a.sout.c + (unsigned)b * (unsigned)a.sout.b;
 #pragma unroll
-          for (int q = 0; q < 8; ++q) sts<T>(out + base + q * G, mk<T>(v[q].x * sc, v[q].y * sc));
+        for (int q = 0; q < 8; ++q) {
+          const int aa = l + q * G;
+          unsigned off;
+          if (a.prune == PR_YFWD) {
+            const int p = a.pr.ym0 + (q < 4 ? aa : aa - L);
+            off = p >= plo && p < phi ? (base + (unsigned)p) * ES : kOob;
+          } else {
+            off = lok ? (base + aa) * ES : kOob;
+          }
+          bst<T>(out, off, mk<T>(v[q].x * sc, v[q].y * sc));
         }
         __syncthreads();
       }
@@ -168,23 +198,14 @@ __global__ __launch_bounds__((TWShape<T, L>::NT)) void tile_wave_k(TilePassArgs 
   }
 }
 
-template <typename T, int L, int S, bool CI, bool SF>
-void run_tw_sf(const TilePassArgs& a, hipStream_t s) {
-  using Sh = TWShape<T, L>;
-  static bool init = false;
-  if (!init) { set_smem(tile_wave_k<T, L, S, CI, SF>, Sh::smem); init = true; }
-  dim3 grid((a.nb + Sh::TL - 1) / Sh::TL, a.nc, batch_n(a.bat));
-  hipLaunchKernelGGL((tile_wave_k<T, L, S, CI, SF>), grid, dim3(Sh::NT), Sh::smem, s, a);
-}
 template <typename T, int L, int S, bool CI>
 void run_tw(const TilePassArgs& a, hipStream_t s) {
-  // stores unguarded when the grid's last tile ends at or below the store
-  // bound (nb_store rows for the segment-side stores, nb for the line stores)
-  const int tl = TWShape<T, L>::TL;
-  const long rows = (long)((a.nb + tl - 1) / tl) * tl;
-  const long bound = CI ? (a.nb_store > a.nb ? a.nb_store : a.nb) : a.nb;
-  if (rows <= bound) run_tw_sf<T, L, S, CI, true>(a, s);
-  else run_tw_sf<T, L, S, CI, false>(a, s);
+  using Sh = TWShape<T, L>;
+  static bool init = false;
+  if (!init) { set_smem(tile_wave_k<T, L, S, CI>, Sh::smem); init = true; }
+  const dim3 grid = a.tiles ? dim3(a.ntiles, 1, batch_n(a.bat))
+                            : dim3((a.nb + Sh::TL - 1) / Sh::TL, a.nc, batch_n(a.bat));
+  hipLaunchKernelGGL((tile_wave_k<T, L, S, CI>), grid, dim3(Sh::NT), Sh::smem, s, a);
 }
 
 template <typename T, int L>
@@ -195,6 +216,8 @@ void run_tw_dir(const TilePassArgs& a, int dir, bool ci, hipStream_t s) {
 
 }  // namespace
 
+int tile_lines(bool fp64) { return fp64 ? TWTile<double>::TL : TWTile<float>::TL; }
+
 bool tile_wave_supported(int L) { return L == 64 || L == 128 || L == 256 || L == 512; }
 
 template <typename T>
@@ -202,6 +225,7 @@ void launch_tile_wave(const TilePassArgs& a, int L, int dir, bool ci, hipStream_
   const bool unit = ci ? (a.sin.a == 1 && a.sout.b == 1) : (a.sin.b == 1 && a.sout.a == 1);
   if (!unit) throw std::runtime_error("tile pass: the contiguous axes must have unit stride");
   if (a.njobs < 1 || a.njobs > 6) throw std::runtime_error("tile pass: 1..6 jobs");
+  if (a.ibytes >= kOob || a.obytes >= kOob) throw std::runtime_error("tile pass: field too large for 32-bit offsets");
   switch (L) {
     case 64: run_tw_dir<T, 64>(a, dir, ci, s); break;
     case 128: run_tw_dir<T, 128>(a, dir, ci, s); break;

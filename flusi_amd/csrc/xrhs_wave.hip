@@ -261,8 +261,8 @@ __global__ __launch_bounds__(XW_NT) __attribute__((amdgpu_waves_per_eu(WPE > 0 ?
   for (int f = 0; f < 6; ++f) {
     const gptr<const cplx<T>> p = in + f * a.fstride_in + lb;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) X[f][q] = gld<T>(p + l + q * G);
-    XM[f] = gld<T>(p + M);
+    for (int q = 0; q < 4; ++q) X[f][q] = l + q * G < a.kin ? gld<T>(p + l + q * G) : mk<T>(T(0), T(0));
+    XM[f] = M < a.kin ? gld<T>(p + M) : mk<T>(T(0), T(0));
   }
 
   // mask at the physical points 2n, 2n+1 (n = l + qG), read early; a line
@@ -459,9 +459,9 @@ __global__ __launch_bounds__(XW_NT) __attribute__((amdgpu_waves_per_eu(WPE > 0 ?
       for (int q = 0; q < 4; ++q) {
         const cplx<T> zk = O[c][q];
         const cplx<T> s1 = add(zk, conj_w(zm[q])), d1 = sub(zk, conj_w(zm[q]));
-        gst<T>(o + l + q * G, scl(sub(s1, ik_w<T>(T(1), cmul(twn[l + q * G], d1))), half));
+        if (l + q * G < a.kout) gst<T>(o + l + q * G, scl(sub(s1, ik_w<T>(T(1), cmul(twn[l + q * G], d1))), half));
       }
-      if (l == 0) {
+      if (l == 0 && M < a.kout) {
         // k = M: partner of k = 0 is itself
         const cplx<T> zk = O[c][0];
         const cplx<T> s2 = add(zk, conj_w(zk)), d2 = sub(zk, conj_w(zk));

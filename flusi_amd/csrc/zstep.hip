@@ -74,24 +74,64 @@ template <typename T> struct ZPre {
   cplx<T> st[3][3];
   double ky, kz, kyt2, kzt2;
 };
+// state field c of a pass operand
+template <typename T> __device__ __forceinline__ brsrc zfield(const ZStepArgs& a, const MOff& mo, const void* base, int c) {
+  return make_brsrc(reinterpret_cast<const cplx<T>*>(base) + mo.mc + c * a.fs, (unsigned)a.fs * (unsigned)sizeof(cplx<T>));
+}
+// off: byte offset of the position in a state field, or kOob where the
+// operands are zero (outside the dealiased region)
 template <typename T, int MG>
-__device__ __forceinline__ void zpreload(const ZStepArgs& a, const MOff& mo, int kx, int ky, int kzi, ZPre<T>& pr) {
+__device__ __forceinline__ void zpreload(const ZStepArgs& a, const MOff& mo, unsigned off, int ky, int kzi, ZPre<T>& pr) {
   constexpr int m = MG - MG_FIXED;
-  const long si = ((long)kx * a.ny + ky) * a.nz + kzi + mo.mc;
   pr.ky = a.ky[ky + mo.md];
   pr.kz = a.kz[kzi + mo.md];
   pr.kyt2 = a.kyt2[ky + mo.md];
   pr.kzt2 = a.kzt2[kzi + mo.md];
-  const cplx<T>* s0 = reinterpret_cast<const cplx<T>*>(m >= SM_RK4_1 ? a.udiff : a.u);
-  const cplx<T>* s1 = reinterpret_cast<const cplx<T>*>(m >= SM_RK4_2 ? a.acc : (m == SM_AB2 ? a.r1 : a.r0));
+  const void* s0 = m >= SM_RK4_1 ? a.udiff : a.u;
+  const void* s1 = m >= SM_RK4_2 ? a.acc : (m == SM_AB2 ? a.r1 : a.r0);
   constexpr bool has1 = m >= SM_RK4_2 || m == SM_AB2 || m == SM_RK2_2;
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
-    pr.st[0][c] = lds<T>(s0 + c * a.fs + si);
-    if constexpr (has1) pr.st[1][c] = lds<T>(s1 + c * a.fs + si);
-    if constexpr (m == SM_RK4_3) pr.st[2][c] = lds<T>(reinterpret_cast<const cplx<T>*>(a.u) + c * a.fs + si);
+    pr.st[0][c] = bld<T>(zfield<T>(a, mo, s0, c), off);
+    if constexpr (has1) pr.st[1][c] = bld<T>(zfield<T>(a, mo, s1, c), off);
+    if constexpr (m == SM_RK4_3) pr.st[2][c] = bld<T>(zfield<T>(a, mo, a.u, c), off);
   }
 }
+
+// A pruned launch at one line (kx, ky): zm = the largest |kz| of the region
+// there (-1: none).  Operands are read at |kz| <= zm; results are written to
+// the whole 128-byte lines that hold such positions, [0, up) and [dn, nz) -
+// zeros between zm and their ends - so that no line is written in part.
+// Without pruning every position is read and written.
+struct ZLim {
+  int zm, up, dn;
+  __device__ __forceinline__ bool in(int kzi, int nz) const { return (kzi < (nz >> 1) ? kzi : nz - kzi) <= zm; }
+  __device__ __forceinline__ bool out(int kzi) const { return kzi < up || kzi >= dn; }
+};
+template <typename T> __device__ __forceinline__ ZLim zlim_at(const ZStepArgs& a, int kx, int p) {
+  ZLim z{a.nz, a.nz, 0};
+  if (a.prune) {
+    z.zm = (kx < a.pr.nkx && p >= 0 && p < a.pr.nyp) ? a.pr.zlim[kx * a.pr.nyp + p] : -1;
+    if (a.prune & 2) {
+      constexpr int SEG = 128 / (int)sizeof(cplx<T>);
+      z.up = z.zm < 0 ? 0 : (z.zm | (SEG - 1)) + 1;
+      z.dn = z.zm <= 0 ? a.nz : (a.nz - z.zm) & ~(SEG - 1);
+    }
+  }
+  return z;
+}
+// the ky index of tile line b: compact Q rows hold ky = b - ym0
+__device__ __forceinline__ int zrow(const ZStepArgs& a, int b) {
+  if (!(a.prune & 2)) return b;
+  const int ky = b - a.pr.ym0;
+  return ky < 0 ? ky + a.ny : ky;
+}
+// the compact position of ky row `row` (beyond the table where outside)
+__device__ __forceinline__ int zpos(const ZStepArgs& a, int row) {
+  return a.pr.ym0 + (row < (a.ny + 1) / 2 ? row : row - a.ny);
+}
+// row length of Q and number of lines of the tile axis
+__device__ __forceinline__ int zq_lines(const ZStepArgs& a) { return (a.prune & 2) ? a.pr.nyp : a.ny; }
 
 // Epilogue at one spectral point (kx, ky, kz): rv[f] is field f of the
 // z-transformed right-hand side (unscaled).  Sponge curl (sponge.f90:22-83),
@@ -107,13 +147,16 @@ __device__ __forceinline__ void zpreload(const ZStepArgs& a, const MOff& mo, int
 // integrating factors exp(-nu k^2 dt) are evaluated in FP64, and the
 // Parseval sum is accumulated in compensated FP64.
 //
+// rd: the state operands are read here (else they are zero, see ZLim; a
+// fixed-mode kernel's preloaded operands already are).
+//
 // FOLDED: rv[f] already holds the scaled right-hand side with the sponge term
 // added (sponge_fold below), so that a kernel need not keep the sponge
 // fields' values live until the epilogue.
 template <typename T, bool SPONGE, int MG, bool FOLDED = false>
 __device__ __forceinline__ void zepilogue(const ZStepArgs& a, const MOff& mo, int kx, int ky, int kzi, const cplx<T>* rv,
                                           double kxv_d, double kxt2, double wE,
-                                          bool final_stage, double& esum, double& ecomp,
+                                          bool final_stage, double& esum, double& ecomp, bool rd,
                                           const ZPre<T>* pre = nullptr) {
   using R = T;
   cplx<T>* U = reinterpret_cast<cplx<T>*>(a.u);
@@ -129,7 +172,7 @@ __device__ __forceinline__ void zepilogue(const ZStepArgs& a, const MOff& mo, in
   // operands: preloaded (fixed-mode kernels) or read here; slot as in ZPre
   auto opnd = [&](const void* base, int slot, int c) -> cplx<T> {
     if constexpr (FIX) return pre->st[slot][c];
-    else return lds<T>(reinterpret_cast<const cplx<T>*>(base) + c * a.fs + si);
+    else return bld<T>(zfield<T>(a, mo, base, c), rd ? (unsigned)(si - mo.mc) * (unsigned)sizeof(cplx<T>) : kOob);
   };
   const double kyv_d = FIX ? pre->ky : a.ky[ky + mo.md], kzv_d = FIX ? pre->kz : a.kz[kzi + mo.md];
   const double k2d = (kxv_d * kxv_d + kyv_d * kyv_d) + kzv_d * kzv_d;  // FP64: integrating factors
@@ -407,9 +450,14 @@ __global__ __launch_bounds__(NT, zb_wpe<T>(L)) void zstep_k(ZStepArgs a) {
   // workgroups x and x + 8 of a row run on one XCD one after the other; they
   // take neighbouring ky tiles, whose Q segments share 128-byte lines.
   int bx = blockIdx.x;
-  if (TL * sizeof(cplx<T>) < 128 && gridDim.x % 8 == 0) bx = (bx % 8) * (gridDim.x / 8) + bx / 8;
-  const int b0 = bx * TL;
-  const int kx = blockIdx.y;
+  if (TL * sizeof(cplx<T>) < 128 && gridDim.x % 8 == 0 && !a.tiles) bx = (bx % 8) * (gridDim.x / 8) + bx / 8;
+  int b0 = bx * TL, kx = blockIdx.y;
+  if (a.tiles) {  // the tiles that meet the dealiased region, in the same order
+    const uint32_t t = a.tiles[blockIdx.x];
+    b0 = (int)(t & 0xffffu) * TL;
+    kx = (int)(t >> 16);
+  }
+  const int nyq = zq_lines(a);
   constexpr bool PARK = ZBShape<T, L, TL>::park;
   // fixed-mode kernels load each epilogue position's operands one position
   // ahead (ZPre); without the sponge, field 2 then waits in the transform tile
@@ -448,10 +496,10 @@ __global__ __launch_bounds__(NT, zb_wpe<T>(L)) void zstep_k(ZStepArgs a) {
       const int beta = tid + p * NT;
       if (NB0 % NT == 0 || beta < NB0) {
         const int bb = beta % TL, j = beta / TL;
-        const bool ok = b0 + bb < a.ny;
+        const bool ok = b0 + bb < nyq;
 #pragma unroll
         for (int q = 0; q < R0; ++q)
-          v[p][q] = ok ? nq[mo.mc + f * a.fs + ((long)kx * a.nz + j + q * (L / R0)) * a.ny + b0 + bb] : mk<T>(T(0), T(0));
+          v[p][q] = ok ? nq[mo.mc + f * a.fs + ((long)kx * a.nz + j + q * (L / R0)) * nyq + b0 + bb] : mk<T>(T(0), T(0));
       }
     }
   };
@@ -566,7 +614,7 @@ __global__ __launch_bounds__(NT, zb_wpe<T>(L)) void zstep_k(ZStepArgs a) {
 #pragma unroll
             for (int q = 0; q < RL; ++q) {
               cplx<T> s0 = PARK ? pk[lp<T>(j + q * (L / RL))] : r[0][p][q];
-              sponge_term<T>(a, mo, kxs, b0 + bb, j + q * (L / RL), s0, r[1][p][q], r[2][p][q]);
+              sponge_term<T>(a, mo, kxs, b0 + bb < nyq ? zrow(a, b0 + bb) : a.ny, j + q * (L / RL), s0, r[1][p][q], r[2][p][q]);
               if constexpr (PARK) pk[lp<T>(j + q * (L / RL))] = s0;
               else r[0][p][q] = s0;
               __builtin_amdgcn_sched_barrier(0);  // one position at a time
@@ -596,16 +644,28 @@ __global__ __launch_bounds__(NT, zb_wpe<T>(L)) void zstep_k(ZStepArgs a) {
     const int beta = tid + (k / RL) * NT;
     bb = beta / (L / RL);
     kzi = beta - bb * (L / RL) + (k % RL) * (L / RL);
-    return (NBL % NT == 0 || beta < NBL) && b0 + bb < a.ny;
+    return (NBL % NT == 0 || beta < NBL) && b0 + bb < nyq;
   };
-  // operands of position k, read at a valid line for every thread (a
-  // position that does not exist reads line b0 and is not used), so that the
-  // loads need no branch
+  // the thread's lines: ky row (a line beyond the grid reads row 0 and is not
+  // used, so that the loads need no branch) and pruning limits
+  int row[PERL];
+  ZLim zl[PERL];
+#pragma unroll
+  for (int p = 0; p < PERL; ++p) {
+    int bb, kzi;
+    const bool ok = at(p * RL, bb, kzi);
+    row[p] = ok ? zrow(a, b0 + bb) : 0;
+    zl[p] = zlim_at<T>(a, kx, (a.prune & 2) ? b0 + bb : zpos(a, row[p]));
+    if (!ok) zl[p] = ZLim{-1, 0, a.nz};
+  }
+  // operands of position k
   ZPre<T> pre[2];
   auto preload = [&](int k, ZPre<T>& pr) {
     int bb, kzi;
-    const bool ok = at(k, bb, kzi);
-    zpreload<T, MG>(a, mo, kx, ok ? b0 + bb : b0, ok ? kzi : 0, pr);
+    const int p = k / RL;
+    const bool ok = at(k, bb, kzi) && zl[p].in(kzi, a.nz);
+    const unsigned off = ok ? (((unsigned)kx * a.ny + row[p]) * a.nz + kzi) * (unsigned)sizeof(cplx<T>) : kOob;
+    zpreload<T, MG>(a, mo, off, row[p], kzi, pr);
   };
   if constexpr (AHEAD) preload(0, pre[0]);
 #pragma unroll
@@ -613,13 +673,14 @@ __global__ __launch_bounds__(NT, zb_wpe<T>(L)) void zstep_k(ZStepArgs a) {
     if constexpr (AHEAD)
       if (k + 1 < NPOS) preload(k + 1, pre[(k + 1) & 1]);
     int bb, kzi;
-    if (!at(k, bb, kzi)) continue;
     const int p = k / RL, q = k % RL;
+    if (!at(k, bb, kzi) || !zl[p].out(kzi)) continue;
     cplx<T> rv[3];
 #pragma unroll
     for (int f = 0; f < 3; ++f)
       rv[f] = (PARK && f == 0) ? park[bb * LSP + lp<T>(kzi)] : ((TILE2 && f == 2) ? buf[bb * LSP + lp<T>(kzi)] : r[f][p][q]);
-    zepilogue<T, false, MG, SPONGE>(a, mo, kx, b0 + bb, kzi, rv, kxv, kxt2, wE, final_stage, esum, ecomp, &pre[k & 1]);
+    zepilogue<T, false, MG, SPONGE>(a, mo, kx, row[p], kzi, rv, kxv, kxt2, wE, final_stage, esum, ecomp,
+                                    zl[p].in(kzi, a.nz), &pre[k & 1]);
     if constexpr (EU > 0)
       if ((k + 1) % EU == 0) __builtin_amdgcn_sched_barrier(0);
   }
@@ -630,7 +691,7 @@ __global__ __launch_bounds__(NT, zb_wpe<T>(L)) void zstep_k(ZStepArgs a) {
     if (tid == 0) {
       double s = 0.0;
       for (int w = 0; w < NT / 64; ++w) s += red[w];
-      a.energy_partial[mo.md + (long)blockIdx.y * gridDim.x + bx] = s;
+      a.energy_partial[mo.md + (a.tiles ? (long)blockIdx.x : (long)blockIdx.y * gridDim.x + bx)] = s;
     }
   }
 }
@@ -665,8 +726,13 @@ __global__ __launch_bounds__((ZWShape<T, L>::NT)) void zstep_wave_k(ZStepArgs a)
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int line = wv * TWPlan<L>::LPW + lane / G, l = lane % G;
   cplx<T>* ln = tile + line * LS;
-  const int b0 = blockIdx.x * TL;
-  const int kx = blockIdx.y;
+  int b0 = blockIdx.x * TL, kx = blockIdx.y;
+  if (a.tiles) {  // the tiles that meet the dealiased region
+    const uint32_t t = a.tiles[blockIdx.x];
+    b0 = (int)(t & 0xffffu) * TL;
+    kx = (int)(t >> 16);
+  }
+  const int nyq = zq_lines(a);
   // twiddles: the block's LDS copy (made after the first field's loads are
   // issued, so that the two memory latencies overlap; first read after the
   // first block barrier), or global memory where it does not fit
@@ -684,8 +750,8 @@ __global__ __launch_bounds__((ZWShape<T, L>::NT)) void zstep_wave_k(ZStepArgs a)
 #pragma unroll
     for (int k = 0; k < K; ++k) {
       const int e = tid + k * NT, bb = e % TL, aa = e / TL;
-      const bool ok = b0 + bb < a.ny;
-      x[k] = ok ? nq[mo.mc + f * a.fs + ((long)kx * a.nz + aa) * a.ny + b0 + bb] : mk<T>(T(0), T(0));
+      const bool ok = b0 + bb < nyq;
+      x[k] = ok ? nq[mo.mc + f * a.fs + ((long)kx * a.nz + aa) * nyq + b0 + bb] : mk<T>(T(0), T(0));
     }
   };
   cplx<T> r[3][8];
@@ -715,8 +781,8 @@ __global__ __launch_bounds__((ZWShape<T, L>::NT)) void zstep_wave_k(ZStepArgs a)
 #pragma unroll
       for (int k = 0; k < K; ++k) {
         const int e = t + k * NT, bb = e % TL, aa = e / TL;
-        const bool ok = b0 + bb < a.ny;
-        x[k] = ok ? nq[mo.mc + f * a.fs + ((long)kx * a.nz + aa) * a.ny + b0 + bb] : mk<T>(T(0), T(0));
+        const bool ok = b0 + bb < nyq;
+        x[k] = ok ? nq[mo.mc + f * a.fs + ((long)kx * a.nz + aa) * nyq + b0 + bb] : mk<T>(T(0), T(0));
       }
     };
     loadt(fld(0), tid);
@@ -744,7 +810,7 @@ __global__ __launch_bounds__((ZWShape<T, L>::NT)) void zstep_wave_k(ZStepArgs a)
         if constexpr (i == 2) {
           const double kxs = a.kx[kx + mo.md];
 #pragma unroll
-          for (int q = 0; q < 8; ++q) sponge_term<T>(a, mo, kxs, b0 + line, l + q * G, r[0][q], r[1][q], r[2][q]);
+          for (int q = 0; q < 8; ++q) sponge_term<T>(a, mo, kxs, b0 + line < nyq ? zrow(a, b0 + line) : a.ny, l + q * G, r[0][q], r[1][q], r[2][q]);
         }
       } else {
 #pragma unroll
@@ -765,20 +831,28 @@ __global__ __launch_bounds__((ZWShape<T, L>::NT)) void zstep_wave_k(ZStepArgs a)
   const double wE = (kx == 0 || kx == a.nx / 2) ? 0.5 : 1.0;
   double esum = 0.0, ecomp = 0.0;
   const bool final_stage = mg_final_stage<MG>(a);
-  const int ky = b0 + line;
-  if (ky < a.ny) {
+  if (b0 + line < nyq) {
+    const int ky = zrow(a, b0 + line);
+    const ZLim zl = zlim_at<T>(a, kx, (a.prune & 2) ? b0 + line : zpos(a, ky));
     // fixed-mode kernels: operands loaded one position ahead (ZPre)
     constexpr bool AHEAD = MG >= MG_FIXED;
     ZPre<T> pre[2];
-    if constexpr (AHEAD) zpreload<T, MG>(a, mo, kx, ky, l, pre[0]);
+    auto preload = [&](int q, ZPre<T>& pr) {
+      const int kzi = l + q * G;
+      const unsigned off = zl.in(kzi, a.nz) ? (((unsigned)kx * a.ny + ky) * a.nz + kzi) * (unsigned)sizeof(cplx<T>) : kOob;
+      zpreload<T, MG>(a, mo, off, ky, kzi, pr);
+    };
+    if constexpr (AHEAD) preload(0, pre[0]);
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
       if constexpr (AHEAD)
-        if (q + 1 < 8) zpreload<T, MG>(a, mo, kx, ky, l + (q + 1) * G, pre[(q + 1) & 1]);
+        if (q + 1 < 8) preload(q + 1, pre[(q + 1) & 1]);
+      if (!zl.out(l + q * G)) continue;
       cplx<T> rv[3];
 #pragma unroll
       for (int f = 0; f < 3; ++f) rv[f] = r[f][q];
-      zepilogue<T, false, MG, SPONGE>(a, mo, kx, ky, l + q * G, rv, kxv, kxt2, wE, final_stage, esum, ecomp, &pre[q & 1]);
+      zepilogue<T, false, MG, SPONGE>(a, mo, kx, ky, l + q * G, rv, kxv, kxt2, wE, final_stage, esum, ecomp,
+                                      zl.in(l + q * G, a.nz), &pre[q & 1]);
     }
   }
   if (final_stage && a.energy_partial) {
@@ -796,13 +870,20 @@ __global__ __launch_bounds__((ZWShape<T, L>::NT)) void zstep_wave_k(ZStepArgs a)
 // The in-wave kernel holds eight positions of three fields per lane; at
 // nz = 512 that exceeds its register budget (it spilled 48-130 bytes per lane
 // in every stepper family), so nz = 512 always takes the block kernel.
+#if FLUSI_PART == 0
 bool zstep_wave_supported(int nz) { return nz == 64 || nz == 128 || nz == 256; }
 
+int zstep_tile_lines(int nz, bool fp64, bool wave) {
+  return (wave && zstep_wave_supported(nz)) ? (fp64 ? Tile<double>::TL : Tile<float>::TL)
+                                            : (fp64 ? zb_tl<double>(nz) : zb_tl<float>(nz));
+}
+
 int zstep_blocks(int nz, int ny, int nxh, bool fp64, bool wave) {
-  const int TL = (wave && zstep_wave_supported(nz)) ? (fp64 ? Tile<double>::TL : Tile<float>::TL)
-                                               : (fp64 ? zb_tl<double>(nz) : zb_tl<float>(nz));
+  const int TL = zstep_tile_lines(nz, fp64, wave);
   return ((ny + TL - 1) / TL) * nxh;
 }
+
+#endif
 
 template <typename T, int L, bool SP, int MG, int EU>
 static void run_zb(const ZStepArgs& a, hipStream_t s) {
@@ -811,7 +892,7 @@ static void run_zb(const ZStepArgs& a, hipStream_t s) {
   const size_t smem = ZBShape<T, L, TL>::smem;
   static bool init = false;
   if (!init) { set_smem(zstep_k<T, L, TL, NT, SP, MG, EU>, smem); init = true; }
-  dim3 grid((a.ny + TL - 1) / TL, a.nxh, batch_n(a.bat));
+  const dim3 grid = a.tiles ? dim3(a.ntiles, 1, batch_n(a.bat)) : dim3((a.ny + TL - 1) / TL, a.nxh, batch_n(a.bat));
   hipLaunchKernelGGL((zstep_k<T, L, TL, NT, SP, MG, EU>), grid, dim3(NT), smem, s, a);
 }
 
@@ -822,7 +903,8 @@ static void run_z(const ZStepArgs& a, hipStream_t s) {
       using Sh = ZWShape<T, L>;
       static bool winit = false;
       if (!winit) { set_smem(zstep_wave_k<T, L, SP, MG>, Sh::smem); winit = true; }
-      dim3 grid((a.ny + Sh::TL - 1) / Sh::TL, a.nxh, batch_n(a.bat));
+      const dim3 grid = a.tiles ? dim3(a.ntiles, 1, batch_n(a.bat))
+                                : dim3((a.ny + Sh::TL - 1) / Sh::TL, a.nxh, batch_n(a.bat));
       hipLaunchKernelGGL((zstep_wave_k<T, L, SP, MG>), grid, dim3(Sh::NT), Sh::smem, s, a);
       return;
     }
@@ -850,9 +932,9 @@ static bool fixed_mode_ok(const ZStepArgs& a) {
 }
 template <typename T, int L, bool SP>
 static void run_z_mg(const ZStepArgs& a, hipStream_t s) {
-  // fixed-mode kernels: without the sponge, nz >= 64, the default epilogue
+  // fixed-mode kernels: without the sponge and with the default epilogue
   // grouping (the other variants keep the run-time mode)
-  if constexpr (!SP && L >= 64) {
+  if constexpr (!SP) {
     if (fixed_mode_ok(a) && (L < 256 || a.eu == 0 || (L == 256 && a.wave))) {
       switch (a.mode) {
         case SM_EULER: run_z<T, L, SP, MG_FIXED + SM_EULER>(a, s); return;
@@ -879,24 +961,44 @@ static void run_z_sp(const ZStepArgs& a, hipStream_t s) {
   if (a.sponge) run_z_mg<T, L, true>(a, s); else run_z_mg<T, L, false>(a, s);
 }
 
-template <typename T>
-void launch_zstep(const ZStepArgs& a, hipStream_t s) {
+// The instantiations are compiled in four parts (build.py), by element type
+// and line length: 0, 1 - FP32, 2, 3 - FP64; the even parts up to nz = 128.
+#ifndef FLUSI_PART
+#error "FLUSI_PART (0..3) selects the instantiations"
+#endif
+template <typename T> void launch_zstep_short(const ZStepArgs& a, hipStream_t s);  // nz <= 128
+template <typename T> void launch_zstep_long(const ZStepArgs& a, hipStream_t s);
+using PartT = std::conditional_t<(FLUSI_PART < 2), float, double>;
+#if FLUSI_PART % 2 == 0
+template <> void launch_zstep_short<PartT>(const ZStepArgs& a, hipStream_t s) {
   switch (a.nz) {
-    case 16: run_z_sp<T, 16>(a, s); break;
-    case 24: run_z_sp<T, 24>(a, s); break;
-    case 32: run_z_sp<T, 32>(a, s); break;
-    case 48: run_z_sp<T, 48>(a, s); break;
-    case 64: run_z_sp<T, 64>(a, s); break;
-    case 96: run_z_sp<T, 96>(a, s); break;
-    case 128: run_z_sp<T, 128>(a, s); break;
-    case 192: run_z_sp<T, 192>(a, s); break;
-    case 256: run_z_sp<T, 256>(a, s); break;
-    case 384: run_z_sp<T, 384>(a, s); break;
-    case 512: run_z_sp<T, 512>(a, s); break;
+    case 16: run_z_sp<PartT, 16>(a, s); break;
+    case 24: run_z_sp<PartT, 24>(a, s); break;
+    case 32: run_z_sp<PartT, 32>(a, s); break;
+    case 48: run_z_sp<PartT, 48>(a, s); break;
+    case 64: run_z_sp<PartT, 64>(a, s); break;
+    case 96: run_z_sp<PartT, 96>(a, s); break;
+    case 128: run_z_sp<PartT, 128>(a, s); break;
     default: throw std::runtime_error("unsupported nz " + std::to_string(a.nz));
   }
 }
-template void launch_zstep<float>(const ZStepArgs&, hipStream_t);
-template void launch_zstep<double>(const ZStepArgs&, hipStream_t);
+template <typename T>
+void launch_zstep(const ZStepArgs& a, hipStream_t s) {
+  if ((size_t)a.fs * sizeof(cplx<T>) >= kOob) throw std::runtime_error("z step: field too large for 32-bit offsets");
+  if (a.nz <= 128) launch_zstep_short<T>(a, s);
+  else launch_zstep_long<T>(a, s);
+}
+template void launch_zstep<PartT>(const ZStepArgs&, hipStream_t);
+#else
+template <> void launch_zstep_long<PartT>(const ZStepArgs& a, hipStream_t s) {
+  switch (a.nz) {
+    case 192: run_z_sp<PartT, 192>(a, s); break;
+    case 256: run_z_sp<PartT, 256>(a, s); break;
+    case 384: run_z_sp<PartT, 384>(a, s); break;
+    case 512: run_z_sp<PartT, 512>(a, s); break;
+    default: throw std::runtime_error("unsupported nz " + std::to_string(a.nz));
+  }
+}
+#endif
 
 }  // namespace flusi
