@@ -97,9 +97,9 @@ struct XPassArgs {
   unsigned fbytes;     // bytes of one P field (buffer descriptor)
   const double* kx;    // nxh wavenumbers
   double kx_scale;     // kx = kx_scale * k
-  int wpe;             // one-wave-per-line RHS pass: register budget for 3 waves per SIMD (3) or none (0)
   const void* twM;     // M = nx/2 twiddles
   const void* twN;     // nxh twiddles exp(-2 pi i k / nx)
+  const void* twX;     // nx twiddles exp(-2 pi i m / nx)
   // RHS extras
   const void* mask;    // N reals (element type of the pass)
   const void* us;      // 3N reals, component stride N
@@ -121,7 +121,7 @@ struct XPassArgs {
 __host__ __device__ __forceinline__ void to_member(XPassArgs& a, int m) {
   const long o = (long)m * a.bat.mstride;
   a.in = mshift(a.in, o); a.out = mshift(a.out, o); a.kx = mshift(a.kx, o);
-  a.twM = mshift(a.twM, o); a.twN = mshift(a.twN, o);
+  a.twM = mshift(a.twM, o); a.twN = mshift(a.twN, o); a.twX = mshift(a.twX, o);
   a.mask = mshift(a.mask, o); a.us = mshift(a.us, o); a.partial = mshift(a.partial, o);
 }
 
@@ -192,10 +192,10 @@ bool zstep_wave_supported(int nz);  // in-wave z step (else the block kernel)
 template <typename T> void launch_x_pass(const XPassArgs& a, int mode, hipStream_t s);
 template <typename T> void launch_zstep(const ZStepArgs& a, hipStream_t s);
 int x_pass_blocks(int nx, int nlines, bool fp64);
-// the right-hand-side x pass with one wavefront per line (xrhs_wave.hip)
+// the right-hand-side x pass with pairs of lines inside one wavefront (xrhs_wave.hip)
 template <typename T> void launch_x_rhs_wave(const XPassArgs& a, hipStream_t s);
 bool x_rhs_wave_supported(int nx);
-int x_rhs_wave_blocks(int nx, int nlines);
+int x_rhs_wave_blocks(int nx, int nlines, bool fp64, int nmem);  // per member of a batch of nmem
 // per x line (iy, iz) of [y0, y1] x [z0, z1]: flag[iz ny + iy] = 1 where any
 // mask value of the line is nonzero, else 0 (xrhs_wave.hip)
 template <typename T>

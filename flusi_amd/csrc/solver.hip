@@ -265,6 +265,7 @@ class Solver : public SolverBase {
   double* tab = nullptr;    // kx ky kz kxt2 kyt2 kzt2
   double *kx_d, *ky_d, *kz_d, *kxt2_d, *kyt2_d, *kzt2_d;
   void* tw_z = nullptr; void* tw_y = nullptr; void* tw_M = nullptr; void* tw_N = nullptr;
+  void* tw_X = nullptr;
   double* xpart = nullptr;  // x-pass partial rows (max|u|^2, penalization sums)
   double* caps_d = nullptr;   // bumblebee capsule records
   // insect mask arguments live in device memory, one record per batch member:
@@ -421,16 +422,19 @@ class Solver : public SolverBase {
     if (fft_ok) {
       setup_prune();
       tw_z = make_tw(nz, nz); tw_y = make_tw(ny, ny); tw_M = make_tw(nx / 2, nx / 2); tw_N = make_tw(nxh, nx);
+      tw_X = make_tw(nx, nx);
       if (const char* e = getenv("FLUSI_TILE_WAVE")) twave = atoi(e) != 0;
       if (const char* e = getenv("FLUSI_ZWAVE")) zwave = atoi(e) != 0;
       if (const char* e = getenv("FLUSI_ZSTEP_EU")) zeu = atoi(e);
       if (const char* e = getenv("FLUSI_MASK_FLAGS")) mflag_on = atoi(e) != 0;
       if (const char* e = getenv("FLUSI_TILE_PREFETCH")) tpf = atoi(e) != 0;
-      if (const char* e = getenv("FLUSI_XWAVE_WPE")) xwpe = atoi(e);
-      xwave = x_rhs_wave_supported(nx);
+      // (FP64 nx = 384 with few lines: twelve positions a lane in FP64 leave
+      // one long wave per SIMD; 384x32x32 36 us, block pass 26 us; 384x48x48
+      // 42 / 64 us)
+      xwave = x_rhs_wave_supported(nx) && !(FP64 && nx == 384 && ny * nz < 2048);
       if (const char* e = getenv("FLUSI_XWAVE")) xwave = xwave && atoi(e) != 0;
       // partial rows for either x-pass form, so the variant can change later
-      const int nxb = std::max(x_rhs_wave_supported(nx) ? x_rhs_wave_blocks(nx, ny * nz) : 0,
+      const int nxb = std::max(x_rhs_wave_supported(nx) ? x_rhs_wave_blocks(nx, ny * nz, FP64, 1) : 0,
                                x_pass_blocks(nx, ny * nz, FP64));
       xpart = (double*)dalloc(sizeof(double) * 4 * nxb);
       // room for either z-step form's partials (the variant can change later)
@@ -547,9 +551,7 @@ class Solver : public SolverBase {
   // kernel variants (chosen by autotune(), or by the FLUSI_* environment overrides)
   bool twave = true;        // y/z passes with the line transform inside one wavefront
   bool tpf = true;          // block y/z passes: prefetch the next job's operand
-  // one-wave-per-line x pass: waves-per-SIMD register budget (3 or 0); FP64
-  // keeps the unconstrained allocation (at 3 it would spill ~480 B per lane)
-  int xwpe = FP64 ? 0 : 3;
+  int xwpe = FP64 ? 0 : 3;  // reported with the variant; the x pass fixes its register budgets itself
   void tile(const TilePassArgs& a0, int L, int dir, bool contig_in) {
     TilePassArgs a = a0;
     a.pf = tpf ? 1 : 0;
@@ -626,7 +628,7 @@ class Solver : public SolverBase {
     a.nlines = ny * nz; a.nx = nx; a.ny = ny; a.nz = nz; a.nxh = nxh; a.prow = p_row;
     a.kin = nxh; a.kout = nxh; a.fbytes = pbytes();
     a.kx = kx_d; a.kx_scale = 2.0 * PI / p.xl; a.twM = tw_M; a.twN = tw_N;
-    a.npts = npts; a.wpe = xwpe;
+    a.twX = tw_X; a.npts = npts;
     a.bat = bat;
     return a;
   }
@@ -685,7 +687,7 @@ class Solver : public SolverBase {
     });
     kcheck("x pass");
     if (a.want_stats) {
-      const int nxblocks = xwave ? x_rhs_wave_blocks(nx, ny * nz) : x_pass_blocks(nx, ny * nz, FP64);
+      const int nxblocks = xwave ? x_rhs_wave_blocks(nx, ny * nz, FP64, batch_n(bat)) : x_pass_blocks(nx, ny * nz, FP64);
       for (int m = 0; m < batch_n(bat); ++m) {
         const long o = m * bat.mstride;
         launch_reduce_rows(mshift(xpart, o), nxblocks, 4, mshift(kinds, o), mshift(rmid, o), mshift(red, o), stream);
@@ -798,8 +800,8 @@ class Solver : public SolverBase {
 
   // ------------------------------------------------------------ autotuning
   // The right-hand side has interchangeable kernel variants: in-wave or block
-  // y/z passes, operand prefetch in the block passes, the one-wave-per-line or
-  // the block x pass with its register budget, and the in-wave or block z
+  // y/z passes, operand prefetch in the block passes, the in-wave (line pairs)
+  // or the block x pass, and the in-wave or block z
   // step.  autotune() runs `reps` right-hand sides of the current state (the
   // whole batch when one is active) for every variant the grid allows and
   // keeps the fastest; results are cached per grid, precision, sponge and
@@ -839,14 +841,11 @@ class Solver : public SolverBase {
         if (!pf && tw && tw_all) continue;  // prefetch only acts in block passes
         for (int xv : {1, 0}) {
           if (xv && !xw) continue;
-          for (int wpe : {3, 0}) {
-            if (!xv && wpe == 0) continue;  // register budget only acts in the wave x pass
-            for (int zv : {0, 1}) {
-              if (zv && !zw) continue;
-              for (int eu : {0, 2, 4}) {
-                if (eu && (zv || nz < 256)) continue;  // grouping acts in the block z step at nz >= 256
-                c.push_back(Variant{tw, pf, xv, wpe, zv, eu});
-              }
+          for (int zv : {0, 1}) {
+            if (zv && !zw) continue;
+            for (int eu : {0, 2, 4}) {
+              if (eu && (zv || nz < 256)) continue;  // grouping acts in the block z step at nz >= 256
+              c.push_back(Variant{tw, pf, xv, xwpe, zv, eu});
             }
           }
         }
@@ -2394,9 +2393,9 @@ class Ensemble : public EnsembleBase {
       for (size_t k = 1; k < g.idx.size(); ++k) {
         Solver<T>& m = S(g.idx[k]);
         const void* a[] = {L.uk, L.reg[0], L.reg[1], L.Q, L.P, L.mask, L.us, L.color, L.tab, L.tw_z, L.tw_y, L.tw_M,
-                           L.tw_N, L.xpart, L.zpart, L.dpart, L.red, L.rmid, L.kinds, L.pr.zlim, L.ptiles[1]};
+                           L.tw_N, L.tw_X, L.xpart, L.zpart, L.dpart, L.red, L.rmid, L.kinds, L.pr.zlim, L.ptiles[1]};
         const void* b[] = {m.uk, m.reg[0], m.reg[1], m.Q, m.P, m.mask, m.us, m.color, m.tab, m.tw_z, m.tw_y, m.tw_M,
-                           m.tw_N, m.xpart, m.zpart, m.dpart, m.red, m.rmid, m.kinds, m.pr.zlim, m.ptiles[1]};
+                           m.tw_N, m.tw_X, m.xpart, m.zpart, m.dpart, m.red, m.rmid, m.kinds, m.pr.zlim, m.ptiles[1]};
         for (size_t j = 0; j < sizeof(a) / sizeof(a[0]); ++j)
           if ((const char*)b[j] - (const char*)a[j] != (long)(k * g.stride))
             throw FlusiError(900014, "ensemble: member buffers do not follow the batch layout");

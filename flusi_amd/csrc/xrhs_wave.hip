@@ -1,15 +1,22 @@
-// x pass of the right-hand side with one wavefront per x line (nx/2 = 256),
-// two per wave (128), four (64), five (48) or eight (32).
+// x pass of the right-hand side: two x lines (neighbours in y) per complex
+// transform of length nx, inside one wavefront.
 //
-// Each line is a length-M = nx/2 complex transform (the real transform of
-// length nx through the even/odd split).  A line lives in the registers of
-// G = M/4 lanes, lane l holding positions l + qG (q = 0..3) before and after
-// every transform.  The Stockham stages of radix 4 (one radix-2 stage for
-// M = 128 and 32; radix 3, 4, 4 for M = 48) exchange data through a small
-// per-wave LDS slot with wave-scope ordering only: waves never wait for each
-// other, so a compute unit keeps as many lines in flight as its register
-// file holds.  For M = 48 the five lines use 60 lanes; the other four work
-// on a spare LDS row and store nothing.
+// The lines' spectra A and B are combined to Z = A + i B over all nx modes
+// (Z[nx - k] = conj A[k] + i conj B[k]), so that one complex transform of
+// length nx gives line a in its real and line b in its imaginary parts, and
+// the other way round.  Against one length-nx/2 transform per line with the
+// even/odd split, a pair needs no split twiddles and, with E = 8 (12 where 3
+// divides nx) positions a lane instead of 4, exchanges its values twice
+// through LDS instead of three or four times: the pass was bound by its VALU
+// issue and its LDS traffic together (nx = 512, FP32: 2000 VALU and 400 LDS
+// instructions a line, 78 % VALU issue).  A pair takes about 2640 VALU and 300
+// LDS instructions: 512^3 FP32 1291 -> 719 us (3.3 GB: 4.6 TB/s), 192x96x384
+// FP32 (block pass before) 205 -> 79 us.
+//
+// A pair lives in the registers of G = nx/E lanes, lane l holding positions
+// l + qG (q = 0..E-1) before and after every transform; 64/G pairs a wave.
+// Stages exchange through the pair's own LDS row with wave-scope ordering
+// only: waves never wait for each other.
 //
 // Per line (rhs.f90:147-330 cal_nlk_fsi, nonlinear and penalisation part):
 //   load the six spectra V_x, V_y, V_z, w_x, A = dz u_x, B = dy u_x
@@ -24,17 +31,16 @@
 #include <stdexcept>
 #include <string>
 
+#ifndef FLUSI_PART
+#define FLUSI_PART 0
+#endif
+
 namespace flusi {
 
 namespace {
 
-constexpr int XW_NT = 256;  // threads of a block: four independent waves
+constexpr int XW_NT = 256;  // most threads of a block: independent waves
 
-template <typename C> __device__ __forceinline__ C conj_w(C a) { a.y = -a.y; return a; }
-template <typename T> __device__ __forceinline__ cplx<T> ik_w(T k, cplx<T> v) { return mk<T>(-k * v.y, k * v.x); }
-
-// orders this wave's LDS writes before its following reads (and the reads
-// before the next writes); no other wave takes part
 __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -52,425 +58,482 @@ __device__ __forceinline__ double wmax(double v) {
   return v;
 }
 
-// Radix plan of the in-wave transform: radix 4 throughout, the last stage of
-// M = 128 and M = 32 is radix 2 (two butterflies per lane).
-template <int M> struct WPlan {
-  static_assert(M == 32 || M == 64 || M == 128 || M == 256, "in-wave transform: M = 32, 64, 128 or 256");
-  static constexpr int G = M / 4;
-  static constexpr int NST = (M <= 64) ? 3 : 4;
-  static constexpr __host__ __device__ int radix(int s) { return ((M == 128 && s == 3) || (M == 32 && s == 2)) ? 2 : 4; }
-  // sub-transform length entering stage s (only the last stage can be radix 2)
-  static constexpr __host__ __device__ int ns(int s) { return 1 << (2 * s); }
+// Radix-12 butterfly as 3 x 4 (prime factors: no twiddles between them).
+// Input n = (4 n1 + 3 n2) mod 12, output k = (4 (k mod 3) + 9 (k mod 4)) mod 12.
+template <int S, typename T> struct Bfly12 {
+  static __device__ __forceinline__ void run(cplx<T>* a) {
+    cplx<T> t[3][4];
+#pragma unroll
+    for (int n2 = 0; n2 < 4; ++n2) {
+      cplx<T> x[3] = {a[(3 * n2) % 12], a[(4 + 3 * n2) % 12], a[(8 + 3 * n2) % 12]};
+      Bfly<3, S, T>::run(x);
+#pragma unroll
+      for (int k1 = 0; k1 < 3; ++k1) t[k1][n2] = x[k1];
+    }
+#pragma unroll
+    for (int k1 = 0; k1 < 3; ++k1) {
+      Bfly<4, S, T>::run(t[k1]);
+#pragma unroll
+      for (int k2 = 0; k2 < 4; ++k2) a[(4 * k1 + 9 * k2) % 12] = t[k1][k2];
+    }
+  }
 };
 
-// lp(b + k) = lp(b) + lp(k) for the padded LDS accesses of the length-M
-// transform: every stage's write base b with offsets q Ns, the lane's read
-// base l with offsets q G and, with MIRROR, the mirrored base G - l with
-// offsets q G.  Where it holds, one address per lane and stage serves all
-// four elements through the LDS instruction's immediate offset.
-template <typename T, int M> constexpr bool split_ok(bool mirror) {
-  if constexpr (M == 48) {
-    return false;  // the radix-3 plan addresses its rows itself
-  } else {
-    constexpr int G = M / 4;
-    for (int l = 0; l < G; ++l) {
-      for (int q = 0; q < 4; ++q) {
-        if (lp<T>(l + q * G) != lp<T>(l) + lp<T>(q * G)) return false;
-        if (mirror && lp<T>(G - l + q * G) != lp<T>(G - l) + lp<T>(q * G)) return false;
-      }
-      for (int s = 0; s + 1 < WPlan<M>::NST; ++s) {
-        if (WPlan<M>::radix(s) != 4) return false;
-        const int Ns = WPlan<M>::ns(s), b = (l / Ns) * Ns * 4 + l % Ns;
-        for (int q = 0; q < 4; ++q)
-          if (lp<T>(b + q * Ns) != lp<T>(b) + lp<T>(q * Ns)) return false;
-      }
+// E = 8: 512 = 8.8.8, 256 = 8.8.4, 128 = 8.4.4, 64 = 8.8, 32 = 8.4;
+// E = 4: 256 = 4.4.4.4, 128 = 4.4.4.2, 64 = 4.4.4, 32 = 4.4.2, 96 = 6.4.4 (its
+// first stage reads its inputs from the row, see pstage0);
+// E = 12: 384 = 12.4.4.2, 192 = 12.4.4, 96 = 12.4.2, 48 = 12.4
+template <int N_, int E_> struct PairPlan {
+  static constexpr int N = N_, E = E_;
+  static constexpr int G = N / E;     // lanes of a pair
+  static constexpr int PPW = 64 / G;  // pairs of a wave
+  static constexpr int ROWS = PPW + (PPW * G < 64 ? 1 : 0);  // a spare row for lanes beyond PPW pairs
+  static constexpr bool ROW0 = E == 4 && N % 3 == 0;
+  static_assert(E * G == N && (PPW * G == 64 || N == 96), "in-wave pair length");
+  static constexpr __host__ __device__ int radix(int s) {
+    int m = N;
+    for (int i = 0;; ++i) {
+      const int r = i == 0 ? (ROW0 ? 6 : E) : (E == 8 && (m == 8 || m == 64 || m == 32) ? 8 : (m % 4 == 0 ? 4 : 2));
+      if (i == s) return r;
+      m /= r;
     }
-    return true;
   }
+  static constexpr __host__ __device__ int ns(int s) { int p = 1; for (int i = 0; i < s; ++i) p *= radix(i); return p; }
+  static constexpr int QL = (E + 2) / 3;  // groups l + qG that hold the modes of a dealiased state (k < N/3 + 1)
+};
+
+// lp(b + k) = lp(b) + lp(k) for a lane's accesses: one address per lane and
+// stage then serves all elements through the instruction's immediate offset
+template <typename T, typename PP> constexpr bool split_rd() {
+  for (int l = 0; l < PP::G; ++l)
+    for (int q = 0; q < PP::E; ++q)
+      if (lp<T>(l + q * PP::G) != lp<T>(l) + lp<T>(q * PP::G) || lp<T>(PP::G - l + q * PP::G) != lp<T>(PP::G - l) + lp<T>(q * PP::G))
+        return false;
+  return true;
+}
+template <typename T, typename PP, int s> constexpr bool split_wr() {
+  constexpr int N = PP::N;
+  constexpr int R = PP::radix(s), Ns = PP::ns(s);
+  for (int j = 0; j < N / R; ++j)
+    for (int q = 0; q < R; ++q) {
+      const int b = (j / Ns) * Ns * R + j % Ns;
+      if (lp<T>(b + q * Ns) != lp<T>(b) + lp<T>(q * Ns)) return false;
+    }
+  return true;
 }
 
-template <int S, typename C> __device__ __forceinline__ C twm(C v, C w) {
-  return (S < 0) ? cmul(v, w) : conjmul(v, w);
+// radix 6 as 2 x 3: input n = (3 n1 + 2 n2) mod 6, output k = (3 (k mod 2) + 4 (k mod 3)) mod 6
+template <int S, typename T> struct Bfly6 {
+  static __device__ __forceinline__ void run(cplx<T>* a) {
+    cplx<T> x[3] = {a[0], a[2], a[4]}, y[3] = {a[3], a[5], a[1]};
+    Bfly<3, S, T>::run(x);
+    Bfly<3, S, T>::run(y);
+#pragma unroll
+    for (int k2 = 0; k2 < 3; ++k2) {
+      a[(4 * k2) % 6] = add(x[k2], y[k2]);
+      a[(3 + 4 * k2) % 6] = sub(x[k2], y[k2]);
+    }
+  }
+};
+template <int R, int S, typename T> __device__ __forceinline__ void bfly(cplx<T>* a) {
+  if constexpr (R == 12) Bfly12<S, T>::run(a);
+  else if constexpr (R == 6) Bfly6<S, T>::run(a);
+  else Bfly<R, S, T>::run(a);
 }
 
-// Stage s of the in-wave Stockham transform.  Inputs: v[q] = x[l + qG].
-// Outputs of butterfly j go to (j / Ns) Ns R + j % Ns + q Ns; all but the
-// last stage pass them through the wave's LDS line `ln` and read back
-// positions l + qG.  The last stage's outputs already sit at l + qG.
-// tw: the block's LDS copy of exp(-2 pi i m / M), m < M.
-template <typename T, int M, int S, int s>
-__device__ __forceinline__ void wstage(cplx<T> (&v)[4], const cplx<T>* tw, cplx<T>* ln, int l) {
-  // index arithmetic on the unsigned lane index: l % Ns and l / Ns are then
-  // a mask and a shift (on a signed int the compiler has to allow l < 0,
-  // which costs four instructions each)
-  const unsigned ul = (unsigned)l;
-  constexpr int G = WPlan<M>::G;
-  constexpr int R = WPlan<M>::radix(s), Ns = WPlan<M>::ns(s);
-  constexpr bool last = (s == WPlan<M>::NST - 1);
-  if (R == 4) {
-    if (s > 0) {
-      const int step = (int)(ul % Ns) * (M / (Ns * 4));
+// reads positions l + qG of the pair's row
+template <typename T, typename PP> __device__ __forceinline__ void row_read(cplx<T> (&v)[PP::E], const cplx<T>* ln, int l) {
+  constexpr int E = PP::E, G = PP::G;
+  const cplx<T>* rd = ln + lp<T>(l);
 #pragma unroll
-      for (int q = 1; q < 4; ++q) v[q] = twm<S>(v[q], tw[q * step]);
-    }
-    Bfly<4, S, T>::run(v);
-    if (!last) {
-      const int base = (int)(ul / Ns) * Ns * 4 + (int)(ul % Ns);
-      if constexpr (split_ok<T, M>(false)) {
-        cplx<T>* wr = ln + lp<T>(base);
+  for (int q = 0; q < E; ++q) v[q] = split_rd<T, PP>() ? rd[lp<T>(q * G)] : ln[lp<T>(l + q * G)];
+}
+
+// Stage s: B = E/R butterflies per lane, j = l + bG; input q of butterfly b
+// is register b + qB (position j + q N/R); outputs go to (j/Ns) Ns R + j%Ns +
+// q Ns, which for the last stage is again register b + qB.  tw: the block's
+// LDS copy of exp(-2 pi i m / N).
+template <typename T, typename PP, int S, int s>
+__device__ __forceinline__ void pstage(cplx<T> (&v)[PP::E], const cplx<T>* tw, cplx<T>* ln, int l) {
+  constexpr int N = PP::N, E = PP::E, G = PP::G, R = PP::radix(s), Ns = PP::ns(s), B = E / R;
+  constexpr bool last = Ns * R == N;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) wr[lp<T>(q * Ns)] = v[q];
-      } else {
+  for (int b = 0; b < B; ++b) {
+    const unsigned j = (unsigned)l + b * G;
+    cplx<T> x[R];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) ln[lp<T>(base + q * Ns)] = v[q];
-      }
+    for (int q = 0; q < R; ++q) x[q] = v[b + q * B];
+    if constexpr (s > 0) {
+      const int step = (int)(j % Ns) * (N / (Ns * R));
+#pragma unroll
+      for (int q = 1; q < R; ++q) x[q] = (S < 0) ? cmul(x[q], tw[q * step]) : conjmul(x[q], tw[q * step]);
     }
-  } else {
-    // butterflies j = l on (v0, v2) and j = l + G on (v1, v3)
-    if (s > 0) {
-      v[2] = twm<S>(v[2], tw[(int)(ul % Ns) * (M / (Ns * 2))]);
-      v[3] = twm<S>(v[3], tw[(int)((ul + G) % Ns) * (M / (Ns * 2))]);
-    }
-    cplx<T> a0[2] = {v[0], v[2]}, a1[2] = {v[1], v[3]};
-    Bfly<2, S, T>::run(a0);
-    Bfly<2, S, T>::run(a1);
-    if (!last) {
-      const int b0 = (int)(ul / Ns) * Ns * 2 + (int)(ul % Ns), b1 = (int)((ul + G) / Ns) * Ns * 2 + (int)((ul + G) % Ns);
-      ln[lp<T>(b0)] = a0[0]; ln[lp<T>(b0 + Ns)] = a0[1];
-      ln[lp<T>(b1)] = a1[0]; ln[lp<T>(b1 + Ns)] = a1[1];
+    bfly<R, S, T>(x);
+    if constexpr (last) {
+#pragma unroll
+      for (int q = 0; q < R; ++q) v[b + q * B] = x[q];
     } else {
-      v[0] = a0[0]; v[2] = a0[1]; v[1] = a1[0]; v[3] = a1[1];
+      const int base = (int)(j / Ns) * Ns * R + (int)(j % Ns);
+      cplx<T>* wr = ln + lp<T>(base);
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        if constexpr (split_wr<T, PP, s>()) wr[lp<T>(q * Ns)] = x[q];
+        else ln[lp<T>(base + q * Ns)] = x[q];
+      }
     }
   }
-  if (!last) {
+  if constexpr (!last) {
     wave_sync();
-    if constexpr (split_ok<T, M>(false)) {
-      const cplx<T>* rd = ln + lp<T>(l);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) v[q] = rd[lp<T>(q * G)];
-    } else {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) v[q] = ln[lp<T>(l + q * G)];
-    }
+    row_read<T, PP>(v, ln, l);
     wave_sync();
+    pstage<T, PP, S, s + 1>(v, tw, ln, l);
   }
 }
 
-template <typename T, int M, int S>
-__device__ __forceinline__ void wfft(cplx<T> (&v)[4], const cplx<T>* tw, cplx<T>* ln, int l_) {
+// Stage 0 of a plan whose first radix is not the lane's E (96 = 6.4.4 over 24
+// lanes): the row holds the inputs at their positions, the first N/R lanes
+// take one butterfly each.
+template <typename T, typename PP, int S>
+__device__ __forceinline__ void pstage0(cplx<T> (&v)[PP::E], const cplx<T>* tw, cplx<T>* ln, int l) {
+  constexpr int N = PP::N, R = PP::radix(0);
+  const int j = l < N / R ? l : 0;
+  cplx<T> x[R];
+#pragma unroll
+  for (int q = 0; q < R; ++q) x[q] = ln[lp<T>(j + q * (N / R))];
+  wave_sync();
+  bfly<R, S, T>(x);
+  if (l < N / R) {
+#pragma unroll
+    for (int q = 0; q < R; ++q) ln[lp<T>(R * j + q)] = x[q];
+  }
+  wave_sync();
+  row_read<T, PP>(v, ln, l);
+  wave_sync();
+  pstage<T, PP, S, 1>(v, tw, ln, l);
+}
+
+// (a plan with ROW0: the row holds the inputs)
+template <typename T, typename PP, int S>
+__device__ __forceinline__ void pfft(cplx<T> (&v)[PP::E], const cplx<T>* tw, cplx<T>* ln, int l_) {
   // recompute the LDS addresses in every transform instead of keeping a
   // few dozen of them live across the whole kernel
   int l = l_;
   asm volatile("" : "+v"(l));
-  wstage<T, M, S, 0>(v, tw, ln, l);
-  wstage<T, M, S, 1>(v, tw, ln, l);
-  wstage<T, M, S, 2>(v, tw, ln, l);
-  if constexpr (WPlan<M>::NST > 3) wstage<T, M, S, 3>(v, tw, ln, l);
+  if constexpr (PP::ROW0) pstage0<T, PP, S>(v, tw, ln, l);
+  else pstage<T, PP, S, 0>(v, tw, ln, l);
 }
 
-// M = 48 = 3 x 4 x 4 (nx = 96).  Stage 0 (radix 3) has 16 butterflies for
-// the 12 lanes of a line, so every stage reads its butterflies' inputs from
-// the line's LDS row: butterfly j of stage 0 reads j + 16q and writes 3j + q
-// (lanes 0..3 also take butterflies 12..15); stage 1 (radix 4, Ns = 3) reads
-// j + 12q and writes (j/3) 12 + j%3 + 3q; stage 2 (radix 4, Ns = 12) reads
-// j + 12q and leaves its outputs at j + 12q, the lane's own positions.
-template <typename T, int S>
-__device__ __forceinline__ void wfft48(cplx<T> (&v)[4], const cplx<T>* tw, cplx<T>* ln, int l_) {
-  int l = l_;
-  asm volatile("" : "+v"(l));
-#pragma unroll
-  for (int q = 0; q < 4; ++q) ln[lp<T>(l + 12 * q)] = v[q];
-  wave_sync();
-  const bool two = l < 4;
-  cplx<T> a[3], b[3];
-#pragma unroll
-  for (int q = 0; q < 3; ++q) {
-    a[q] = ln[lp<T>(l + 16 * q)];
-    b[q] = ln[lp<T>((two ? 12 + l : l) + 16 * q)];
-  }
-  wave_sync();
-  Bfly<3, S, T>::run(a);
-#pragma unroll
-  for (int q = 0; q < 3; ++q) ln[lp<T>(3 * l + q)] = a[q];
-  if (two) {
-    Bfly<3, S, T>::run(b);
-#pragma unroll
-    for (int q = 0; q < 3; ++q) ln[lp<T>(3 * (12 + l) + q)] = b[q];
-  }
-  wave_sync();
-#pragma unroll
-  for (int q = 0; q < 4; ++q) v[q] = ln[lp<T>(l + 12 * q)];
-  wave_sync();
-  {
-    const int step = (l % 3) * 4;
-#pragma unroll
-    for (int q = 1; q < 4; ++q) v[q] = twm<S>(v[q], tw[q * step]);
-    Bfly<4, S, T>::run(v);
-    const int base = (l / 3) * 12 + (l % 3);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) ln[lp<T>(base + 3 * q)] = v[q];
-  }
-  wave_sync();
-#pragma unroll
-  for (int q = 0; q < 4; ++q) v[q] = ln[lp<T>(l + 12 * q)];
-  wave_sync();
-#pragma unroll
-  for (int q = 1; q < 4; ++q) v[q] = twm<S>(v[q], tw[q * l]);
-  Bfly<4, S, T>::run(v);
+// i k x a pair's combined modes: Z takes i kx Z, the mirrored M its conjugate
+template <typename T> __device__ __forceinline__ cplx<T> ik_p(T k, cplx<T> v) { return mk<T>(-k * v.y, k * v.x); }
+
+// complex load through a buffer with a wave-uniform byte offset on top of the
+// lane's (an out-of-range lane offset reads zero).  Stores carry the whole
+// offset in the lane's register (bst): the hazard of a 16-byte store whose data
+// registers the next instruction overwrites is not covered by the compiler
+// where the store has a scalar offset (seen: four lanes' data replaced).
+template <typename T> __device__ __forceinline__ cplx<T> bld_s(brsrc r, unsigned off, unsigned soff) {
+  if constexpr (sizeof(T) == 4) return __builtin_bit_cast(cplx<T>, __builtin_amdgcn_raw_buffer_load_b64(r, off, soff, 0));
+  else return __builtin_bit_cast(cplx<T>, __builtin_amdgcn_raw_buffer_load_b128(r, off, soff, 0));
+}
+// one real through a buffer
+template <typename T> __device__ __forceinline__ T rld(brsrc r, unsigned off) {
+  if constexpr (sizeof(T) == 4) return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+  else return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
+}
+template <typename T, int N> constexpr int pair_row() { return line_stride<T>(N + 1); }
+template <typename T, typename PP> constexpr size_t pair_smem(int waves) {
+  return sizeof(cplx<T>) * ((size_t)waves * PP::ROWS * pair_row<T, PP::N>() + PP::N);
 }
 
-template <typename T, int M, int S>
-__device__ __forceinline__ void wtransform(cplx<T> (&v)[4], const cplx<T>* tw, cplx<T>* ln, int l) {
-  if constexpr (M == 48) wfft48<T, S>(v, tw, ln, l);
-  else wfft<T, M, S>(v, tw, ln, l);
+// waves per SIMD the register allocation must allow
+template <typename T, int N, int E, int VAR, int PR> constexpr int pair_wpe() {
+  if (E == 12) return sizeof(T) == 4 ? 2 : 1;
+  if (E == 4) return sizeof(T) == 4 ? 4 : (N % 3 == 0 ? 2 : 3);
+  return sizeof(T) == 4 ? (VAR == 0 && PR > 0 ? 4 : 3) : 2;
 }
 
-// WPE: minimum waves per SIMD the register allocation must allow (0: none)
-template <typename T, int M, bool SPONGE, bool STATS, int WPE>
-__global__ __launch_bounds__(XW_NT) __attribute__((amdgpu_waves_per_eu(WPE > 0 ? WPE : 1))) void x_rhs_wave_k(XPassArgs a) {
+// PR 1: the spectra are zero at k >= QL G (a dealiased state), so that only QL
+// groups a line are loaded and mirrored; PR 2: no more are stored, either.
+// VAR: 0 plain, 1 with the statistics, 2 sponge (and the statistics if asked)
+template <typename T, int N, int E, int VAR, int PR>
+__global__ __launch_bounds__(XW_NT) __attribute__((amdgpu_waves_per_eu(pair_wpe<T, N, E, VAR, PR>()))) void x_rhs_pair_k(XPassArgs a) {
   to_member(a, blockIdx.y);
-  constexpr int G = M / 4, LPW = 64 / G, NXH = M + 1;
-  constexpr int LS = line_stride<T>(M + 1);
-  constexpr int WPB = XW_NT / 64;
-  constexpr int NFO = SPONGE ? 6 : 3;
-  constexpr int ROWS = LPW + (LPW * G < 64 ? 1 : 0);  // a spare row for lanes beyond LPW lines
-  __shared__ cplx<T> sh[WPB][ROWS * LS];
-  __shared__ cplx<T> twl[M], twn[NXH];
-  __shared__ double red[WPB][4];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  using PP = PairPlan<N, E>;
+  constexpr int G = PP::G, PPW = PP::PPW, H = E / 2;
+  constexpr bool PIN = PR > 0;
+  constexpr int QL = PIN ? PP::QL : H, QO = PR == 2 ? PP::QL : H;
+  constexpr int LS = pair_row<T, N>();
+  constexpr bool SPONGE = VAR == 2;
+  constexpr unsigned ES = sizeof(cplx<T>);
+  extern __shared__ char smem_raw[];
+  __shared__ double red[XW_NT / 64][4];
+  cplx<T>* twl = reinterpret_cast<cplx<T>*>(smem_raw);
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, wpb = blockDim.x >> 6;
   const int l = lane % G;
-  const int gl = (blockIdx.x * WPB + wv) * LPW + lane / G;
-  const bool live = lane < LPW * G && gl < a.nlines;
-  cplx<T>* ln = sh[wv] + (lane / G) * LS;
+  const int pair = (blockIdx.x * wpb + wv) * PPW + lane / G;  // lines 2 pair, 2 pair + 1
+  const bool live = lane < PPW * G && 2 * pair < a.nlines;
+  const int gl = live ? 2 * pair : 0;
+  cplx<T>* ln = twl + N + (wv * PP::ROWS + lane / G) * LS;
+  const bool stats = VAR == 1 || (VAR == 2 && a.want_stats);
 
-  // global-address-space views of the arguments (see gptr)
-  const gptr<const cplx<T>> twM = (gptr<const cplx<T>>)a.twM;
-  const gptr<const cplx<T>> twN = (gptr<const cplx<T>>)a.twN;
-  const gptr<const cplx<T>> in = (gptr<const cplx<T>>)a.in;
-  const gptr<cplx<T>> out = (gptr<cplx<T>>)a.out;
-  const gptr<const T> mask = (gptr<const T>)a.mask;
-  const gptr<const T> us = (gptr<const T>)a.us;
+  {
+    const gptr<const cplx<T>> t = (gptr<const cplx<T>>)a.twX;
+    for (int i = threadIdx.x; i < N; i += blockDim.x) twl[i] = gld<T>(t + i);
+  }
 
-  for (int i = threadIdx.x; i < M; i += XW_NT) twl[i] = gld<T>(twM + i);
-  for (int i = threadIdx.x; i < NXH; i += XW_NT) twn[i] = gld<T>(twN + i);
-
-  // ---- loads: six spectra at k = l + qG and k = M
-  cplx<T> X[6][4], XM[6];
-  const long lb = (long)(live ? gl : 0) * a.prow;
+  // ---- loads: the two lines' spectra at k = l + qG in X[f][q] and
+  // X[f][E - QL + q], and (not PIN) at k = N/2 on lane 0
+  const unsigned rowb = (unsigned)a.prow * ES;
+  const unsigned lb = (unsigned)gl * rowb + (unsigned)l * ES;
+  auto field = [&](const void* base, long stride, int f) {
+    return make_brsrc(reinterpret_cast<const cplx<T>*>(base) + f * stride, a.fbytes);
+  };
+  cplx<T> X[6][E], nyq[6];
 #pragma unroll
   for (int f = 0; f < 6; ++f) {
-    const gptr<const cplx<T>> p = in + f * a.fstride_in + lb;
+    const brsrc r = field(a.in, a.fstride_in, f);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) X[f][q] = l + q * G < a.kin ? gld<T>(p + l + q * G) : mk<T>(T(0), T(0));
-    XM[f] = M < a.kin ? gld<T>(p + M) : mk<T>(T(0), T(0));
+    for (int q = 0; q < QL; ++q) {
+      const unsigned off = live && l + q * G < a.kin ? lb + q * G * ES : kOob;
+      X[f][q] = bld_s<T>(r, off, 0);
+      X[f][E - QL + q] = bld_s<T>(r, off, rowb);
+    }
+    if constexpr (!PIN) {
+      const unsigned off = live && l == 0 && N / 2 < a.kin ? lb + N / 2 * ES : kOob;
+      const cplx<T> xa = bld_s<T>(r, off, 0), xb = bld_s<T>(r, off, rowb);
+      nyq[f] = xa;  // (real part of line a, of line b); w below
+      nyq[f].y = xb.x;
+      if (f == 4 || f == 5) {  // w_y = A - i kx V_z, w_z = i kx V_y - B: real parts at k = N/2
+        const T kx = (T)(a.kx_scale * double(N / 2));
+        const brsrc rv = field(a.in, a.fstride_in, f == 4 ? 2 : 1);
+        const cplx<T> va = bld_s<T>(rv, off, 0), vb = bld_s<T>(rv, off, rowb);
+        nyq[f] = f == 4 ? mk<T>(xa.x + kx * va.y, xb.x + kx * vb.y) : mk<T>(-kx * va.y - xa.x, -kx * vb.y - xb.x);
+      }
+    }
   }
-
-  // mask at the physical points 2n, 2n+1 (n = l + qG), read early; a line
-  // whose flag says its mask is all zero (most lines of a flow around a
-  // small body) reads the shared zero row instead, which stays in cache
-  cplx<T> mk2[4];
-  {
-    const long ml = live ? gl : 0;
-    const bool zero_line = a.mflag && ((gptr<const uint8_t>)a.mflag)[ml] == 0;
-    const gptr<const T> mrow = zero_line ? (gptr<const T>)a.mzero : mask + ml * a.nx;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) mk2[q] = gld<T>(reinterpret_cast<gptr<const cplx<T>>>(mrow + 2 * (l + q * G)));
+  // Whether any line of the wave meets the mask.  The mask and us are read
+  // through buffers, whose out-of-range offset stands for "not needed"; a line
+  // whose flag says that its mask is all zero is not read.
+  const brsrc rm = make_brsrc(a.mask, (unsigned)(a.npts * sizeof(T)));
+  const unsigned pb = (unsigned)(gl * N + l) * (unsigned)sizeof(T);
+  bool ma = live, mb = live;
+  if (a.mflag) {
+    ma = live && ((gptr<const uint8_t>)a.mflag)[gl] != 0;
+    mb = live && ((gptr<const uint8_t>)a.mflag)[gl + 1] != 0;
   }
-
-  __syncthreads();  // twiddle tables (the only block-wide wait besides the statistics)
-
-  // ---- w_y = A - i kx V_z, w_z = i kx V_y - B
+  bool masked = ma || mb;
+  if (!a.mflag) {  // no flags (members of a batch): the wave looks at its own points
+    bool any = false;
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < E; ++q) {
+      const unsigned pq = live ? pb + (unsigned)(q * G) * sizeof(T) : kOob;
+      any = any || rld<T>(rm, pq) != T(0) || rld<T>(rm, pq + N * sizeof(T)) != T(0);
+    }
+    masked = any;
+  }
+  masked = __any(masked);
+
+  __syncthreads();  // twiddle table (the only block-wide wait besides the statistics)
+
+  // ---- Z = A + i B and its mirrored modes M = conj A + i conj B, then w_y, w_z
+#pragma unroll
+  for (int f = 0; f < 6; ++f)
+#pragma unroll
+    for (int q = 0; q < QL; ++q) {
+      cplx<T> xa = X[f][q], xb = X[f][E - QL + q];
+      if (q == 0 && l == 0) { xa.y = T(0); xb.y = T(0); }  // a C2R transform ignores these (cof_p3dfft.f90:65-83)
+      X[f][q] = mk<T>(xa.x - xb.y, xa.y + xb.x);
+      X[f][E - QL + q] = mk<T>(xa.x + xb.y, xb.x - xa.y);
+    }
+#pragma unroll
+  for (int q = 0; q < QL; ++q) {
     const T kx = (T)(a.kx_scale * double(l + q * G));
-    X[4][q] = sub(X[4][q], ik_w<T>(kx, X[2][q]));
-    X[5][q] = sub(ik_w<T>(kx, X[1][q]), X[5][q]);
-  }
-  {
-    const T kx = (T)(a.kx_scale * double(M));
-    XM[4] = sub(XM[4], ik_w<T>(kx, XM[2]));
-    XM[5] = sub(ik_w<T>(kx, XM[1]), XM[5]);
+    const int m = E - QL + q;
+    X[4][q] = sub(X[4][q], ik_p<T>(kx, X[2][q]));
+    X[5][q] = sub(ik_p<T>(kx, X[1][q]), X[5][q]);
+    X[4][m] = add(X[4][m], ik_p<T>(kx, X[2][m]));
+    X[5][m] = sub(ik_p<T>(-kx, X[1][m]), X[5][m]);
   }
 
-  // ---- C2R of the six fields: z[n] = x[2n] + i x[2n+1] at n = l + qG
+  // ---- C2R of the six fields
 #pragma unroll
   for (int f = 0; f < 6; ++f) {
     // one field at a time: keeps the scheduler from interleaving the
     // independent transforms (their temporaries would exhaust the registers)
     __builtin_amdgcn_sched_barrier(0);
-    cplx<T> xb[4];
-    if constexpr (split_ok<T, M>(true)) {
-      // positions l + qG and their mirrors M - l - qG = (G - l) + (3 - q) G
-      int lo = l;
-      asm volatile("" : "+v"(lo));
-      cplx<T>* rw = ln + lp<T>(lo);
-      const cplx<T>* mr = ln + lp<T>(G - lo);
+    int lo = l;
+    asm volatile("" : "+v"(lo));
+    if constexpr (PP::ROW0) {
+      // the whole of Z goes to the row, from which the first stage reads
 #pragma unroll
-      for (int q = 0; q < 4; ++q) rw[lp<T>(q * G)] = X[f][q];
-      if (lo == 0) ln[lp<T>(M)] = XM[f];
-      wave_sync();
-#pragma unroll
-      for (int q = 0; q < 4; ++q) xb[q] = mr[lp<T>((3 - q) * G)];
+      for (int q = 0; q < QL; ++q) {
+        ln[lp<T>(lo + q * G)] = X[f][q];
+        ln[lp<T>(N - lo - q * G)] = X[f][E - QL + q];
+      }
+      if (lo == 0) ln[lp<T>(N / 2)] = PIN ? mk<T>(T(0), T(0)) : nyq[f];
       wave_sync();
     } else {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) ln[lp<T>(l + q * G)] = X[f][q];
-      if (l == 0) ln[lp<T>(M)] = XM[f];
+      // mode N - k of k = l + qG comes through the row: position p reads N - p
+      // = (G - l) + (E - 1 - q) G
+      cplx<T>* rw = ln + lp<T>(lo);
+      const cplx<T>* mr = ln + lp<T>(G - lo);
+  #pragma unroll
+      for (int q = 0; q < QL; ++q) {
+        if constexpr (split_rd<T, PP>()) rw[lp<T>(q * G)] = X[f][E - QL + q];
+        else ln[lp<T>(lo + q * G)] = X[f][E - QL + q];
+      }
       wave_sync();
-#pragma unroll
-      for (int q = 0; q < 4; ++q) xb[q] = ln[lp<T>(M - l - q * G)];
+  #pragma unroll
+      for (int q = E - QL; q < E; ++q) {
+        if constexpr (split_rd<T, PP>()) X[f][q] = mr[lp<T>((E - 1 - q) * G)];
+        else X[f][q] = ln[lp<T>(G - lo + (E - 1 - q) * G)];
+      }
       wave_sync();
+      // lane 0's N - p = QL G was not written: k = N/2, or beyond the region
+      if (l == 0) X[f][E - QL] = PIN ? mk<T>(T(0), T(0)) : nyq[f];
+  #pragma unroll
+      for (int q = QL; q < E - QL; ++q) X[f][q] = mk<T>(T(0), T(0));
     }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      cplx<T> xa = X[f][q], xm = xb[q];
-      if (q == 0 && l == 0) { xa.y = T(0); xm.y = T(0); }
-      const cplx<T> s1 = add(xa, conj_w(xm)), d1 = sub(xa, conj_w(xm));
-      X[f][q] = add(s1, ik_w<T>(T(1), cmul(conj_w(twn[l + q * G]), d1)));
-    }
-    wtransform<T, M, +1>(X[f], twl, ln, l);
+    pfft<T, PP, +1>(X[f], twl, ln, l);
   }
 
-  // ---- u x w - chi (u - us) [+ sponge]
+  // ---- u x w - chi (u - us) [+ sponge], in place: X[0..2] (and X[3..5])
   double umax2 = 0.0, fs[3] = {0.0, 0.0, 0.0}, fc[3] = {0.0, 0.0, 0.0};
-  cplx<T> O[NFO][4];
-  const int iy = live ? gl % a.ny : 0, iz = live ? gl / a.ny : 0;
-  // A wave whose points all lie outside the mask (most waves of a flow
-  // around a small body) has chi = 0 at every point, so that nl = u x w: it
-  // skips the FP64 penalisation term (which is 0 there for finite u; only
-  // the variant without statistics and sponge, whose other terms need every
-  // point).  The skipped code also frees the registers for a fourth wave
-  // per SIMD in the FP32 kernel.
-  bool masked = false;
+  if (stats && live) {
 #pragma unroll
-  for (int q = 0; q < 4; ++q) masked = masked || mk2[q].x != T(0) || mk2[q].y != T(0);
-  if (!SPONGE && !STATS && !__any(masked)) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const cplx<T> u0 = X[0][q], u1 = X[1][q], u2 = X[2][q], w0 = X[3][q], w1 = X[4][q], w2 = X[5][q];
-      O[0][q] = mk<T>(u1.x * w2.x - u2.x * w1.x, u1.y * w2.y - u2.y * w1.y);
-      O[1][q] = mk<T>(u2.x * w0.x - u0.x * w2.x, u2.y * w0.y - u0.y * w2.y);
-      O[2][q] = mk<T>(u0.x * w1.x - u1.x * w0.x, u0.y * w1.y - u1.y * w0.y);
+    for (int q = 0; q < E; ++q) {
+      const double ax = X[0][q].x, ay = X[1][q].x, az = X[2][q].x, bx = X[0][q].y, by = X[1][q].y, bz = X[2][q].y;
+      umax2 = nanmax(nanmax(umax2, ax * ax + ay * ay + az * az), bx * bx + by * by + bz * bz);
     }
-  } else
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    // one position at a time (FP64 temporaries of several would not fit)
-    __builtin_amdgcn_sched_barrier(0);
-    const int n = l + q * G;
-    const long pt0 = (long)(live ? gl : 0) * a.nx + 2 * n;
-    double nv[3][2], sv[3][2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      __builtin_amdgcn_sched_barrier(0);
-      const double ux = h ? X[0][q].y : X[0][q].x, uy = h ? X[1][q].y : X[1][q].x, uz = h ? X[2][q].y : X[2][q].x;
-      const double wx = h ? X[3][q].y : X[3][q].x, wy = h ? X[4][q].y : X[4][q].x, wz = h ? X[5][q].y : X[5][q].x;
-      const long pt = pt0 + h;
-      const double mkv = live ? (double)(h ? mk2[q].y : mk2[q].x) : 0.0;
-      double dux = ux, duy = uy, duz = uz;
-      if (mkv != 0.0) {
-        dux -= (double)us[pt];
-        duy -= (double)us[a.npts + pt];
-        duz -= (double)us[2 * a.npts + pt];
-      }
-      const double chi = mkv * a.eps_inv;
-      const double pv[3] = {chi * dux, chi * duy, chi * duz};
-      if (STATS && live) {
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-          const double t = fs[c] + pv[c];
-          fc[c] += (fabs(fs[c]) >= fabs(pv[c])) ? (fs[c] - t) + pv[c] : (pv[c] - t) + fs[c];
-          fs[c] = t;
-        }
-        umax2 = nanmax(umax2, ux * ux + uy * uy + uz * uz);
-      }
-      if constexpr (sizeof(T) == 4) {
-        // FP32-mixed: u x w in FP32, the precision of the transforms that
-        // produced u and w; the penalisation term stays FP64 (chi = mask/eta
-        // is large at small eta).  Keeps the kernel at 3 waves per SIMD
-        // without spilling.
-        const float fx = h ? X[0][q].y : X[0][q].x, fy = h ? X[1][q].y : X[1][q].x, fz = h ? X[2][q].y : X[2][q].x;
-        const float gx = h ? X[3][q].y : X[3][q].x, gy = h ? X[4][q].y : X[4][q].x, gz = h ? X[5][q].y : X[5][q].x;
-        nv[0][h] = (double)(fy * gz - fz * gy) - pv[0];
-        nv[1][h] = (double)(fz * gx - fx * gz) - pv[1];
-        nv[2][h] = (double)(fx * gy - fy * gx) - pv[2];
-      } else {
-        nv[0][h] = uy * wz - uz * wy - pv[0];
-        nv[1][h] = uz * wx - ux * wz - pv[1];
-        nv[2][h] = ux * wy - uy * wx - pv[2];
-      }
-      if constexpr (SPONGE) {
-        const int ix = 2 * n + h, th = a.sponge_thickness;
-        bool in_sp = false;
-        if (a.sponge == 1) {
-          if (a.nx > 4 && (ix <= th - 1 || ix >= a.nx - th)) in_sp = true;
-          if (iy <= th - 1 || iy >= a.ny - th) in_sp = true;
-          if (iz <= th - 1 || iz >= a.nz - th) in_sp = true;
-        } else if (a.sponge == 2) {
-          in_sp = ix >= a.nx - th;
-        }
-        in_sp = in_sp && (mkv < a.sponge_mask_thr);
-        sv[0][h] = in_sp ? -wx * a.sponge_eps_inv : 0.0;
-        sv[1][h] = in_sp ? -wy * a.sponge_eps_inv : 0.0;
-        sv[2][h] = in_sp ? -wz * a.sponge_eps_inv : 0.0;
-      }
-    }
+  }
+  // u x w in place of w (of u with the sponge, which needs w).  FP32-mixed:
+  // in FP32, the precision of the transforms that produced u and w.
+  constexpr int OF = SPONGE ? 0 : 3;  // the outputs' registers
+  // The penalisation term - chi (u - us), in FP64 (chi = mask/eta is large at
+  // small eta).  Most waves of a flow around a small body meet no mask.  A
+  // rolled loop rotates the positions through the first register: unrolled,
+  // the FP64 temporaries of several positions were live at once.
+  auto cross = [&](int q, cplx<T> (&nl)[3]) {
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-      O[c][q] = mk<T>((T)nv[c][0], (T)nv[c][1]);
-      if constexpr (SPONGE) O[3 + c][q] = mk<T>((T)sv[c][0], (T)sv[c][1]);
+      const int c1 = (c + 1) % 3, c2 = (c + 2) % 3;
+      const cplx<T> u1 = X[c1][q], u2 = X[c2][q], w1 = X[3 + c1][q], w2 = X[3 + c2][q];
+      nl[c] = mk<T>(u1.x * w2.x - u2.x * w1.x, u1.y * w2.y - u2.y * w1.y);
+    }
+  };
+  if (!SPONGE || !masked) {
+#pragma unroll
+    for (int q = 0; q < E; ++q) {
+      cplx<T> nl[3];
+      cross(q, nl);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) X[OF + c][q] = nl[c];
+    }
+  }
+  if (masked) {
+    brsrc ru[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) ru[c] = make_brsrc((const T*)a.us + c * a.npts, (unsigned)(a.npts * sizeof(T)));
+    cplx<T> mn = mk<T>(rld<T>(rm, ma ? pb : kOob), rld<T>(rm, mb ? pb + N * sizeof(T) : kOob));
+    // (keeps the block before the loop, where the loop's copies of X belong:
+    // merged with the branch's own block they were live on both paths)
+    asm volatile("" : "+v"(mn.x), "+v"(mn.y));
+#pragma unroll 1
+    for (int q = 0; q < E; ++q) {
+      const cplx<T> m = mn;
+      const unsigned pq = pb + (unsigned)(q * G) * sizeof(T), pn = pq + G * sizeof(T);
+      const bool more = q + 1 < E;
+      mn = mk<T>(rld<T>(rm, ma && more ? pn : kOob), rld<T>(rm, mb && more ? pn + N * sizeof(T) : kOob));
+      cplx<T> nl[3];
+      if constexpr (SPONGE) cross(0, nl);
+      else { nl[0] = X[3][0]; nl[1] = X[4][0]; nl[2] = X[5][0]; }
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const double usa = rld<T>(ru[c], m.x != T(0) ? pq : kOob), usb = rld<T>(ru[c], m.y != T(0) ? pq + N * sizeof(T) : kOob);
+        const double pa = (double)m.x * a.eps_inv * ((double)X[c][0].x - usa), pv = (double)m.y * a.eps_inv * ((double)X[c][0].y - usb);
+        nl[c] = mk<T>((T)((double)nl[c].x - pa), (T)((double)nl[c].y - pv));
+        if (stats) {
+          double t = fs[c] + pa;
+          fc[c] += (fabs(fs[c]) >= fabs(pa)) ? (fs[c] - t) + pa : (pa - t) + fs[c];
+          fs[c] = t;
+          t = fs[c] + pv;
+          fc[c] += (fabs(fs[c]) >= fabs(pv)) ? (fs[c] - t) + pv : (pv - t) + fs[c];
+          fs[c] = t;
+        }
+      }
+#pragma unroll
+      for (int f = 0; f < 6; ++f) {
+        const int c = f - OF;
+        const cplx<T> back = c >= 0 && c < 3 ? nl[c >= 0 && c < 3 ? c : 0] : X[f][0];
+#pragma unroll
+        for (int e = 0; e + 1 < E; ++e) X[f][e] = X[f][e + 1];
+        X[f][E - 1] = back;
+      }
+    }
+  }
+  if constexpr (SPONGE) {  // -w / eta_sponge at the sponge's points, in place of w
+    const int th = a.sponge_thickness;
+    bool yz[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int iy = (gl + h) % a.ny, iz = (gl + h) / a.ny;
+      yz[h] = a.sponge == 1 && (iy <= th - 1 || iy >= a.ny - th || iz <= th - 1 || iz >= a.nz - th);
+    }
+#pragma unroll
+    for (int q = 0; q < E; ++q) {
+      const int ix = l + q * G;
+      const bool x = a.sponge == 1 ? N > 4 && (ix <= th - 1 || ix >= N - th) : a.sponge == 2 && ix >= N - th;
+      const unsigned pq = pb + (unsigned)(q * G) * sizeof(T);
+      const T m0 = rld<T>(rm, ma && masked ? pq : kOob), m1 = rld<T>(rm, mb && masked ? pq + N * sizeof(T) : kOob);
+      const bool s0 = (x || yz[0]) && (double)m0 < a.sponge_mask_thr, s1 = (x || yz[1]) && (double)m1 < a.sponge_mask_thr;
+#pragma unroll
+      for (int c = 3; c < 6; ++c)
+        X[c][q] = mk<T>(s0 ? (T)(-(double)X[c][q].x * a.sponge_eps_inv) : T(0), s1 ? (T)(-(double)X[c][q].y * a.sponge_eps_inv) : T(0));
     }
   }
 
-  // ---- R2C of the outputs, split into the nx/2+1 entries
+  // ---- R2C of the outputs: A = (Z[k] + conj Z[N-k]) / 2, B = -i (Z[k] - conj Z[N-k]) / 2
   const T half = T(0.5);
 #pragma unroll
-  for (int c = 0; c < NFO; ++c) {
+  for (int c = 0; c < (SPONGE ? 6 : 3); ++c) {
     __builtin_amdgcn_sched_barrier(0);
-    wtransform<T, M, -1>(O[c], twl, ln, l);
-    cplx<T> zm[4];
-    if constexpr (split_ok<T, M>(true)) {
-      // mirrors M - n of n = l + qG, through (G - l) + (3 - q) G; n = 0 pairs with 0
-      int lo = l;
-      asm volatile("" : "+v"(lo));
-      cplx<T>* rw = ln + lp<T>(lo);
-      const cplx<T>* mr = ln + lp<T>(G - lo);
+    const int f = OF + c;
+    if constexpr (PP::ROW0) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q) rw[lp<T>(q * G)] = O[c][q];
-      wave_sync();
-      zm[0] = (lo == 0 ? ln : mr + lp<T>(3 * G))[0];
-#pragma unroll
-      for (int q = 1; q < 4; ++q) zm[q] = mr[lp<T>((3 - q) * G)];
-      wave_sync();
-    } else {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) ln[lp<T>(l + q * G)] = O[c][q];
-      wave_sync();
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int n = l + q * G;
-        zm[q] = ln[lp<T>(n == 0 ? 0 : M - n)];
-      }
+      for (int q = 0; q < E; ++q) ln[lp<T>(l + q * G)] = X[f][q];
       wave_sync();
     }
-    if (live) {
-      const gptr<cplx<T>> o = out + c * a.fstride_out + (long)gl * a.prow;
+    pfft<T, PP, -1>(X[f], twl, ln, l);
+    int lo = l;
+    asm volatile("" : "+v"(lo));
+    cplx<T>* rw = ln + lp<T>(lo);
+    const cplx<T>* mr = ln + lp<T>(G - lo);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const cplx<T> zk = O[c][q];
-        const cplx<T> s1 = add(zk, conj_w(zm[q])), d1 = sub(zk, conj_w(zm[q]));
-        if (l + q * G < a.kout) gst<T>(o + l + q * G, scl(sub(s1, ik_w<T>(T(1), cmul(twn[l + q * G], d1))), half));
-      }
-      if (l == 0 && M < a.kout) {
-        // k = M: partner of k = 0 is itself
-        const cplx<T> zk = O[c][0];
-        const cplx<T> s2 = add(zk, conj_w(zk)), d2 = sub(zk, conj_w(zk));
-        gst<T>(o + M, scl(sub(s2, ik_w<T>(T(1), cmul(twn[M], d2))), half));
-      }
+    for (int q = E - QO; q < E; ++q) {
+      if constexpr (split_rd<T, PP>()) rw[lp<T>(q * G)] = X[f][q];
+      else ln[lp<T>(lo + q * G)] = X[f][q];
     }
+    wave_sync();
+    const brsrc r = field(a.out, a.fstride_out, c);
+#pragma unroll
+    for (int q = 0; q < QO; ++q) {
+      const cplx<T> z = X[f][q];
+      cplx<T> zm = split_rd<T, PP>() ? mr[lp<T>((E - 1 - q) * G)] : ln[lp<T>(G - lo + (E - 1 - q) * G)];
+      if (q == 0 && l == 0) zm = z;
+      const unsigned off = live && l + q * G < a.kout ? lb + q * G * ES : kOob;
+      bst<T, 0>(r, off, mk<T>((z.x + zm.x) * half, (z.y - zm.y) * half));
+      bst<T, 0>(r, off + rowb, mk<T>((z.y + zm.y) * half, (zm.x - z.x) * half));
+    }
+    if constexpr (PR < 2) {  // k = N/2: its own partner
+      const cplx<T> z = X[f][H];
+      const unsigned off = live && l == 0 && N / 2 < a.kout ? lb + N / 2 * ES : kOob;
+      bst<T, 0>(r, off, mk<T>(z.x, T(0)));
+      bst<T, 0>(r, off + rowb, mk<T>(z.y, T(0)));
+    }
+    wave_sync();
   }
 
-  if (STATS) {
+  if (VAR > 0 && stats) {
     double v4[4] = {wmax(umax2), wsum(fs[0] + fc[0]), wsum(fs[1] + fc[1]), wsum(fs[2] + fc[2])};
     if (lane == 0) {
 #pragma unroll
@@ -479,7 +542,7 @@ __global__ __launch_bounds__(XW_NT) __attribute__((amdgpu_waves_per_eu(WPE > 0 ?
     __syncthreads();
     if (threadIdx.x == 0) {
       double r[4] = {red[0][0], red[0][1], red[0][2], red[0][3]};
-      for (int w = 1; w < WPB; ++w) {
+      for (int w = 1; w < wpb; ++w) {
         r[0] = nanmax(r[0], red[w][0]);
         for (int c = 1; c < 4; ++c) r[c] += red[w][c];
       }
@@ -488,21 +551,91 @@ __global__ __launch_bounds__(XW_NT) __attribute__((amdgpu_waves_per_eu(WPE > 0 ?
   }
 }
 
-template <typename T, int M>
-void run_wave(const XPassArgs& a, hipStream_t s) {
-  constexpr int LPB = (XW_NT / 64) * (256 / M);  // lines per block
-  const int blocks = (a.nlines + LPB - 1) / LPB;
-  if (a.sponge) {
-    if (a.want_stats) hipLaunchKernelGGL((x_rhs_wave_k<T, M, true, true, 0>), dim3(blocks, batch_n(a.bat)), dim3(XW_NT), 0, s, a);
-    else hipLaunchKernelGGL((x_rhs_wave_k<T, M, true, false, 0>), dim3(blocks, batch_n(a.bat)), dim3(XW_NT), 0, s, a);
-  } else if (a.want_stats) {
-    if (a.wpe == 3) hipLaunchKernelGGL((x_rhs_wave_k<T, M, false, true, 3>), dim3(blocks, batch_n(a.bat)), dim3(XW_NT), 0, s, a);
-    else hipLaunchKernelGGL((x_rhs_wave_k<T, M, false, true, 0>), dim3(blocks, batch_n(a.bat)), dim3(XW_NT), 0, s, a);
-  } else {
-    if (a.wpe == 3) hipLaunchKernelGGL((x_rhs_wave_k<T, M, false, false, 3>), dim3(blocks, batch_n(a.bat)), dim3(XW_NT), 0, s, a);
-    else hipLaunchKernelGGL((x_rhs_wave_k<T, M, false, false, 0>), dim3(blocks, batch_n(a.bat)), dim3(XW_NT), 0, s, a);
+// Positions a lane.  Four keep every wave's instruction stream short and
+// spread a small grid over more waves, eight exchange less through LDS (x
+// pass, four / eight a lane: FP32 64^3 11.4 / 12.8 us, 128^3 29.0 / 26.4 us;
+// FP32 96x64x64, four / twelve: 14.1 / 19.6 us).  FP64 keeps four up to nx = 256: eight
+// positions of six fields leave no room for a second wave per SIMD without
+// spills (64^3 13.2 / 13.9 us, 256x128x128 76 / 82 us).  The plan does not
+// depend on the batch: a member's results are those of its own run.
+int pair_e(int nx, long nlines, bool fp64) {
+  const bool small = nlines * nx < (1L << 20);
+  if (nx % 3 == 0) return nx == 96 && small ? 4 : 12;
+  return nx <= 256 && (fp64 || small) ? 4 : 8;
+}
+
+// Waves of a block: four share a twiddle table; a grid that leaves compute
+// units idle spreads its waves over more of them instead.
+int pair_waves(int nx, long nlines, int e) {
+  const long waves = (nlines / 2 * (nx / e) + 63) / 64;
+  return waves >= 1024 ? XW_NT / 64 : 1;
+}
+
+template <typename T, int N, int E, int VAR, int PR>
+void run_pair(const XPassArgs& a, hipStream_t s) {
+  using PP = PairPlan<N, E>;
+  const int w = pair_waves(N, (long)a.nlines * batch_n(a.bat), E), ppb = w * PP::PPW;
+  static_assert(pair_smem<T, PP>(XW_NT / 64) + sizeof(double) * XW_NT / 16 <= 65536, "LDS of a block");
+  const int blocks = (a.nlines / 2 + ppb - 1) / ppb;
+  const size_t smem = pair_smem<T, PP>(w);
+  hipLaunchKernelGGL((x_rhs_pair_k<T, N, E, VAR, PR>), dim3(blocks, batch_n(a.bat)), dim3(64 * w), smem, s, a);
+}
+template <typename T, int N, int E>
+void run_pair_e(const XPassArgs& a, hipStream_t s) {
+  constexpr int KQ = PairPlan<N, E>::QL * PairPlan<N, E>::G;
+  const int var = a.sponge ? 2 : (a.want_stats ? 1 : 0);
+  const int pr = a.kin > KQ ? 0 : (a.kout > KQ ? 1 : 2);
+  switch (3 * var + pr) {
+    case 0: run_pair<T, N, E, 0, 0>(a, s); break;
+    case 1: run_pair<T, N, E, 0, 1>(a, s); break;
+    case 2: run_pair<T, N, E, 0, 2>(a, s); break;
+    case 3: run_pair<T, N, E, 1, 0>(a, s); break;
+    case 4: run_pair<T, N, E, 1, 1>(a, s); break;
+    case 5: run_pair<T, N, E, 1, 2>(a, s); break;
+    case 6: run_pair<T, N, E, 2, 0>(a, s); break;
+    case 7: run_pair<T, N, E, 2, 1>(a, s); break;
+    default: run_pair<T, N, E, 2, 2>(a, s); break;
   }
 }
+template <typename T, int N>
+void run_pair_n(const XPassArgs& a, hipStream_t s) {
+  const int e = pair_e(N, a.nlines, sizeof(T) == 8);
+  if constexpr (N % 3 == 0) {
+    if constexpr (N == 96) { if (e == 4) { run_pair_e<T, N, 4>(a, s); return; } }
+    run_pair_e<T, N, 12>(a, s);
+  } else if constexpr (N <= 256) {
+    if constexpr (sizeof(T) == 4) { if (e == 8) { run_pair_e<T, N, 8>(a, s); return; } }
+    run_pair_e<T, N, 4>(a, s);
+  } else {
+    run_pair_e<T, N, 8>(a, s);
+  }
+}
+
+}  // namespace
+
+// Compiled in parts (per precision and family of lengths) for compile time.
+template <typename T, int N, int... M>
+static void pair_dispatch(const XPassArgs& a, hipStream_t s) {
+  if (a.nx == N) run_pair_n<T, N>(a, s);
+  else if constexpr (sizeof...(M) > 0) pair_dispatch<T, M...>(a, s);
+  else throw std::runtime_error("in-wave x pass: unsupported nx " + std::to_string(a.nx));
+}
+void launch_pair_f32_2(const XPassArgs& a, hipStream_t s);
+void launch_pair_f32_3(const XPassArgs& a, hipStream_t s);
+void launch_pair_f64_2(const XPassArgs& a, hipStream_t s);
+void launch_pair_f64_3(const XPassArgs& a, hipStream_t s);
+#if FLUSI_PART == 0
+void launch_pair_f32_2(const XPassArgs& a, hipStream_t s) { pair_dispatch<float, 32, 64, 128, 256, 512>(a, s); }
+#elif FLUSI_PART == 1
+void launch_pair_f32_3(const XPassArgs& a, hipStream_t s) { pair_dispatch<float, 48, 96, 192, 384>(a, s); }
+#elif FLUSI_PART == 2
+void launch_pair_f64_2(const XPassArgs& a, hipStream_t s) { pair_dispatch<double, 32, 64, 128, 256, 512>(a, s); }
+#elif FLUSI_PART == 3
+void launch_pair_f64_3(const XPassArgs& a, hipStream_t s) { pair_dispatch<double, 48, 96, 192, 384>(a, s); }
+#endif
+
+#if FLUSI_PART == 0
+namespace {
 
 // One wavefront per x line of the region: the line's flag is 1 where any of
 // its nx mask values is nonzero (NaN included).  The wavefront returns as a
@@ -534,25 +667,25 @@ void launch_mask_flags(const void* mask, uint8_t* flag, int nx, int ny, int y0, 
 template void launch_mask_flags<float>(const void*, uint8_t*, int, int, int, int, int, int, hipStream_t);
 template void launch_mask_flags<double>(const void*, uint8_t*, int, int, int, int, int, int, hipStream_t);
 
-bool x_rhs_wave_supported(int nx) { return nx == 64 || nx == 96 || nx == 128 || nx == 256 || nx == 512; }
+bool x_rhs_wave_supported(int nx) {
+  return nx == 32 || nx == 48 || nx == 64 || nx == 96 || nx == 128 || nx == 192 || nx == 256 || nx == 384 || nx == 512;
+}
 
-int x_rhs_wave_blocks(int nx, int nlines) {
-  const int lpb = (XW_NT / 64) * (256 / (nx / 2));
-  return (nlines + lpb - 1) / lpb;
+int x_rhs_wave_blocks(int nx, int nlines, bool fp64, int nmem) {
+  const int e = pair_e(nx, nlines, fp64);
+  const int ppb = pair_waves(nx, (long)nlines * nmem, e) * (64 / (nx / e));
+  return (nlines / 2 + ppb - 1) / ppb;
 }
 
 template <typename T>
 void launch_x_rhs_wave(const XPassArgs& a, hipStream_t s) {
-  switch (a.nx / 2) {
-    case 32: run_wave<T, 32>(a, s); break;
-    case 48: run_wave<T, 48>(a, s); break;
-    case 64: run_wave<T, 64>(a, s); break;
-    case 128: run_wave<T, 128>(a, s); break;
-    case 256: run_wave<T, 256>(a, s); break;
-    default: throw std::runtime_error("in-wave x pass: nx must be 64, 96, 128, 256 or 512");
-  }
+  if (a.nlines % 2) throw std::runtime_error("in-wave x pass: the lines come in pairs");
+  if (a.fbytes >= kOob) throw std::runtime_error("in-wave x pass: field too large for 32-bit offsets");
+  if (a.nx % 3 == 0) sizeof(T) == 4 ? launch_pair_f32_3(a, s) : launch_pair_f64_3(a, s);
+  else sizeof(T) == 4 ? launch_pair_f32_2(a, s) : launch_pair_f64_2(a, s);
 }
 template void launch_x_rhs_wave<float>(const XPassArgs&, hipStream_t);
 template void launch_x_rhs_wave<double>(const XPassArgs&, hipStream_t);
+#endif
 
 }  // namespace flusi
