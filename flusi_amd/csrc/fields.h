@@ -108,6 +108,8 @@ template <typename T> void launch_vortex_ring(const GridGeom& g, double x0, doub
 template <typename T> void launch_biot_savart(const GridGeom& g, const double* kx, const double* ky, const double* kz, const void* vk, void* uk, hipStream_t s);
 template <typename T> void launch_divergence(const GridGeom& g, const double* kx, const double* ky, const double* kz, const void* uk, void* dk, hipStream_t s);
 template <typename T> void launch_set_mode0(const GridGeom& g, void* uk, int comp, double re, double im, hipStream_t s);
+// the zero modes of the three components (re, im pairs) into mapped host memory
+template <typename T> void launch_mode0_out(const GridGeom& g, const void* uk, double* mirror, hipStream_t s);
 template <typename T> int diag_blocks(const GridGeom& g);
 template <typename T> void launch_diag(const GridGeom& g, const DiagArgs& a, hipStream_t s);
 // precision conversion host-layout <-> device arrays

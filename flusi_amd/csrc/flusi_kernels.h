@@ -194,6 +194,8 @@ template <typename T> void launch_zstep(const ZStepArgs& a, hipStream_t s);
 int x_pass_blocks(int nx, int nlines, bool fp64);
 // the right-hand-side x pass with pairs of lines inside one wavefront (xrhs_wave.hip)
 template <typename T> void launch_x_rhs_wave(const XPassArgs& a, hipStream_t s);
+// its inverse transforms alone: XM_INV (1 or 3 fields) and XM_INV_UW
+template <typename T> void launch_x_inv_wave(const XPassArgs& a, int mode, hipStream_t s);
 bool x_rhs_wave_supported(int nx);
 int x_rhs_wave_blocks(int nx, int nlines, bool fp64, int nmem);  // per member of a batch of nmem
 // per x line (iy, iz) of [y0, y1] x [z0, z1]: flag[iz ny + iy] = 1 where any
@@ -211,7 +213,9 @@ bool x_length_supported(int m);     // nx/2 of the real x axis
 
 // reductions (fields.hip)
 // out[v] = combine over rows of partial[row*nv + v]; kind[v]: 0 = Neumaier sum, 1 = max, 2 = min
-void launch_reduce_rows(const double* partial, int nrows, int nv, const int* kinds_dev, double* mid, double* out, hipStream_t s);
+// mirror (mapped host memory, may be null) receives the results, too
+void launch_reduce_rows(const double* partial, int nrows, int nv, const int* kinds_dev, double* mid, double* out, hipStream_t s,
+                        double* mirror = nullptr);
 size_t reduce_rows_scratch(int nv);  // doubles of `mid` needed for nv values
 
 }  // namespace flusi

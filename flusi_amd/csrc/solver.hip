@@ -310,6 +310,7 @@ class Solver : public SolverBase {
   double* dpart = nullptr; int ndblocks = 0;
   double* noalloc_scratch = nullptr;  // device address of `scratch` on this context's GPU
   double* red = nullptr;    // small results
+  double* red_h = nullptr;  // the same in mapped host memory: read after a synchronisation, without a copy
   double* rmid = nullptr;   // reduction scratch
   int* kinds = nullptr;     // reduction kinds: [0..3] x pass, [4] energy, [8..8+DIAG_NV) diag
   double* stage = nullptr; size_t stage_n = 0;
@@ -325,6 +326,7 @@ class Solver : public SolverBase {
     for (auto& e : ev) { (void)hipEventDestroy(e.second.first); (void)hipEventDestroy(e.second.second); }
     for (void* q : owned) (void)hipFree(q);
     for (hipEvent_t e : ins_ev) if (e) (void)hipEventDestroy(e);
+    if (red_h) (void)hipHostFree(red_h);
     if (ins_h) (void)hipHostFree(ins_h);
     if (stream) (void)hipStreamDestroy(stream);
   }
@@ -444,6 +446,7 @@ class Solver : public SolverBase {
       dpart = (double*)dalloc(sizeof(double) * DIAG_NV * ndblocks);
     }
     red = (double*)dalloc(sizeof(double) * 128);
+    HIPCHECK(hipHostMalloc((void**)&red_h, sizeof(double) * 128, hipHostMallocDefault));
     rmid = (double*)dalloc(sizeof(double) * reduce_rows_scratch(DIAG_NV));
     std::vector<int> k(8 + DIAG_NV, 0);
     k[0] = 1;  // umax^2: max
@@ -663,7 +666,9 @@ class Solver : public SolverBase {
   // and the reduction of max|u|^2 and sum chi (u - us) into red[0..3].  in:
   // u_in is zero outside the dealiased region; out: only the result's modes
   // inside it are used (post_rhs with prune & 2).
-  void pre_rhs(const void* u_in, double t, bool with_mask = true, bool in = false, bool out = false) {
+  // umax: whether the step size is derived from this right-hand side's
+  // max|u|^2 (a step's first stage).
+  void pre_rhs(const void* u_in, double t, bool with_mask = true, bool in = false, bool out = false, bool umax = true) {
     if (with_mask && p.iMoving == 1 && p.iPenalization == 1) create_mask(t);
     if (p.eps < 1.0e-11) throw FlusiError(77363800, "Value of eps is very small, maybe even zero.");
     p_row = in && out ? prowc : prow;
@@ -679,7 +684,7 @@ class Solver : public SolverBase {
     a.sponge_eps_inv = a.sponge ? 1.0 / p.eps_sponge : 0.0;
     a.sponge_mask_thr = (a.sponge == 2) ? (double)1.0e-12f : 1.0e-12;
     a.partial = xpart;
-    a.want_stats = (p.dt_fixed <= 0.0 || p.iMeanFlow[0] == "dynamic" || p.iMeanFlow[1] == "dynamic" ||
+    a.want_stats = ((umax && p.dt_fixed <= 0.0) || p.iMeanFlow[0] == "dynamic" || p.iMeanFlow[1] == "dynamic" ||
                     p.iMeanFlow[2] == "dynamic") ? 1 : 0;
     timed(TM_X, [&] {
       if (xwave) launch_x_rhs_wave<T>(a, stream);
@@ -690,7 +695,8 @@ class Solver : public SolverBase {
       const int nxblocks = xwave ? x_rhs_wave_blocks(nx, ny * nz, FP64, batch_n(bat)) : x_pass_blocks(nx, ny * nz, FP64);
       for (int m = 0; m < batch_n(bat); ++m) {
         const long o = m * bat.mstride;
-        launch_reduce_rows(mshift(xpart, o), nxblocks, 4, mshift(kinds, o), mshift(rmid, o), mshift(red, o), stream);
+        launch_reduce_rows(mshift(xpart, o), nxblocks, 4, mshift(kinds, o), mshift(rmid, o), mshift(red, o), stream,
+                           m == 0 ? red_h : nullptr);
       }
     }
     kcheck("reduce x");
@@ -739,10 +745,8 @@ class Solver : public SolverBase {
   }
 
   double host_umax() {
-    double v = 0.0;
-    HIPCHECK(hipMemcpyAsync(&v, red, sizeof(double), hipMemcpyDeviceToHost, stream));
     HIPCHECK(hipStreamSynchronize(stream));
-    return std::sqrt(v);
+    return std::sqrt(red_h[0]);
   }
 
   // fluid_time_step.f90:917-1042 adjust_dt
@@ -778,10 +782,9 @@ class Solver : public SolverBase {
   // for every member after the step)
   void record_ekin(bool force = false) {
     if (out_dir.empty() || (ens_step && !force)) return;
-    launch_reduce_rows(zpart, nzpart, 1, kinds + 4, rmid, red + 8, stream);
-    double e = 0.0;
-    HIPCHECK(hipMemcpyAsync(&e, red + 8, sizeof(double), hipMemcpyDeviceToHost, stream));
+    launch_reduce_rows(zpart, nzpart, 1, kinds + 4, rmid, red + 8, stream, red_h + 8);
     HIPCHECK(hipStreamSynchronize(stream));
+    const double e = red_h[8];
     append("ekin.t", {time + dt1, e * p.xl * p.yl * p.zl}, "%          time            ekin");
   }
 
@@ -790,11 +793,10 @@ class Solver : public SolverBase {
   // NaN or Inf anywhere makes it non-finite)
   void check_nan() override {
     need_fft();
-    launch_reduce_rows(zpart, nzpart, 1, kinds + 4, rmid, red + 10, stream);
+    launch_reduce_rows(zpart, nzpart, 1, kinds + 4, rmid, red + 10, stream, red_h + 10);
     kcheck("checknan");
-    double e = 0.0;
-    HIPCHECK(hipMemcpyAsync(&e, red + 10, sizeof(double), hipMemcpyDeviceToHost, stream));
     HIPCHECK(hipStreamSynchronize(stream));
+    const double e = red_h[10];
     if (!std::isfinite(e)) throw FlusiError(202, "NaN in uk after time step " + std::to_string(it));
   }
 
@@ -944,7 +946,7 @@ class Solver : public SolverBase {
       ZStepArgs z = zargs(SM_RK2_1);
       z.u = uk; z.r0 = reg[0]; z.dt = dt1; z.vis_dt_old = old; z.vis_dt_new = vis_dt; z.prune = dea ? 2 : 0;
       post_rhs(z);
-      pre_rhs(uk, time, true, dea);
+      pre_rhs(uk, time, true, dea, false, false);
       ZStepArgs z2 = zargs(SM_RK2_2);
       z2.u = uk; z2.r0 = reg[0]; z2.dt = dt1; z2.prune = dea ? 1 : 0;
       post_rhs(z2);
@@ -956,7 +958,7 @@ class Solver : public SolverBase {
       const double ts[4] = {time, time + 0.5 * dt1, time + 0.5 * dt1, time + dt1};
       if (!in) { set_reg_pruned(0, false); set_reg_pruned(1, false); }
       for (int s = 0; s < 4; ++s) {
-        if (s > 0) pre_rhs(reg[0], ts[s], true, in, in);
+        if (s > 0) pre_rhs(reg[0], ts[s], true, in, in, false);
         ZStepArgs z = zargs(modes[s]);
         z.u = uk; z.udiff = (s == 0) ? uk : reg[0]; z.ustage = reg[0]; z.acc = reg[1]; z.dt = dt1;
         z.prune = in ? 3 : 0;
@@ -1066,11 +1068,9 @@ class Solver : public SolverBase {
     HIPCHECK(hipMemcpyAsync(dst, src, state_bytes(), hipMemcpyDeviceToDevice, stream));
   }
   double reduce_partials(double* part, int nb) {
-    launch_reduce_rows(part, nb, 1, kinds + 4, rmid, red + 100, stream);  // red[16..77]: diagnostics
-    double v = 0.0;
-    HIPCHECK(hipMemcpyAsync(&v, red + 100, sizeof(double), hipMemcpyDeviceToHost, stream));
+    launch_reduce_rows(part, nb, 1, kinds + 4, rmid, red + 100, stream, red_h + 100);  // red[16..77]: diagnostics
     HIPCHECK(hipStreamSynchronize(stream));
-    return v;
+    return red_h[100];
   }
   void adjoint_check() {
     need_fft();
@@ -1775,6 +1775,10 @@ class Solver : public SolverBase {
   void ensure_phys() { if (!phys) phys = dalloc(7 * sizeof(T) * npts); }
   T* pf(int f) { return reinterpret_cast<T*>(phys) + (long)f * npts; }
 
+  void x_inverse(const XPassArgs& a, int mode) {
+    if (xwave) launch_x_inv_wave<T>(a, mode, stream);
+    else launch_x_pass<T>(a, mode, stream);
+  }
   // in: u_in is zero outside the dealiased region
   void inv_uw_phys(const void* u_in, bool in) {
     p_row = prow;
@@ -1783,7 +1787,7 @@ class Solver : public SolverBase {
     XPassArgs a = xargs();
     if (in) a.kin = pr.nkx;
     a.in = P; a.out = phys; a.fstride_in = pc; a.fstride_out = npts; a.nf = 6;
-    timed(TM_X, [&] { launch_x_pass<T>(a, XM_INV_UW, stream); });
+    timed(TM_X, [&] { x_inverse(a, XM_INV_UW); });
     kcheck("x inverse uw");
   }
   // 1 or 3 spectral S-layout fields -> physical
@@ -1800,7 +1804,7 @@ class Solver : public SolverBase {
     XPassArgs a = xargs();
     if (in) a.kin = pr.nkx;
     a.in = P; a.out = dst; a.fstride_in = pc; a.fstride_out = npts; a.nf = nf;
-    timed(TM_X, [&] { launch_x_pass<T>(a, XM_INV, stream); });
+    timed(TM_X, [&] { x_inverse(a, XM_INV); });
     kcheck("x inverse");
   }
   // 1 or 3 physical fields -> S-layout spectral (times 1/N)
@@ -1993,7 +1997,8 @@ class Solver : public SolverBase {
 
   void get_u(double* u, bool vort) override {
     need_fft();
-    inv_uw_phys(uk, uk_pruned);
+    if (vort) inv_uw_phys(uk, uk_pruned);
+    else { ensure_phys(); ifft_fields(uk, 3, pf(0), uk_pruned); }
     copy_real_out(vort ? (void*)pf(3) : (void*)pf(0), u, 3 * npts);
   }
 
@@ -2077,11 +2082,10 @@ class Solver : public SolverBase {
     need_fft();
     if (!epart) epart = (double*)dalloc(sizeof(double) * energy_k_blocks());
     launch_energy_k<T>(geom, uk, epart, stream);
-    launch_reduce_rows(epart, energy_k_blocks(), 1, kinds + 4, rmid, red + 9, stream);
+    launch_reduce_rows(epart, energy_k_blocks(), 1, kinds + 4, rmid, red + 9, stream, red_h + 9);
     kcheck("energy_k");
-    double e = 0.0;
-    HIPCHECK(hipMemcpyAsync(&e, red + 9, sizeof(double), hipMemcpyDeviceToHost, stream));
     HIPCHECK(hipStreamSynchronize(stream));
+    const double e = red_h[9];
     return e * p.xl * p.yl * p.zl;
   }
 
@@ -2140,12 +2144,10 @@ class Solver : public SolverBase {
     d.partial = dpart;
     timed(TM_DIAG, [&] { launch_diag<T>(geom, d, stream); });
     kcheck("diag");
-    launch_reduce_rows(dpart, ndblocks, DIAG_NV, kinds + 8, rmid, red + 16, stream);
+    launch_reduce_rows(dpart, ndblocks, DIAG_NV, kinds + 8, rmid, red + 16, stream, red_h + 16);
     kcheck("reduce diag");
-    std::vector<double> r(DIAG_NV);
-    HIPCHECK(hipMemcpyAsync(r.data(), red + 16, sizeof(double) * DIAG_NV, hipMemcpyDeviceToHost, stream));
     HIPCHECK(hipStreamSynchronize(stream));
-    return r;
+    return std::vector<double>(red_h + 16, red_h + 16 + DIAG_NV);
   }
 
   // drag.f90:336-453: forces, moments, penalisation power, residual velocity
@@ -2232,11 +2234,9 @@ class Solver : public SolverBase {
     launch_divergence<T>(geom, kx_d, ky_d, kz_d, uk, dk, stream);
     kcheck("divergence");
     ifft_fields(dk, 1, pf(6), uk_pruned);
+    launch_mode0_out<T>(geom, uk, red_h + 104, stream);  // (red[16..77]: diagnostics)
     const std::vector<double> r = diag_sums(pf(0), pf(3), pf(6));
-    std::vector<C> m0(3);
-    for (int c = 0; c < 3; ++c)
-      HIPCHECK(hipMemcpyAsync(&m0[c], cf(uk, c), sizeof(C), hipMemcpyDeviceToHost, stream));
-    HIPCHECK(hipStreamSynchronize(stream));
+    const double* m0 = red_h + 104;
     const double dv = p.dx() * p.dy() * p.dz();
     double o[FLUSI_INTEGRALS_NV] = {0};
     drag_assemble(t, r, o, forces);
@@ -2257,7 +2257,7 @@ class Solver : public SolverBase {
     for (int i = 10; i < 26; ++i) erow.push_back(o[i]);
     for (int i = 6; i < 10; ++i) erow.push_back(o[i]);
     append("energy.t", erow, "%          time         E_kin_f       E_kin_x_f       E_kin_y_f       E_kin_z_f          diss_f        diss_x_f        diss_y_f        diss_z_f       E_kin_tot     E_kin_tot_x     E_kin_tot_y     E_kin_tot_z        diss_tot      diss_tot_x      diss_tot_y      diss_tot_z      flux_penal");
-    append("meanflow.t", {t, (double)m0[0].x, (double)m0[1].x, (double)m0[2].x}, "%          time          uxmean          uymean          uzmean");
+    append("meanflow.t", {t, m0[0], m0[2], m0[4]}, "%          time          uxmean          uymean          uzmean");
     append("mask_volume.t", {t, o[28], o[29], o[30], o[31]}, "%          time     mask_volume      usx_integral    usy_integral    usz_integral");
     if (out) std::memcpy(out, o, sizeof(o));
   }

@@ -246,7 +246,8 @@ template <typename T, typename PP> constexpr size_t pair_smem(int waves) {
 }
 
 // waves per SIMD the register allocation must allow
-template <typename T, int N, int E, int VAR, int PR> constexpr int pair_wpe() {
+template <typename T, int N, int E, int VAR, int PR, int NF> constexpr int pair_wpe() {
+  if (NF < 6) return sizeof(T) == 4 ? 4 : 3;
   if (E == 12) return sizeof(T) == 4 ? 2 : 1;
   if (E == 4) return sizeof(T) == 4 ? 4 : (N % 3 == 0 ? 2 : 3);
   return sizeof(T) == 4 ? (VAR == 0 && PR > 0 ? 4 : 3) : 2;
@@ -254,9 +255,11 @@ template <typename T, int N, int E, int VAR, int PR> constexpr int pair_wpe() {
 
 // PR 1: the spectra are zero at k >= QL G (a dealiased state), so that only QL
 // groups a line are loaded and mirrored; PR 2: no more are stored, either.
-// VAR: 0 plain, 1 with the statistics, 2 sponge (and the statistics if asked)
-template <typename T, int N, int E, int VAR, int PR>
-__global__ __launch_bounds__(XW_NT) __attribute__((amdgpu_waves_per_eu(pair_wpe<T, N, E, VAR, PR>()))) void x_rhs_pair_k(XPassArgs a) {
+// VAR: 0 plain, 1 with the statistics, 2 sponge (and the statistics if asked),
+// 3 the inverse transforms alone, to physical fields: NF = 6 (u and w), 3 or 1
+// fields as they come
+template <typename T, int N, int E, int VAR, int PR, int NF>
+__global__ __launch_bounds__(XW_NT) __attribute__((amdgpu_waves_per_eu(pair_wpe<T, N, E, VAR, PR, NF>()))) void x_rhs_pair_k(XPassArgs a) {
   to_member(a, blockIdx.y);
   using PP = PairPlan<N, E>;
   constexpr int G = PP::G, PPW = PP::PPW, H = E / 2;
@@ -288,9 +291,9 @@ __global__ __launch_bounds__(XW_NT) __attribute__((amdgpu_waves_per_eu(pair_wpe<
   auto field = [&](const void* base, long stride, int f) {
     return make_brsrc(reinterpret_cast<const cplx<T>*>(base) + f * stride, a.fbytes);
   };
-  cplx<T> X[6][E], nyq[6];
+  cplx<T> X[NF][E], nyq[NF];
 #pragma unroll
-  for (int f = 0; f < 6; ++f) {
+  for (int f = 0; f < NF; ++f) {
     const brsrc r = field(a.in, a.fstride_in, f);
 #pragma unroll
     for (int q = 0; q < QL; ++q) {
@@ -303,6 +306,7 @@ __global__ __launch_bounds__(XW_NT) __attribute__((amdgpu_waves_per_eu(pair_wpe<
       const cplx<T> xa = bld_s<T>(r, off, 0), xb = bld_s<T>(r, off, rowb);
       nyq[f] = xa;  // (real part of line a, of line b); w below
       nyq[f].y = xb.x;
+      if constexpr (NF == 6)
       if (f == 4 || f == 5) {  // w_y = A - i kx V_z, w_z = i kx V_y - B: real parts at k = N/2
         const T kx = (T)(a.kx_scale * double(N / 2));
         const brsrc rv = field(a.in, a.fstride_in, f == 4 ? 2 : 1);
@@ -317,12 +321,12 @@ __global__ __launch_bounds__(XW_NT) __attribute__((amdgpu_waves_per_eu(pair_wpe<
   const brsrc rm = make_brsrc(a.mask, (unsigned)(a.npts * sizeof(T)));
   const unsigned pb = (unsigned)(gl * N + l) * (unsigned)sizeof(T);
   bool ma = live, mb = live;
-  if (a.mflag) {
+  if (VAR < 3 && a.mflag) {
     ma = live && ((gptr<const uint8_t>)a.mflag)[gl] != 0;
     mb = live && ((gptr<const uint8_t>)a.mflag)[gl + 1] != 0;
   }
   bool masked = ma || mb;
-  if (!a.mflag) {  // no flags (members of a batch): the wave looks at its own points
+  if (VAR < 3 && !a.mflag) {  // no flags (members of a batch): the wave looks at its own points
     bool any = false;
 #pragma unroll
     for (int q = 0; q < E; ++q) {
@@ -337,7 +341,7 @@ __global__ __launch_bounds__(XW_NT) __attribute__((amdgpu_waves_per_eu(pair_wpe<
 
   // ---- Z = A + i B and its mirrored modes M = conj A + i conj B, then w_y, w_z
 #pragma unroll
-  for (int f = 0; f < 6; ++f)
+  for (int f = 0; f < NF; ++f)
 #pragma unroll
     for (int q = 0; q < QL; ++q) {
       cplx<T> xa = X[f][q], xb = X[f][E - QL + q];
@@ -345,6 +349,7 @@ __global__ __launch_bounds__(XW_NT) __attribute__((amdgpu_waves_per_eu(pair_wpe<
       X[f][q] = mk<T>(xa.x - xb.y, xa.y + xb.x);
       X[f][E - QL + q] = mk<T>(xa.x + xb.y, xb.x - xa.y);
     }
+  if constexpr (NF == 6)
 #pragma unroll
   for (int q = 0; q < QL; ++q) {
     const T kx = (T)(a.kx_scale * double(l + q * G));
@@ -355,9 +360,9 @@ __global__ __launch_bounds__(XW_NT) __attribute__((amdgpu_waves_per_eu(pair_wpe<
     X[5][m] = sub(ik_p<T>(-kx, X[1][m]), X[5][m]);
   }
 
-  // ---- C2R of the six fields
+  // ---- C2R of the fields
 #pragma unroll
-  for (int f = 0; f < 6; ++f) {
+  for (int f = 0; f < NF; ++f) {
     // one field at a time: keeps the scheduler from interleaving the
     // independent transforms (their temporaries would exhaust the registers)
     __builtin_amdgcn_sched_barrier(0);
@@ -395,7 +400,15 @@ __global__ __launch_bounds__(XW_NT) __attribute__((amdgpu_waves_per_eu(pair_wpe<
       for (int q = QL; q < E - QL; ++q) X[f][q] = mk<T>(T(0), T(0));
     }
     pfft<T, PP, +1>(X[f], twl, ln, l);
+    if constexpr (VAR == 3) {
+      const gptr<T> o = (gptr<T>)a.out + f * a.fstride_out + (long)gl * N + l;
+      if (live) {
+#pragma unroll
+        for (int q = 0; q < E; ++q) { o[q * G] = X[f][q].x; o[N + q * G] = X[f][q].y; }
+      }
+    }
   }
+  if constexpr (VAR < 3) {
 
   // ---- u x w - chi (u - us) [+ sponge], in place: X[0..2] (and X[3..5])
   double umax2 = 0.0, fs[3] = {0.0, 0.0, 0.0}, fc[3] = {0.0, 0.0, 0.0};
@@ -549,6 +562,7 @@ __global__ __launch_bounds__(XW_NT) __attribute__((amdgpu_waves_per_eu(pair_wpe<
       for (int c = 0; c < 4; ++c) ((gptr<double>)a.partial)[(long)blockIdx.x * 4 + c] = r[c];
     }
   }
+  }  // VAR < 3
 }
 
 // Positions a lane.  Four keep every wave's instruction stream short and
@@ -571,18 +585,26 @@ int pair_waves(int nx, long nlines, int e) {
   return waves >= 1024 ? XW_NT / 64 : 1;
 }
 
-template <typename T, int N, int E, int VAR, int PR>
+template <typename T, int N, int E, int VAR, int PR, int NF = 6>
 void run_pair(const XPassArgs& a, hipStream_t s) {
   using PP = PairPlan<N, E>;
   const int w = pair_waves(N, (long)a.nlines * batch_n(a.bat), E), ppb = w * PP::PPW;
   static_assert(pair_smem<T, PP>(XW_NT / 64) + sizeof(double) * XW_NT / 16 <= 65536, "LDS of a block");
   const int blocks = (a.nlines / 2 + ppb - 1) / ppb;
   const size_t smem = pair_smem<T, PP>(w);
-  hipLaunchKernelGGL((x_rhs_pair_k<T, N, E, VAR, PR>), dim3(blocks, batch_n(a.bat)), dim3(64 * w), smem, s, a);
+  hipLaunchKernelGGL((x_rhs_pair_k<T, N, E, VAR, PR, NF>), dim3(blocks, batch_n(a.bat)), dim3(64 * w), smem, s, a);
 }
+// inv: the inverse transforms of that many fields alone (0: the right-hand side)
 template <typename T, int N, int E>
-void run_pair_e(const XPassArgs& a, hipStream_t s) {
+void run_pair_e(const XPassArgs& a, int inv, hipStream_t s) {
   constexpr int KQ = PairPlan<N, E>::QL * PairPlan<N, E>::G;
+  if (inv) {
+    const bool pin = a.kin <= KQ;
+    if (inv == 6) pin ? run_pair<T, N, E, 3, 1, 6>(a, s) : run_pair<T, N, E, 3, 0, 6>(a, s);
+    else if (inv == 3) pin ? run_pair<T, N, E, 3, 1, 3>(a, s) : run_pair<T, N, E, 3, 0, 3>(a, s);
+    else pin ? run_pair<T, N, E, 3, 1, 1>(a, s) : run_pair<T, N, E, 3, 0, 1>(a, s);
+    return;
+  }
   const int var = a.sponge ? 2 : (a.want_stats ? 1 : 0);
   const int pr = a.kin > KQ ? 0 : (a.kout > KQ ? 1 : 2);
   switch (3 * var + pr) {
@@ -598,16 +620,16 @@ void run_pair_e(const XPassArgs& a, hipStream_t s) {
   }
 }
 template <typename T, int N>
-void run_pair_n(const XPassArgs& a, hipStream_t s) {
+void run_pair_n(const XPassArgs& a, int inv, hipStream_t s) {
   const int e = pair_e(N, a.nlines, sizeof(T) == 8);
   if constexpr (N % 3 == 0) {
-    if constexpr (N == 96) { if (e == 4) { run_pair_e<T, N, 4>(a, s); return; } }
-    run_pair_e<T, N, 12>(a, s);
+    if constexpr (N == 96) { if (e == 4) { run_pair_e<T, N, 4>(a, inv, s); return; } }
+    run_pair_e<T, N, 12>(a, inv, s);
   } else if constexpr (N <= 256) {
-    if constexpr (sizeof(T) == 4) { if (e == 8) { run_pair_e<T, N, 8>(a, s); return; } }
-    run_pair_e<T, N, 4>(a, s);
+    if constexpr (sizeof(T) == 4) { if (e == 8) { run_pair_e<T, N, 8>(a, inv, s); return; } }
+    run_pair_e<T, N, 4>(a, inv, s);
   } else {
-    run_pair_e<T, N, 8>(a, s);
+    run_pair_e<T, N, 8>(a, inv, s);
   }
 }
 
@@ -615,23 +637,23 @@ void run_pair_n(const XPassArgs& a, hipStream_t s) {
 
 // Compiled in parts (per precision and family of lengths) for compile time.
 template <typename T, int N, int... M>
-static void pair_dispatch(const XPassArgs& a, hipStream_t s) {
-  if (a.nx == N) run_pair_n<T, N>(a, s);
-  else if constexpr (sizeof...(M) > 0) pair_dispatch<T, M...>(a, s);
+static void pair_dispatch(const XPassArgs& a, int inv, hipStream_t s) {
+  if (a.nx == N) run_pair_n<T, N>(a, inv, s);
+  else if constexpr (sizeof...(M) > 0) pair_dispatch<T, M...>(a, inv, s);
   else throw std::runtime_error("in-wave x pass: unsupported nx " + std::to_string(a.nx));
 }
-void launch_pair_f32_2(const XPassArgs& a, hipStream_t s);
-void launch_pair_f32_3(const XPassArgs& a, hipStream_t s);
-void launch_pair_f64_2(const XPassArgs& a, hipStream_t s);
-void launch_pair_f64_3(const XPassArgs& a, hipStream_t s);
+void launch_pair_f32_2(const XPassArgs& a, int inv, hipStream_t s);
+void launch_pair_f32_3(const XPassArgs& a, int inv, hipStream_t s);
+void launch_pair_f64_2(const XPassArgs& a, int inv, hipStream_t s);
+void launch_pair_f64_3(const XPassArgs& a, int inv, hipStream_t s);
 #if FLUSI_PART == 0
-void launch_pair_f32_2(const XPassArgs& a, hipStream_t s) { pair_dispatch<float, 32, 64, 128, 256, 512>(a, s); }
+void launch_pair_f32_2(const XPassArgs& a, int inv, hipStream_t s) { pair_dispatch<float, 32, 64, 128, 256, 512>(a, inv, s); }
 #elif FLUSI_PART == 1
-void launch_pair_f32_3(const XPassArgs& a, hipStream_t s) { pair_dispatch<float, 48, 96, 192, 384>(a, s); }
+void launch_pair_f32_3(const XPassArgs& a, int inv, hipStream_t s) { pair_dispatch<float, 48, 96, 192, 384>(a, inv, s); }
 #elif FLUSI_PART == 2
-void launch_pair_f64_2(const XPassArgs& a, hipStream_t s) { pair_dispatch<double, 32, 64, 128, 256, 512>(a, s); }
+void launch_pair_f64_2(const XPassArgs& a, int inv, hipStream_t s) { pair_dispatch<double, 32, 64, 128, 256, 512>(a, inv, s); }
 #elif FLUSI_PART == 3
-void launch_pair_f64_3(const XPassArgs& a, hipStream_t s) { pair_dispatch<double, 48, 96, 192, 384>(a, s); }
+void launch_pair_f64_3(const XPassArgs& a, int inv, hipStream_t s) { pair_dispatch<double, 48, 96, 192, 384>(a, inv, s); }
 #endif
 
 #if FLUSI_PART == 0
@@ -678,14 +700,26 @@ int x_rhs_wave_blocks(int nx, int nlines, bool fp64, int nmem) {
 }
 
 template <typename T>
-void launch_x_rhs_wave(const XPassArgs& a, hipStream_t s) {
+static void launch_pair(const XPassArgs& a, int inv, hipStream_t s) {
   if (a.nlines % 2) throw std::runtime_error("in-wave x pass: the lines come in pairs");
-  if (a.fbytes >= kOob) throw std::runtime_error("in-wave x pass: field too large for 32-bit offsets");
-  if (a.nx % 3 == 0) sizeof(T) == 4 ? launch_pair_f32_3(a, s) : launch_pair_f64_3(a, s);
-  else sizeof(T) == 4 ? launch_pair_f32_2(a, s) : launch_pair_f64_2(a, s);
+  if (a.fbytes >= kOob || a.npts * (long)sizeof(T) >= (long)kOob)
+    throw std::runtime_error("in-wave x pass: field too large for 32-bit offsets");
+  if (a.nx % 3 == 0) sizeof(T) == 4 ? launch_pair_f32_3(a, inv, s) : launch_pair_f64_3(a, inv, s);
+  else sizeof(T) == 4 ? launch_pair_f32_2(a, inv, s) : launch_pair_f64_2(a, inv, s);
+}
+template <typename T>
+void launch_x_rhs_wave(const XPassArgs& a, hipStream_t s) {
+  launch_pair<T>(a, 0, s);
+}
+template <typename T>
+void launch_x_inv_wave(const XPassArgs& a, int mode, hipStream_t s) {
+  if (mode == XM_INV ? (a.nf != 1 && a.nf != 3) : mode != XM_INV_UW) throw std::runtime_error("x inverse pass: nf must be 1 or 3");
+  launch_pair<T>(a, mode == XM_INV ? a.nf : 6, s);
 }
 template void launch_x_rhs_wave<float>(const XPassArgs&, hipStream_t);
 template void launch_x_rhs_wave<double>(const XPassArgs&, hipStream_t);
+template void launch_x_inv_wave<float>(const XPassArgs&, int, hipStream_t);
+template void launch_x_inv_wave<double>(const XPassArgs&, int, hipStream_t);
 #endif
 
 }  // namespace flusi
