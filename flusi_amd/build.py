@@ -19,7 +19,8 @@ CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(ROOT, "_build")
 LIB = os.path.join(HERE, "libflusi_hip.so")
 SOURCES = ["zstep.hip:0", "zstep.hip:1", "zstep.hip:2", "zstep.hip:3", "passes.hip", "tiles_wave.hip",
-           "xrhs_wave.hip:0", "xrhs_wave.hip:1", "xrhs_wave.hip:2", "xrhs_wave.hip:3", "fields.hip", "adjoint.hip", "solver.hip", "host_params.cpp", "h5bind.cc"]
+           "xrhs_wave.hip:0", "xrhs_wave.hip:1", "xrhs_wave.hip:2", "xrhs_wave.hip:3", "fields.hip", "adjoint.hip", "solver.hip", "host_params.cpp",
+           "hostcopy.cpp", "h5bind.cc"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("FLUSI_OFFLOAD_ARCH", "gfx950")
 FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",

@@ -1,0 +1,21 @@
+// Copies of large fields between the device and the caller's (pageable) FP64 host arrays.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <memory>
+
+namespace flusi {
+
+// One pool of pinned staging memory per device, shared by the contexts on it;
+// it is freed with the last of them.
+class HostCopyPool;
+std::shared_ptr<HostCopyPool> host_copy_pool();  // of the current device
+
+// n reals: device element type T (float or double), host doubles.  Ordered
+// after the stream's earlier work; complete on return.
+bool host_copy_pays(long n, size_t elem);  // else a plain copy is as good
+template <typename T>
+hipError_t host_copy_out(HostCopyPool& pool, const T* dev, double* host, long n, hipStream_t s);
+template <typename T>
+hipError_t host_copy_in(HostCopyPool& pool, const double* host, T* dev, long n, hipStream_t s);
+
+}  // namespace flusi

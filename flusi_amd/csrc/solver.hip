@@ -4,6 +4,7 @@
 #include "adjoint.h"
 #include "fft_core.h"
 #include "fields.h"
+#include "hostcopy.h"
 #include "flusi_kernels.h"
 #include "h5bind.h"
 #include "host_params.h"
@@ -309,11 +310,11 @@ class Solver : public SolverBase {
   int nzpart = 0;           // partial sums the last z step wrote
   double* dpart = nullptr; int ndblocks = 0;
   double* noalloc_scratch = nullptr;  // device address of `scratch` on this context's GPU
+  double* stage = nullptr; size_t stage_n = 0;  // FP64 copies of single-precision fields
   double* red = nullptr;    // small results
   double* red_h = nullptr;  // the same in mapped host memory: read after a synchronisation, without a copy
   double* rmid = nullptr;   // reduction scratch
   int* kinds = nullptr;     // reduction kinds: [0..3] x pass, [4] energy, [8..8+DIAG_NV) diag
-  double* stage = nullptr; size_t stage_n = 0;
   std::vector<double> kx_h, ky_h, kz_h, kxt2_h, kyt2_h, kzt2_h;
   double ksy = 0.0, ksz = 0.0;  // 2 pi / yl, 2 pi / zl
   GridGeom geom{};
@@ -1736,6 +1737,11 @@ class Solver : public SolverBase {
   }
 
   // ------------------------------------------------------------ host copies
+  std::shared_ptr<HostCopyPool> host_pool;  // pinned staging shared by the contexts of this device
+  HostCopyPool& pool() {
+    if (!host_pool) host_pool = host_copy_pool();
+    return *host_pool;
+  }
   double* staging(size_t n) {
     if (n > stage_n) {
       dfree(stage);
@@ -1745,6 +1751,10 @@ class Solver : public SolverBase {
     return stage;
   }
   void copy_real_out(const void* src, double* dst, long n) {
+    if (host_copy_pays(n, sizeof(T))) {
+      HIPCHECK(host_copy_out<T>(pool(), (const T*)src, dst, n, stream));
+      return;
+    }
     if (FP64) { HIPCHECK(hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyDeviceToHost, stream)); }
     else {
       double* s = staging(n);
@@ -1754,6 +1764,10 @@ class Solver : public SolverBase {
     HIPCHECK(hipStreamSynchronize(stream));
   }
   void copy_real_in(const double* src, void* dst, long n) {
+    if (host_copy_pays(n, sizeof(T))) {
+      HIPCHECK(host_copy_in<T>(pool(), src, (T*)dst, n, stream));
+      return;
+    }
     if (FP64) { HIPCHECK(hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyHostToDevice, stream)); }
     else {
       double* s = staging(n);
