@@ -328,6 +328,7 @@ class Solver : public SolverBase {
     for (void* q : owned) (void)hipFree(q);
     for (hipEvent_t e : ins_ev) if (e) (void)hipEventDestroy(e);
     if (red_h) (void)hipHostFree(red_h);
+    if (ev_stats) (void)hipEventDestroy(ev_stats);
     if (ins_h) (void)hipHostFree(ins_h);
     if (stream) (void)hipStreamDestroy(stream);
   }
@@ -411,8 +412,14 @@ class Solver : public SolverBase {
     for (int i = 0; i < nxh; ++i) { kx_h[i] = sx * double(i); double t = (kx_h[i] / sx) / kxt; kxt2_h[i] = t * t; }
     for (int i = 0; i < ny; ++i) { ky_h[i] = sy * double(wrap(i, ny)); double t = (ky_h[i] / sy) / kyt; kyt2_h[i] = t * t; }
     for (int i = 0; i < nz; ++i) { kz_h[i] = sz * double(wrap(i, nz)); double t = (kz_h[i] / sz) / kzt; kzt2_h[i] = t * t; }
-    const size_t ntab = 2 * ((size_t)nxh + ny + nz);
-    tab = (double*)dalloc(ntab * sizeof(double));
+    // every constant table of the context: one allocation, one copy
+    std::vector<char> th;
+    auto put = [&](const void* src, size_t bytes) {
+      const size_t o = (th.size() + 255) / 256 * 256;
+      th.resize(o + bytes);
+      std::memcpy(th.data() + o, src, bytes);
+      return o;
+    };
     std::vector<double> h;
     h.insert(h.end(), kx_h.begin(), kx_h.end());
     h.insert(h.end(), ky_h.begin(), ky_h.end());
@@ -420,12 +427,34 @@ class Solver : public SolverBase {
     h.insert(h.end(), kxt2_h.begin(), kxt2_h.end());
     h.insert(h.end(), kyt2_h.begin(), kyt2_h.end());
     h.insert(h.end(), kzt2_h.begin(), kzt2_h.end());
-    HIPCHECK(hipMemcpy(tab, h.data(), ntab * sizeof(double), hipMemcpyHostToDevice));
+    const size_t o_tab = put(h.data(), h.size() * sizeof(double));
+    std::vector<int> k(8 + DIAG_NV, 0);  // reduction kinds
+    k[0] = 1;  // umax^2: max
+    for (int v = 0; v < DIAG_NV; ++v) {
+      if (v >= DG_URES && v < DG_URES + 4) k[8 + v] = 2;
+      if (v == DG_DIVMAX || v == DG_DIVMAXF) k[8 + v] = 1;
+    }
+    const size_t o_kinds = put(k.data(), k.size() * sizeof(int));
+    size_t o_tw[5] = {0}, o_pr[4] = {0};
+    if (fft_ok) {
+      const int tw[5][2] = {{nz, nz}, {ny, ny}, {nx / 2, nx / 2}, {nxh, nx}, {nx, nx}};
+      for (int i = 0; i < 5; ++i) {
+        const std::vector<C> t = make_tw(tw[i][0], tw[i][1]);
+        o_tw[i] = put(t.data(), t.size() * sizeof(C));
+      }
+      setup_prune(put, o_pr);
+    }
+    char* td = (char*)dalloc(th.size());
+    HIPCHECK(hipMemcpy(td, th.data(), th.size(), hipMemcpyHostToDevice));
+    tab = (double*)(td + o_tab);
+    kinds = (int*)(td + o_kinds);
     kx_d = tab; ky_d = kx_d + nxh; kz_d = ky_d + ny; kxt2_d = kz_d + nz; kyt2_d = kxt2_d + nxh; kzt2_d = kyt2_d + ny;
     if (fft_ok) {
-      setup_prune();
-      tw_z = make_tw(nz, nz); tw_y = make_tw(ny, ny); tw_M = make_tw(nx / 2, nx / 2); tw_N = make_tw(nxh, nx);
-      tw_X = make_tw(nx, nx);
+      tw_z = td + o_tw[0]; tw_y = td + o_tw[1]; tw_M = td + o_tw[2]; tw_N = td + o_tw[3]; tw_X = td + o_tw[4];
+      pr.ylim = (const int16_t*)(td + o_pr[0]);
+      pr.zlim = (const int16_t*)(td + o_pr[1]);
+      ptiles[0] = (uint32_t*)(td + o_pr[2]);
+      ptiles[1] = (uint32_t*)(td + o_pr[3]);
       if (const char* e = getenv("FLUSI_TILE_WAVE")) twave = atoi(e) != 0;
       if (const char* e = getenv("FLUSI_ZWAVE")) zwave = atoi(e) != 0;
       if (const char* e = getenv("FLUSI_ZSTEP_EU")) zeu = atoi(e);
@@ -448,22 +477,16 @@ class Solver : public SolverBase {
     }
     red = (double*)dalloc(sizeof(double) * 128);
     HIPCHECK(hipHostMalloc((void**)&red_h, sizeof(double) * 128, hipHostMallocDefault));
+    HIPCHECK(hipEventCreateWithFlags(&ev_stats, hipEventDisableTiming));
     rmid = (double*)dalloc(sizeof(double) * reduce_rows_scratch(DIAG_NV));
-    std::vector<int> k(8 + DIAG_NV, 0);
-    k[0] = 1;  // umax^2: max
-    for (int v = 0; v < DIAG_NV; ++v) {
-      if (v >= DG_URES && v < DG_URES + 4) k[8 + v] = 2;
-      if (v == DG_DIVMAX || v == DG_DIVMAXF) k[8 + v] = 1;
-    }
-    kinds = (int*)dalloc(sizeof(int) * k.size());
-    HIPCHECK(hipMemcpy(kinds, k.data(), sizeof(int) * k.size(), hipMemcpyHostToDevice));
     HIPCHECK(hipStreamSynchronize(stream));
   }
 
   // The dealiased region's tables, from the predicate the steppers evaluate
   // (kxt2 + kyt2) + kzt2 < 1 in FP64; each term grows with |k|, so the region
-  // is an interval of every axis.
-  void setup_prune() {
+  // is an interval of every axis.  put(data, bytes) adds a table to the
+  // context's and returns its offset.
+  template <typename F> void setup_prune(F&& put, size_t* off) {
     const int seg = 128 / (int)sizeof(C);
     auto last = [](int n, auto&& inside) { int m = -1; while (m + 1 < n && inside(m + 1)) ++m; return m; };
     pr.nkx = 1 + last(nx / 2, [&](int k) { return (kxt2_h[k] + kyt2_h[0]) + kzt2_h[0] < 1.0; });
@@ -503,28 +526,22 @@ class Solver : public SolverBase {
       }
     }
     // (fixed sizes per grid: batch members' buffers keep one layout)
-    int16_t* y = (int16_t*)dalloc(sizeof(int16_t) * yl.size());
-    int16_t* z = (int16_t*)dalloc(sizeof(int16_t) * zl.size());
-    HIPCHECK(hipMemcpy(y, yl.data(), sizeof(int16_t) * yl.size(), hipMemcpyHostToDevice));
-    HIPCHECK(hipMemcpy(z, zl.data(), sizeof(int16_t) * zl.size(), hipMemcpyHostToDevice));
-    pr.ylim = y; pr.zlim = z;
+    off[0] = put(yl.data(), sizeof(int16_t) * yl.size());
+    off[1] = put(zl.data(), sizeof(int16_t) * zl.size());
     for (int v = 0; v < 2; ++v) {
       nptiles[v] = (int)tl[v].size();
-      ptiles[v] = (uint32_t*)dalloc(sizeof(uint32_t) * tl[v].size());
-      HIPCHECK(hipMemcpy(ptiles[v], tl[v].data(), sizeof(uint32_t) * tl[v].size(), hipMemcpyHostToDevice));
+      off[2 + v] = put(tl[v].data(), sizeof(uint32_t) * tl[v].size());
     }
   }
 
-  void* make_tw(int n, int period) {
+  std::vector<C> make_tw(int n, int period) {
     std::vector<C> t(n);
     for (int m = 0; m < n; ++m) {
       const double a = -2.0 * PI * double(m) / double(period);
       t[m].x = (T)std::cos(a);
       t[m].y = (T)std::sin(a);
     }
-    void* d = dalloc(sizeof(C) * n);
-    HIPCHECK(hipMemcpy(d, t.data(), sizeof(C) * n, hipMemcpyHostToDevice));
-    return d;
+    return t;
   }
 
   // ------------------------------------------------------------ timing
@@ -667,9 +684,13 @@ class Solver : public SolverBase {
   // and the reduction of max|u|^2 and sum chi (u - us) into red[0..3].  in:
   // u_in is zero outside the dealiased region; out: only the result's modes
   // inside it are used (post_rhs with prune & 2).
-  // umax: whether the step size is derived from this right-hand side's
-  // max|u|^2 (a step's first stage).
-  void pre_rhs(const void* u_in, double t, bool with_mask = true, bool in = false, bool out = false, bool umax = true) {
+  // first: a step's first stage, whose max|u|^2 gives the step size
+  // (adjust_dt, before post_rhs).
+  bool yfwd_done = false;  // the forward y pass of the current right-hand side is launched
+  hipEvent_t ev_stats = nullptr;  // after the reduction of the first stage's statistics
+  void pre_rhs(const void* u_in, double t, bool with_mask = true, bool in = false, bool out = false, bool first = false) {
+    yfwd_done = false;
+    const bool early_yfwd = first && p.dt_fixed <= 0.0;
     if (with_mask && p.iMoving == 1 && p.iPenalization == 1) create_mask(t);
     if (p.eps < 1.0e-11) throw FlusiError(77363800, "Value of eps is very small, maybe even zero.");
     p_row = in && out ? prowc : prow;
@@ -685,7 +706,7 @@ class Solver : public SolverBase {
     a.sponge_eps_inv = a.sponge ? 1.0 / p.eps_sponge : 0.0;
     a.sponge_mask_thr = (a.sponge == 2) ? (double)1.0e-12f : 1.0e-12;
     a.partial = xpart;
-    a.want_stats = ((umax && p.dt_fixed <= 0.0) || p.iMeanFlow[0] == "dynamic" || p.iMeanFlow[1] == "dynamic" ||
+    a.want_stats = ((first && p.dt_fixed <= 0.0) || p.iMeanFlow[0] == "dynamic" || p.iMeanFlow[1] == "dynamic" ||
                     p.iMeanFlow[2] == "dynamic") ? 1 : 0;
     timed(TM_X, [&] {
       if (xwave) launch_x_rhs_wave<T>(a, stream);
@@ -701,6 +722,13 @@ class Solver : public SolverBase {
       }
     }
     kcheck("reduce x");
+    // the forward y pass does not need the step size: it runs while the host
+    // waits for max|u|^2 (post_rhs then leaves it out)
+    yfwd_done = early_yfwd;
+    if (early_yfwd) {
+      HIPCHECK(hipEventRecord(ev_stats, stream));
+      yfwd(a.sponge ? 6 : 3, out);
+    }
   }
 
   ZStepArgs zargs(int mode) {
@@ -727,7 +755,8 @@ class Solver : public SolverBase {
       const int v = zstep_tile_lines(nz, FP64, zwave) == 16;
       z.tiles = ptiles[v]; z.ntiles = nptiles[v];
     }
-    yfwd(z.sponge ? 6 : 3, (z.prune & 2) != 0);
+    if (!yfwd_done) yfwd(z.sponge ? 6 : 3, (z.prune & 2) != 0);
+    yfwd_done = false;
     nzpart = z.tiles ? z.ntiles : zstep_blocks(nz, ny, nxh, FP64, zwave);
     const bool fin = z.mode == SM_EULER || z.mode == SM_AB2 || z.mode == SM_RK2_2 || z.mode == SM_RK4_4;
     if (fin) {
@@ -746,7 +775,7 @@ class Solver : public SolverBase {
   }
 
   double host_umax() {
-    HIPCHECK(hipStreamSynchronize(stream));
+    HIPCHECK(hipEventSynchronize(ev_stats));
     return std::sqrt(red_h[0]);
   }
 
@@ -917,14 +946,14 @@ class Solver : public SolverBase {
       const int both = in ? 3 : 0;
       if (in) prune_reg(n0);
       if (it == 0) {  // fluid_time_step.f90:675-748 euler_startup
-        pre_rhs(uk, time, true, in, in);
+        pre_rhs(uk, time, true, in, in, true);
         dt1 = adjust_dt(time);
         if (dt1 != dt0) vis_dt = dt1;
         ZStepArgs z = zargs(SM_EULER);
         z.u = uk; z.r0 = reg[n0]; z.dt = dt1; z.vis_dt_new = vis_dt; z.prune = both;
         post_rhs(z);
       } else {        // :752-832 adamsbashforth
-        pre_rhs(uk, time, true, in, in);
+        pre_rhs(uk, time, true, in, in, true);
         double d = adjust_dt(time);
         if (d > p.tmax - time) d = p.tmax - time;
         dt1 = d;
@@ -938,7 +967,7 @@ class Solver : public SolverBase {
       set_state_pruned(dea);
       if (dea) set_reg_pruned(n0);
     } else if (m == "RK2") {  // :519-598
-      pre_rhs(uk, time, true, in, dea);
+      pre_rhs(uk, time, true, in, dea, true);
       dt1 = adjust_dt(time);
       const double old = vis_dt;
       if (dt1 != dt0) vis_dt = dt1;
@@ -947,19 +976,19 @@ class Solver : public SolverBase {
       ZStepArgs z = zargs(SM_RK2_1);
       z.u = uk; z.r0 = reg[0]; z.dt = dt1; z.vis_dt_old = old; z.vis_dt_new = vis_dt; z.prune = dea ? 2 : 0;
       post_rhs(z);
-      pre_rhs(uk, time, true, dea, false, false);
+      pre_rhs(uk, time, true, dea);
       ZStepArgs z2 = zargs(SM_RK2_2);
       z2.u = uk; z2.r0 = reg[0]; z2.dt = dt1; z2.prune = dea ? 1 : 0;
       post_rhs(z2);
     } else if (m == "RK4") {  // :602-671 (explicit diffusion, accumulator register)
       if (in) { prune_reg(0); prune_reg(1); }
-      pre_rhs(uk, time, true, in, in);
+      pre_rhs(uk, time, true, in, in, true);
       dt1 = adjust_dt(time);
       const int modes[4] = {SM_RK4_1, SM_RK4_2, SM_RK4_3, SM_RK4_4};
       const double ts[4] = {time, time + 0.5 * dt1, time + 0.5 * dt1, time + dt1};
       if (!in) { set_reg_pruned(0, false); set_reg_pruned(1, false); }
       for (int s = 0; s < 4; ++s) {
-        if (s > 0) pre_rhs(reg[0], ts[s], true, in, in, false);
+        if (s > 0) pre_rhs(reg[0], ts[s], true, in, in);
         ZStepArgs z = zargs(modes[s]);
         z.u = uk; z.udiff = (s == 0) ? uk : reg[0]; z.ustage = reg[0]; z.acc = reg[1]; z.dt = dt1;
         z.prune = in ? 3 : 0;
