@@ -1,5 +1,5 @@
 // Device-side building blocks shared by every transform pass: complex helpers,
-// radix-2/3/4/8 butterflies, radix plans and Stockham stages over lines held
+// radix-2/3/4/6/8/12 butterflies, radix plans and Stockham stages over lines held
 // in LDS.
 //
 // LDS addressing is padded: element a of a line sits at a + (a >> PS) (one
@@ -157,6 +157,39 @@ template <int S, typename T> struct Bfly<8, S, T> {
     a[1] = add(e[1], o1);   a[5] = sub(e[1], o1);
     a[2] = add(e[2], o2);   a[6] = sub(e[2], o2);
     a[3] = add(e[3], o3);   a[7] = sub(e[3], o3);
+  }
+};
+// radix 6 as 2 x 3: input n = (3 n1 + 2 n2) mod 6, output k = (3 (k mod 2) + 4 (k mod 3)) mod 6
+template <int S, typename T> struct Bfly<6, S, T> {
+  static __device__ __forceinline__ void run(cplx<T>* a) {
+    cplx<T> x[3] = {a[0], a[2], a[4]}, y[3] = {a[3], a[5], a[1]};
+    Bfly<3, S, T>::run(x);
+    Bfly<3, S, T>::run(y);
+#pragma unroll
+    for (int k2 = 0; k2 < 3; ++k2) {
+      a[(4 * k2) % 6] = add(x[k2], y[k2]);
+      a[(3 + 4 * k2) % 6] = sub(x[k2], y[k2]);
+    }
+  }
+};
+// Radix-12 butterfly as 3 x 4 (prime factors: no twiddles between them).
+// Input n = (4 n1 + 3 n2) mod 12, output k = (4 (k mod 3) + 9 (k mod 4)) mod 12.
+template <int S, typename T> struct Bfly<12, S, T> {
+  static __device__ __forceinline__ void run(cplx<T>* a) {
+    cplx<T> t[3][4];
+#pragma unroll
+    for (int n2 = 0; n2 < 4; ++n2) {
+      cplx<T> x[3] = {a[(3 * n2) % 12], a[(4 + 3 * n2) % 12], a[(8 + 3 * n2) % 12]};
+      Bfly<3, S, T>::run(x);
+#pragma unroll
+      for (int k1 = 0; k1 < 3; ++k1) t[k1][n2] = x[k1];
+    }
+#pragma unroll
+    for (int k1 = 0; k1 < 3; ++k1) {
+      Bfly<4, S, T>::run(t[k1]);
+#pragma unroll
+      for (int k2 = 0; k2 < 4; ++k2) a[(4 * k1 + 9 * k2) % 12] = t[k1][k2];
+    }
   }
 };
 

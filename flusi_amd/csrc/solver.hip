@@ -700,7 +700,7 @@ class Solver : public SolverBase {
     if (out) a.kout = (int)std::min<long>(prowc, nxh);
     a.in = P; a.out = P; a.fstride_in = pc; a.fstride_out = pc; a.nf = 6;
     a.mask = mask; a.us = us; a.eps_inv = 1.0 / p.eps;
-    a.mflag = mflag_valid ? mflag : nullptr; a.mzero = mzero;
+    a.mflag = mflag_valid && batch_n(bat) == 1 ? mflag : nullptr; a.mzero = mzero;
     a.sponge = sponge_code();
     a.sponge_thickness = p.sponge_thickness;
     a.sponge_eps_inv = a.sponge ? 1.0 / p.eps_sponge : 0.0;
@@ -1545,19 +1545,30 @@ class Solver : public SolverBase {
         }
       }
     });
+    // (one drawing for all steps; members of a batch are drawn by the leader)
+    if (!mflag_valid && p.iMoving != 1 && M == 1 && !capture && mflag_on) all_mask_flags();
     kcheck("create_mask");
   }
 
-  // Line flags after an insect update: insect_k writes only inside its region
-  // box, so lines outside it keep their flags; the lines crossing the box
-  // (or every line, when the flags were not valid before) are recomputed
-  // from the mask.
-  void update_mask_flags(const InsectArgs& r, bool were_valid) {
+  // Line flags of a mask that no step redraws (none, a resting sphere, a cavity)
+  void all_mask_flags() {
+    alloc_mask_flags();
+    launch_mask_flags<T>(mask, mflag, nx, ny, 0, ny - 1, 0, nz - 1, stream);
+    mflag_valid = true;
+  }
+  void alloc_mask_flags() {
     if (!mflag) {
       mflag = (uint8_t*)dalloc((size_t)ny * nz);
       mzero = dalloc(sizeof(T) * nx);
       launch_zero(mzero, sizeof(T) * nx, stream);
     }
+  }
+  // Line flags after an insect update: insect_k writes only inside its region
+  // box, so lines outside it keep their flags; the lines crossing the box
+  // (or every line, when the flags were not valid before) are recomputed
+  // from the mask.
+  void update_mask_flags(const InsectArgs& r, bool were_valid) {
+    alloc_mask_flags();
     const bool empty = r.reg_lo[0] > r.reg_hi[0] || r.reg_lo[1] > r.reg_hi[1] || r.reg_lo[2] > r.reg_hi[2];
     if (!were_valid) launch_mask_flags<T>(mask, mflag, nx, ny, 0, ny - 1, 0, nz - 1, stream);
     else if (!empty) launch_mask_flags<T>(mask, mflag, nx, ny, r.reg_lo[1], r.reg_hi[1], r.reg_lo[2], r.reg_hi[2], stream);
@@ -2107,6 +2118,7 @@ class Solver : public SolverBase {
       insect.init(*ini, p, base_dir);
     }
     if (p.iPenalization == 1) create_mask(time);
+    else if (!mflag_valid && mflag_on) all_mask_flags();  // an all-zero mask
     HIPCHECK(hipStreamSynchronize(stream));
     fields_initialized = true;
   }

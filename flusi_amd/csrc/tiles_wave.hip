@@ -1,15 +1,22 @@
 // y and z tile passes (ZINV, YINV, YFWD, plain z forward) with every line
-// transformed inside one wavefront, for line lengths 64, 128, 256 and 512.
+// transformed inside one wavefront, for line lengths 64, 96, 128, 192, 256,
+// 384 and 512.
 //
 // A workgroup owns TL lines (16 FP32 / 8 FP64: 128-byte segments on the
 // strided side) and one LDS row per line.  A line of L points lives in the
-// registers of G = L/8 lanes, lane l holding positions l + qG (q = 0..7)
-// before and after the transform; the radix-8/4 Stockham stages exchange
-// through the line's own LDS row with wave-scope ordering only.  The block
+// registers of G = L/E lanes, lane l holding positions l + qG (q = 0..E-1,
+// E = 8, or 12 where 3 divides L) before and after the transform; the Stockham
+// stages exchange through the line's own LDS row with wave-scope ordering only.  The block
 // waits twice per transform: once to turn the tile around between the
 // contiguous side (a wave's own line) and the 128-byte segments of TL lines,
 // and once before the tile is reused.  The next job's loads are issued as
 // soon as the current operands are consumed.
+//
+// Bound by HBM from 128^3 on (4-5.4 TB/s).  The radix-3 lengths ran in block
+// passes before, whose stages wait for the whole block: 96^3 FP32, two members,
+// 38 -> 28 us, 192x96x384 FP32 z inverse 37 -> 26 us, y inverse 45 -> 40 us,
+// 64x384x96 FP64 y inverse 65 -> 43 us; at a few thousand lines both forms
+// take the latency of their stages (64x32x96 FP64: 15-16 us).
 #include "fft_core.h"
 #include "flusi_kernels.h"
 #include "pass_common.h"
@@ -32,7 +39,7 @@ template <typename T, int L> struct TWShape {
   static constexpr int NW = TL / TWPlan<L>::LPW;     // waves per block
   static constexpr int NT = NW * 64;
   static constexpr int LS = line_stride<T>(L);
-  static constexpr int K = TL * L / NT;              // tile elements per thread (8)
+  static constexpr int K = TL * L / NT;              // tile elements per thread (E)
   // twiddles in LDS when two blocks still fit in 160 KB
   static constexpr bool TWL = 2 * (TL * LS + L) * (int)sizeof(cplx<T>) <= 160 * 1024;
   static constexpr size_t smem = (size_t)(TL * LS + (TWL ? L : 0)) * sizeof(cplx<T>);
@@ -57,7 +64,7 @@ template <typename T, int L, int S, bool CONTIG_IN>
 __global__ __launch_bounds__((TWShape<T, L>::NT)) void tile_wave_k(TilePassArgs a) {
   using Sh = TWShape<T, L>;
   constexpr int TL = Sh::TL, NT = Sh::NT, LS = Sh::LS, K = Sh::K;
-  constexpr int G = TWPlan<L>::G;
+  constexpr int G = TWPlan<L>::G, E = TWPlan<L>::E;
   constexpr unsigned ES = sizeof(cplx<T>);
   extern __shared__ char smem_raw[];
   cplx<T>* tile = reinterpret_cast<cplx<T>*>(smem_raw);
@@ -109,17 +116,17 @@ __global__ __launch_bounds__((TWShape<T, L>::NT)) void tile_wave_k(TilePassArgs 
     phi = lok ? min(a.pr.nyp, ((a.pr.ym0 + ym) | (SEG - 1)) + 1) : 0;
   }
 
-  // operands: CONTIG_IN - the lane's 8 positions of its own line;
+  // operands: CONTIG_IN - the lane's E positions of its own line;
   // otherwise - the thread's K tile elements (bb = e % TL, a = e / TL)
-  cplx<T> r0[8], r1[8];
+  cplx<T> r0[E], r1[E];
   auto load = [&](int jb, int which) {
     const brsrc in = make_brsrc(mshift(which ? a.jobs[jb].in1 : a.jobs[jb].in0, moff), a.ibytes);
     if (CONTIG_IN) {
       const unsigned base = (unsigned)c * (unsigned)a.sin.c + (unsigned)row * (unsigned)a.sin.b + l;
 #pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const int w = q < 4 ? l + q * G : L - l - q * G;  // |wave number|
-        const unsigned off = w <= lim ? (base + (q < 4 ? lo : hi) + q * G) * ES : kOob;
+      for (int q = 0; q < E; ++q) {
+        const int w = q < E / 2 ? l + q * G : L - l - q * G;  // |wave number|
+        const unsigned off = w <= lim ? (base + (q < E / 2 ? lo : hi) + q * G) * ES : kOob;
         const cplx<T> x = bld<T>(in, off);
         if (which) r1[q] = x; else r0[q] = x;
       }
@@ -148,16 +155,16 @@ __global__ __launch_bounds__((TWShape<T, L>::NT)) void tile_wave_k(TilePassArgs 
       const int op = o ? a.jobs[jb].op2 : a.jobs[jb].op;
       const brsrc out = make_brsrc(mshift(o ? a.jobs[jb].out2 : a.jobs[jb].out, moff), a.obytes);
       const bool pf = (o == nout - 1) && (jb + 1 < a.njobs);
-      cplx<T> v[8];
+      cplx<T> v[E];
       if (CONTIG_IN) {
 #pragma unroll
-        for (int q = 0; q < 8; ++q) v[q] = apply_op<T, L>(op, a.kscale, l + q * G, r0[q], r1[q]);
+        for (int q = 0; q < E; ++q) v[q] = apply_op<T, L>(op, a.kscale, l + q * G, r0[q], r1[q]);
         if (pf) load_job(jb + 1);
         twfft<T, L, S>(v, tw, ln, l);
         // turn the tile: natural order into the line's row, then 128-byte
         // segments of TL lines out
 #pragma unroll
-        for (int q = 0; q < 8; ++q) ln[lp<T>(l + q * G)] = v[q];
+        for (int q = 0; q < E; ++q) ln[lp<T>(l + q * G)] = v[q];
         __syncthreads();
 #pragma unroll
         for (int k = 0; k < K; ++k) {
@@ -176,16 +183,16 @@ __global__ __launch_bounds__((TWShape<T, L>::NT)) void tile_wave_k(TilePassArgs 
         __syncthreads();
         if (pf) load_job(jb + 1);
 #pragma unroll
-        for (int q = 0; q < 8; ++q) v[q] = ln[lp<T>(l + q * G)];
+        for (int q = 0; q < E; ++q) v[q] = ln[lp<T>(l + q * G)];
         wave_sync();
         twfft<T, L, S>(v, tw, ln, l);
         const unsigned base = (unsigned)c * (unsigned)a.sout.c + (unsigned)b * (unsigned)a.sout.b;
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {
+        for (int q = 0; q < E; ++q) {
           const int aa = l + q * G;
           unsigned off;
           if (a.prune == PR_YFWD) {
-            const int p = a.pr.ym0 + (q < 4 ? aa : aa - L);
+            const int p = a.pr.ym0 + (q < E / 2 ? aa : aa - L);
             off = p >= plo && p < phi ? (base + (unsigned)p) * ES : kOob;
           } else {
             off = lok ? (base + aa) * ES : kOob;
@@ -218,7 +225,7 @@ void run_tw_dir(const TilePassArgs& a, int dir, bool ci, hipStream_t s) {
 
 int tile_lines(bool fp64) { return fp64 ? TWTile<double>::TL : TWTile<float>::TL; }
 
-bool tile_wave_supported(int L) { return L == 64 || L == 128 || L == 256 || L == 512; }
+bool tile_wave_supported(int L) { return L == 64 || L == 96 || L == 128 || L == 192 || L == 256 || L == 384 || L == 512; }
 
 template <typename T>
 void launch_tile_wave(const TilePassArgs& a, int L, int dir, bool ci, hipStream_t s) {
@@ -228,8 +235,11 @@ void launch_tile_wave(const TilePassArgs& a, int L, int dir, bool ci, hipStream_
   if (a.ibytes >= kOob || a.obytes >= kOob) throw std::runtime_error("tile pass: field too large for 32-bit offsets");
   switch (L) {
     case 64: run_tw_dir<T, 64>(a, dir, ci, s); break;
+    case 96: run_tw_dir<T, 96>(a, dir, ci, s); break;
     case 128: run_tw_dir<T, 128>(a, dir, ci, s); break;
+    case 192: run_tw_dir<T, 192>(a, dir, ci, s); break;
     case 256: run_tw_dir<T, 256>(a, dir, ci, s); break;
+    case 384: run_tw_dir<T, 384>(a, dir, ci, s); break;
     case 512: run_tw_dir<T, 512>(a, dir, ci, s); break;
     default: throw std::runtime_error("in-wave tile pass: unsupported length " + std::to_string(L));
   }

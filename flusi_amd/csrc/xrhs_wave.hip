@@ -58,27 +58,6 @@ __device__ __forceinline__ double wmax(double v) {
   return v;
 }
 
-// Radix-12 butterfly as 3 x 4 (prime factors: no twiddles between them).
-// Input n = (4 n1 + 3 n2) mod 12, output k = (4 (k mod 3) + 9 (k mod 4)) mod 12.
-template <int S, typename T> struct Bfly12 {
-  static __device__ __forceinline__ void run(cplx<T>* a) {
-    cplx<T> t[3][4];
-#pragma unroll
-    for (int n2 = 0; n2 < 4; ++n2) {
-      cplx<T> x[3] = {a[(3 * n2) % 12], a[(4 + 3 * n2) % 12], a[(8 + 3 * n2) % 12]};
-      Bfly<3, S, T>::run(x);
-#pragma unroll
-      for (int k1 = 0; k1 < 3; ++k1) t[k1][n2] = x[k1];
-    }
-#pragma unroll
-    for (int k1 = 0; k1 < 3; ++k1) {
-      Bfly<4, S, T>::run(t[k1]);
-#pragma unroll
-      for (int k2 = 0; k2 < 4; ++k2) a[(4 * k1 + 9 * k2) % 12] = t[k1][k2];
-    }
-  }
-};
-
 // E = 8: 512 = 8.8.8, 256 = 8.8.4, 128 = 8.4.4, 64 = 8.8, 32 = 8.4;
 // E = 4: 256 = 4.4.4.4, 128 = 4.4.4.2, 64 = 4.4.4, 32 = 4.4.2, 96 = 6.4.4 (its
 // first stage reads its inputs from the row, see pstage0);
@@ -122,25 +101,6 @@ template <typename T, typename PP, int s> constexpr bool split_wr() {
   return true;
 }
 
-// radix 6 as 2 x 3: input n = (3 n1 + 2 n2) mod 6, output k = (3 (k mod 2) + 4 (k mod 3)) mod 6
-template <int S, typename T> struct Bfly6 {
-  static __device__ __forceinline__ void run(cplx<T>* a) {
-    cplx<T> x[3] = {a[0], a[2], a[4]}, y[3] = {a[3], a[5], a[1]};
-    Bfly<3, S, T>::run(x);
-    Bfly<3, S, T>::run(y);
-#pragma unroll
-    for (int k2 = 0; k2 < 3; ++k2) {
-      a[(4 * k2) % 6] = add(x[k2], y[k2]);
-      a[(3 + 4 * k2) % 6] = sub(x[k2], y[k2]);
-    }
-  }
-};
-template <int R, int S, typename T> __device__ __forceinline__ void bfly(cplx<T>* a) {
-  if constexpr (R == 12) Bfly12<S, T>::run(a);
-  else if constexpr (R == 6) Bfly6<S, T>::run(a);
-  else Bfly<R, S, T>::run(a);
-}
-
 // reads positions l + qG of the pair's row
 template <typename T, typename PP> __device__ __forceinline__ void row_read(cplx<T> (&v)[PP::E], const cplx<T>* ln, int l) {
   constexpr int E = PP::E, G = PP::G;
@@ -168,7 +128,7 @@ __device__ __forceinline__ void pstage(cplx<T> (&v)[PP::E], const cplx<T>* tw, c
 #pragma unroll
       for (int q = 1; q < R; ++q) x[q] = (S < 0) ? cmul(x[q], tw[q * step]) : conjmul(x[q], tw[q * step]);
     }
-    bfly<R, S, T>(x);
+    Bfly<R, S, T>::run(x);
     if constexpr (last) {
 #pragma unroll
       for (int q = 0; q < R; ++q) v[b + q * B] = x[q];
@@ -201,7 +161,7 @@ __device__ __forceinline__ void pstage0(cplx<T> (&v)[PP::E], const cplx<T>* tw, 
 #pragma unroll
   for (int q = 0; q < R; ++q) x[q] = ln[lp<T>(j + q * (N / R))];
   wave_sync();
-  bfly<R, S, T>(x);
+  Bfly<R, S, T>::run(x);
   if (l < N / R) {
 #pragma unroll
     for (int q = 0; q < R; ++q) ln[lp<T>(R * j + q)] = x[q];
