@@ -534,12 +534,22 @@ class Solver : public SolverBase {
     }
   }
 
+  // exp(-2 pi i m / period), m < n.  The angle is reduced to the first octant
+  // by whole numbers first: near 2 pi its own rounding (4e-16) was the larger
+  // part of an FP64 twiddle's error.
   std::vector<C> make_tw(int n, int period) {
     std::vector<C> t(n);
     for (int m = 0; m < n; ++m) {
-      const double a = -2.0 * PI * double(m) / double(period);
-      t[m].x = (T)std::cos(a);
-      t[m].y = (T)std::sin(a);
+      const int quad = (int)(4L * m / period);
+      int r = (int)(4L * m - (long)quad * period);  // quarter turns: r / period
+      const bool swap = 2L * r > period;
+      if (swap) r = period - r;
+      const double phi = 0.5 * PI * double(r) / double(period);
+      double c = std::cos(phi), s = std::sin(phi);
+      if (swap) std::swap(c, s);
+      const double re[4] = {c, -s, -c, s}, im[4] = {s, c, -s, -c};
+      t[m].x = (T)re[quad & 3];
+      t[m].y = (T)-im[quad & 3];
     }
     return t;
   }
@@ -1558,9 +1568,10 @@ class Solver : public SolverBase {
   }
   void alloc_mask_flags() {
     if (!mflag) {
-      mflag = (uint8_t*)dalloc((size_t)ny * nz);
-      mzero = dalloc(sizeof(T) * nx);
-      launch_zero(mzero, sizeof(T) * nx, stream);
+      const size_t zb = (sizeof(T) * nx + 255) / 256 * 256;
+      mzero = dalloc(zb + (size_t)ny * nz);
+      mflag = (uint8_t*)mzero + zb;
+      launch_zero(mzero, zb, stream);
     }
   }
   // Line flags after an insect update: insect_k writes only inside its region
