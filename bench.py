@@ -36,8 +36,6 @@ sys.path.insert(0, ROOT)
 
 METRIC = "grid-pt·steps/s at 512^3, FP32-mixed vs FP64 (force rel err≤1e-4); % HBM roofline"
 HBM_PEAK = 8.0e12          # MI355X HBM3E, bytes/s
-B_PT_RK4 = {4: 895.2, 8: 1790.5}   # algorithmic bytes per grid-point-step, RK4 (penalised)
-B_PT_RK2 = {4: 423.0, 8: 846.0}    # the same for RK2 (ensemble members)
 ENS_METRIC = "ensemble grid-pt·steps/s (48 sims: 16x64^3+16x96^3+16x128^3, RK2, FP32-mixed, one hipGraph); % HBM roofline"
 
 
@@ -57,18 +55,31 @@ def make_ini(tmpdir, n, nt):
 
 def pass_bytes(n, s, stepper="RK4"):
     """Algorithmic HBM bytes per launch of each pass at an n^3 grid (complex
-    field C = 2*(n/2+1)*n*n*s bytes, real field R = n^3*s)."""
-    C = 2 * (n // 2 + 1) * n * n * s
-    R = n ** 3 * s
-    return {
-        "ZINV": 8 * C,            # 3 fields in, 5 out
-        "YINV": 11 * C,           # 5 in, 6 out
-        "XPASS": 9 * C + R,       # 6 in, 3 out, mask (us only inside the mask)
-        "YFWD": 6 * C,            # 3 in, 3 out
-        # RK4: average of 12/15/18/12 C (stage 2 rebuilds u_n from its two
-        # stage-1 registers); RK2: 12 C in both stages
-        "ZSTEP": (14.25 if stepper == "RK4" else 12) * C,
-    }
+    field C = 2*(n/2+1)*n*n*s bytes), with the passes pruned to the dealiased
+    ellipsoid: N the modes inside it, Q its (kx, ky) shadow times nz, P its kx
+    range times ny*nz.  The mask is read only on the lines that meet the body
+    (left out here)."""
+    full = (n // 2 + 1) * n * n
+    k = np.arange(n // 2 + 1) / ((2.0 / 3.0) * (n // 2 - 1))
+    t = k * k
+    w = np.where(np.arange(n // 2 + 1) == 0, 1, 2)  # -k and +k of a whole axis
+    inside = (t[:, None, None] + t[None, :, None]) + t[None, None, :] < 1.0
+    N = int((inside * w[None, :, None] * w[None, None, :]).sum())
+    Q = int((inside[:, :, 0] * w[None, :]).sum()) * n
+    P = int(inside[:, 0, 0].sum()) * n * n
+    b = 2 * s
+    if stepper == "RK4":  # both sides of every stage; z step: 3 Q in, 9/12/15/9 state fields
+        return {"ZINV": (3 * N + 5 * Q) * b, "YINV": (5 * Q + 6 * P) * b, "XPASS": 9 * P * b, "YFWD": (3 * P + 3 * Q) * b,
+                "ZSTEP": (3 * Q + 11.25 * N) * b}
+    # RK2: the first stage prunes its result, the second its input; averages
+    return {"ZINV": (8 * full + 3 * N + 5 * Q) * b / 2, "YINV": (11 * full + 5 * Q + 6 * P) * b / 2,
+            "XPASS": (9 * full + 9 * P) * b / 2, "YFWD": (3 * P + 3 * Q + 6 * full) * b / 2,
+            "ZSTEP": (3 * Q + 9 * full + 12 * N) * b / 2}
+
+
+def step_bytes_per_point(n, s, stepper="RK4"):
+    """Algorithmic bytes per grid-point-step: the passes of every stage."""
+    return {"RK4": 4, "RK2": 2}[stepper] * sum(pass_bytes(n, s, stepper).values()) / float(n) ** 3
 
 
 def measured_traffic(n, kernel):
@@ -288,7 +299,7 @@ def run_ensemble(args):
                      "frac": ach / HBM_PEAK, "traffic": None, "kernel": best,
                      "algorithmic_bytes_per_launch": per_bytes[best] / nlaunch,
                      "avg_launch_ms": per_pass[best] / nlaunch},
-        "step_roofline_frac": B_PT_RK2[4] * value / HBM_PEAK,
+        "step_roofline_frac": step_bytes_per_point(128, 4, "RK2") * value / HBM_PEAK,
         "batched_eager_gps": pts * k_eager / dt_eager,
         "members_alone_gps": pts / dt_members,
         "pass_ms_per_step": {k: v / k_eager for k, v in per_pass.items()},
@@ -453,7 +464,7 @@ def main():
     out["pass_ms_per_step"] = {k: v / args.steps for k, v in ms32.items() if v > 0}
     out["pass_achieved_GBps"] = {k: round(pb[k] / (ms32[k] / launches / 1e3) / 1e9, 1)
                                  for k in pb if ms32.get(k, 0.0) > 0}
-    out["step_roofline_frac"] = B_PT_RK4[4] * gps32 / HBM_PEAK
+    out["step_roofline_frac"] = step_bytes_per_point(args.grid, 4) * gps32 / HBM_PEAK
 
     if not args.no_fp64:
         dt64, ms64, integ64 = run_gpu(ini, flusi_amd.FP64, args.warmup, args.steps, True)
