@@ -305,7 +305,7 @@ class Solver : public SolverBase {
   long prowc = 0;             // P row stride of the passes pruned on both sides
   // zero outside the dealiased region: the state, the two registers
   bool uk_pruned = false, reg_pruned[2] = {false, false};
-  bool xwave = false;       // right-hand-side x pass with one wavefront per line
+  bool xwave = false;       // right-hand-side x pass on pairs of lines inside one wavefront
   double* zpart = nullptr; int nzblocks = 0;
   int nzpart = 0;           // partial sums the last z step wrote
   double* dpart = nullptr; int ndblocks = 0;
