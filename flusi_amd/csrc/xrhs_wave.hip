@@ -66,9 +66,14 @@ template <int N_, int E_> struct PairPlan {
   static constexpr int N = N_, E = E_;
   static constexpr int G = N / E;     // lanes of a pair
   static constexpr int PPW = 64 / G;  // pairs of a wave
-  static constexpr int ROWS = PPW + (PPW * G < 64 ? 1 : 0);  // a spare row for lanes beyond PPW pairs
+  // 96 over 24 lanes leaves 16 lanes of a wave idle: they run the same code on
+  // a spare row, which the kernel clears first, so that all they hold is zero
+  // (a few positions of that row are read that no lane writes), and neither
+  // store nor enter the statistics
+  static constexpr int IDLE = 64 - PPW * G;
+  static constexpr int ROWS = PPW + (IDLE > 0 ? 1 : 0);
   static constexpr bool ROW0 = E == 4 && N % 3 == 0;
-  static_assert(E * G == N && (PPW * G == 64 || N == 96), "in-wave pair length");
+  static_assert(E * G == N && (IDLE == 0 || N == 96), "in-wave pair length");
   static constexpr __host__ __device__ int radix(int s) {
     int m = N;
     for (int i = 0;; ++i) {
@@ -242,6 +247,10 @@ __global__ __launch_bounds__(XW_NT) __attribute__((amdgpu_waves_per_eu(pair_wpe<
   {
     const gptr<const cplx<T>> t = (gptr<const cplx<T>>)a.twX;
     for (int i = threadIdx.x; i < N; i += blockDim.x) twl[i] = gld<T>(t + i);
+  }
+  if constexpr (PP::IDLE > 0) {  // the idle lanes' row (see PairPlan)
+    if (lane >= PPW * G)
+      for (int i = l; i < LS; i += PP::IDLE) ln[i] = mk<T>(T(0), T(0));
   }
 
   // ---- loads: the two lines' spectra at k = l + qG in X[f][q] and
@@ -425,7 +434,7 @@ __global__ __launch_bounds__(XW_NT) __attribute__((amdgpu_waves_per_eu(pair_wpe<
         const double usa = rld<T>(ru[c], m.x != T(0) ? pq : kOob), usb = rld<T>(ru[c], m.y != T(0) ? pq + N * sizeof(T) : kOob);
         const double pa = (double)m.x * a.eps_inv * ((double)X[c][0].x - usa), pv = (double)m.y * a.eps_inv * ((double)X[c][0].y - usb);
         nl[c] = mk<T>((T)((double)nl[c].x - pa), (T)((double)nl[c].y - pv));
-        if (stats) {
+        if (stats && live) {
           double t = fs[c] + pa;
           fc[c] += (fabs(fs[c]) >= fabs(pa)) ? (fs[c] - t) + pa : (pa - t) + fs[c];
           fs[c] = t;
