@@ -307,7 +307,7 @@ class Solver : public SolverBase {
   bool uk_pruned = false, reg_pruned[2] = {false, false};
   bool xwave = false;       // right-hand-side x pass on pairs of lines inside one wavefront
   double* zpart = nullptr; int nzblocks = 0;
-  int nzpart = 0;           // partial sums the last z step wrote
+  int nzpart = 0;           // energy partial sums in zpart: those of the last step's last z step
   double* dpart = nullptr; int ndblocks = 0;
   double* noalloc_scratch = nullptr;  // device address of `scratch` on this context's GPU
   double* stage = nullptr; size_t stage_n = 0;  // FP64 copies of single-precision fields
@@ -767,7 +767,6 @@ class Solver : public SolverBase {
     }
     if (!yfwd_done) yfwd(z.sponge ? 6 : 3, (z.prune & 2) != 0);
     yfwd_done = false;
-    nzpart = z.tiles ? z.ntiles : zstep_blocks(nz, ny, nxh, FP64, zwave);
     const bool fin = z.mode == SM_EULER || z.mode == SM_AB2 || z.mode == SM_RK2_2 || z.mode == SM_RK4_4;
     if (fin) {
       // set_mean_flow (fluid_time_step.f90:1066-1090) with the time of the step start
@@ -779,6 +778,8 @@ class Solver : public SolverBase {
         }
       }
       z.energy_partial = zpart;
+      const int n = z.tiles ? z.ntiles : zstep_blocks(nz, ny, nxh, FP64, zwave);
+      members([&](Solver<T>& m) { m.nzpart = n; });
     }
     timed(TM_ZSTEP, [&] { launch_zstep<T>(z, stream); });
     kcheck("zstep");
@@ -2391,6 +2392,7 @@ class Ensemble : public EnsembleBase {
     char* slab = nullptr;
     size_t stride = 0;
     int nstage = 0;         // insect mask updates per captured step
+    int nzpart = 0;         // energy partial sums a captured step writes per member
     hipEvent_t join = nullptr;
     Solver<T>* lead = nullptr;
   };
@@ -2606,6 +2608,7 @@ class Ensemble : public EnsembleBase {
         }
         L.capture = false;
         if (L.stage_slot != g.nstage) throw FlusiError(900018, "ensemble graph: unexpected number of mask updates");
+        g.nzpart = L.nzpart;
         L.dt0 = d0; L.dt1 = d1; L.vis_dt = vd; L.n0 = n0; L.n1 = n1;
         for (size_t k = 0; k < g.idx.size(); ++k) S(g.idx[k]).insect = saved[k];
         HIPCHECK(hipEventRecord(g.join, L.stream));
@@ -2655,7 +2658,10 @@ class Ensemble : public EnsembleBase {
     }
     HIPCHECK(hipEventRecord(ring_ev[r], origin));
     HIPCHECK(hipGraphLaunch(exec, origin));
-    for (Group& g : groups) g.lead->dt0 = g.lead->dt1;
+    for (Group& g : groups) {
+      g.lead->dt0 = g.lead->dt1;
+      for (int i : g.idx) S(i).nzpart = g.nzpart;  // (an eager step may have left another count)
+    }
     after_step(false);
   }
 
