@@ -197,7 +197,7 @@ template <typename T> void launch_x_rhs_wave(const XPassArgs& a, hipStream_t s);
 // its inverse transforms alone: XM_INV (1 or 3 fields) and XM_INV_UW
 template <typename T> void launch_x_inv_wave(const XPassArgs& a, int mode, hipStream_t s);
 bool x_rhs_wave_supported(int nx);
-int x_rhs_wave_blocks(int nx, int nlines, bool fp64, int nmem);  // per member of a batch of nmem
+int x_rhs_wave_blocks(int nx, int nlines, bool fp64);
 // per x line (iy, iz) of [y0, y1] x [z0, z1]: flag[iz ny + iy] = 1 where any
 // mask value of the line is nonzero, else 0 (xrhs_wave.hip)
 template <typename T>

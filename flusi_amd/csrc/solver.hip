@@ -466,7 +466,7 @@ class Solver : public SolverBase {
       xwave = x_rhs_wave_supported(nx) && !(FP64 && nx == 384 && ny * nz < 2048);
       if (const char* e = getenv("FLUSI_XWAVE")) xwave = xwave && atoi(e) != 0;
       // partial rows for either x-pass form, so the variant can change later
-      const int nxb = std::max(x_rhs_wave_supported(nx) ? x_rhs_wave_blocks(nx, ny * nz, FP64, 1) : 0,
+      const int nxb = std::max(x_rhs_wave_supported(nx) ? x_rhs_wave_blocks(nx, ny * nz, FP64) : 0,
                                x_pass_blocks(nx, ny * nz, FP64));
       xpart = (double*)dalloc(sizeof(double) * 4 * nxb);
       // room for either z-step form's partials (the variant can change later)
@@ -724,7 +724,7 @@ class Solver : public SolverBase {
     });
     kcheck("x pass");
     if (a.want_stats) {
-      const int nxblocks = xwave ? x_rhs_wave_blocks(nx, ny * nz, FP64, batch_n(bat)) : x_pass_blocks(nx, ny * nz, FP64);
+      const int nxblocks = xwave ? x_rhs_wave_blocks(nx, ny * nz, FP64) : x_pass_blocks(nx, ny * nz, FP64);
       for (int m = 0; m < batch_n(bat); ++m) {
         const long o = m * bat.mstride;
         launch_reduce_rows(mshift(xpart, o), nxblocks, 4, mshift(kinds, o), mshift(rmid, o), mshift(red, o), stream,
