@@ -64,15 +64,18 @@ class HostCopyPool {
  public:
   explicit HostCopyPool(int d) : device(d) {}
   const int device;
-  hipError_t take(std::unique_ptr<Ring>& r) {
+  // null: no pinned memory or events to be had
+  std::unique_ptr<Ring> take() {
     {
       std::lock_guard<std::mutex> g(mu_);
-      if (idle_) { r = std::move(idle_); return hipSuccess; }
+      if (idle_) return std::move(idle_);
     }
-    r.reset(new Ring());
-    const hipError_t e = r->init();
-    if (e != hipSuccess) r.reset();
-    return e;
+    std::unique_ptr<Ring> r(new Ring());
+    if (r->init() != hipSuccess) {
+      (void)hipGetLastError();  // not the next call's error
+      r.reset();
+    }
+    return r;
   }
   void give(std::unique_ptr<Ring> r) {
     std::lock_guard<std::mutex> g(mu_);
@@ -120,9 +123,9 @@ template <typename F> void run_workers(int threads, F&& work) {
 
 // out: device -> host, else host -> device
 template <typename T, bool OUT>
-hipError_t staged(HostCopyPool& pool, T* dev, double* host, long n, hipStream_t s) {
-  std::unique_ptr<Ring> ring;
-  if (hipError_t e = pool.take(ring)) return e;
+bool staged(HostCopyPool& pool, T* dev, double* host, long n, hipStream_t s, hipError_t& result) {
+  std::unique_ptr<Ring> ring = pool.take();
+  if (!ring) return false;
   const long per = (long)(kSlot / sizeof(T)), chunks = (n + per - 1) / per;
   const int threads = (int)std::min<long>({(long)kMaxThreads, (long)cpus(), (chunks + 1) / 2});
   std::atomic<long> next{0};
@@ -160,7 +163,8 @@ hipError_t staged(HostCopyPool& pool, T* dev, double* host, long n, hipStream_t 
   // (also after an error: no transfer may outlive the ring)
   const hipError_t e = hipStreamSynchronize(s);
   if (e == hipSuccess && err.load() == (int)hipSuccess) pool.give(std::move(ring));
-  return err.load() != (int)hipSuccess ? (hipError_t)err.load() : e;
+  result = err.load() != (int)hipSuccess ? (hipError_t)err.load() : e;
+  return true;
 }
 
 }  // namespace
@@ -168,17 +172,17 @@ hipError_t staged(HostCopyPool& pool, T* dev, double* host, long n, hipStream_t 
 bool host_copy_pays(long n, size_t elem) { return (size_t)n * elem >= kStagedBytes; }
 
 template <typename T>
-hipError_t host_copy_out(HostCopyPool& pool, const T* dev, double* host, long n, hipStream_t s) {
-  return staged<T, true>(pool, const_cast<T*>(dev), host, n, s);
+bool host_copy_out(HostCopyPool& pool, const T* dev, double* host, long n, hipStream_t s, hipError_t& result) {
+  return staged<T, true>(pool, const_cast<T*>(dev), host, n, s, result);
 }
 template <typename T>
-hipError_t host_copy_in(HostCopyPool& pool, const double* host, T* dev, long n, hipStream_t s) {
-  return staged<T, false>(pool, dev, const_cast<double*>(host), n, s);
+bool host_copy_in(HostCopyPool& pool, const double* host, T* dev, long n, hipStream_t s, hipError_t& result) {
+  return staged<T, false>(pool, dev, const_cast<double*>(host), n, s, result);
 }
 
-template hipError_t host_copy_out<float>(HostCopyPool&, const float*, double*, long, hipStream_t);
-template hipError_t host_copy_out<double>(HostCopyPool&, const double*, double*, long, hipStream_t);
-template hipError_t host_copy_in<float>(HostCopyPool&, const double*, float*, long, hipStream_t);
-template hipError_t host_copy_in<double>(HostCopyPool&, const double*, double*, long, hipStream_t);
+template bool host_copy_out<float>(HostCopyPool&, const float*, double*, long, hipStream_t, hipError_t&);
+template bool host_copy_out<double>(HostCopyPool&, const double*, double*, long, hipStream_t, hipError_t&);
+template bool host_copy_in<float>(HostCopyPool&, const double*, float*, long, hipStream_t, hipError_t&);
+template bool host_copy_in<double>(HostCopyPool&, const double*, double*, long, hipStream_t, hipError_t&);
 
 }  // namespace flusi

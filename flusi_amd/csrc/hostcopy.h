@@ -11,11 +11,12 @@ class HostCopyPool;
 std::shared_ptr<HostCopyPool> host_copy_pool();  // of the current device
 
 // n reals: device element type T (float or double), host doubles.  Ordered
-// after the stream's earlier work; complete on return.
+// after the stream's earlier work; complete on return, with its outcome in
+// `result`.  False: no staging memory, nothing copied (a plain copy needs none).
 bool host_copy_pays(long n, size_t elem);  // else a plain copy is as good
 template <typename T>
-hipError_t host_copy_out(HostCopyPool& pool, const T* dev, double* host, long n, hipStream_t s);
+bool host_copy_out(HostCopyPool& pool, const T* dev, double* host, long n, hipStream_t s, hipError_t& result);
 template <typename T>
-hipError_t host_copy_in(HostCopyPool& pool, const double* host, T* dev, long n, hipStream_t s);
+bool host_copy_in(HostCopyPool& pool, const double* host, T* dev, long n, hipStream_t s, hipError_t& result);
 
 }  // namespace flusi

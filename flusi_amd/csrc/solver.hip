@@ -1803,8 +1803,9 @@ class Solver : public SolverBase {
     return stage;
   }
   void copy_real_out(const void* src, double* dst, long n) {
-    if (host_copy_pays(n, sizeof(T))) {
-      HIPCHECK(host_copy_out<T>(pool(), (const T*)src, dst, n, stream));
+    hipError_t staged = hipSuccess;
+    if (host_copy_pays(n, sizeof(T)) && host_copy_out<T>(pool(), (const T*)src, dst, n, stream, staged)) {
+      HIPCHECK(staged);
       return;
     }
     if (FP64) { HIPCHECK(hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyDeviceToHost, stream)); }
@@ -1816,8 +1817,9 @@ class Solver : public SolverBase {
     HIPCHECK(hipStreamSynchronize(stream));
   }
   void copy_real_in(const double* src, void* dst, long n) {
-    if (host_copy_pays(n, sizeof(T))) {
-      HIPCHECK(host_copy_in<T>(pool(), src, (T*)dst, n, stream));
+    hipError_t staged = hipSuccess;
+    if (host_copy_pays(n, sizeof(T)) && host_copy_in<T>(pool(), src, (T*)dst, n, stream, staged)) {
+      HIPCHECK(staged);
       return;
     }
     if (FP64) { HIPCHECK(hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyHostToDevice, stream)); }
