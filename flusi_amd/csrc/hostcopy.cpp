@@ -36,6 +36,17 @@ constexpr int kMaxThreads = 8;
 constexpr size_t kStagedBytes = 48u << 20;  // transfers from which the threads pay
 constexpr size_t kSlot = 4u << 20;
 
+// makes a device current for this thread while alive
+struct DeviceScope {
+  int old = -1;
+  hipError_t status;
+  explicit DeviceScope(int d) {
+    if ((status = hipGetDevice(&old)) == hipSuccess && old != d) status = hipSetDevice(d);
+    else old = -1;
+  }
+  ~DeviceScope() { if (old >= 0) (void)hipSetDevice(old); }
+};
+
 // pinned slots and their events, two per thread
 struct Ring {
   char* mem = nullptr;
@@ -87,11 +98,9 @@ class HostCopyPool {
   std::unique_ptr<Ring> idle_;
 };
 
-std::shared_ptr<HostCopyPool> host_copy_pool() {
+std::shared_ptr<HostCopyPool> host_copy_pool(int d) {
   static std::mutex mu;
   static std::map<int, std::weak_ptr<HostCopyPool>> pools;
-  int d = 0;
-  (void)hipGetDevice(&d);
   std::lock_guard<std::mutex> g(mu);
   std::shared_ptr<HostCopyPool> p = pools[d].lock();
   if (!p) pools[d] = p = std::make_shared<HostCopyPool>(d);
@@ -124,6 +133,7 @@ template <typename F> void run_workers(int threads, F&& work) {
 // out: device -> host, else host -> device
 template <typename T, bool OUT>
 bool staged(HostCopyPool& pool, T* dev, double* host, long n, hipStream_t s, hipError_t& result) {
+  const DeviceScope scope(pool.device);  // the ring's events are the stream's device's
   std::unique_ptr<Ring> ring = pool.take();
   if (!ring) return false;
   const long per = (long)(kSlot / sizeof(T)), chunks = (n + per - 1) / per;
@@ -136,7 +146,8 @@ bool staged(HostCopyPool& pool, T* dev, double* host, long n, hipStream_t s, hip
     return e == hipSuccess;
   };
   auto work = [&](int w) {
-    if (!check(hipSetDevice(pool.device))) return;
+    const DeviceScope on(pool.device);
+    if (!check(on.status)) return;
     long c[2] = {-1, -1};  // the chunk in each slot
     auto len = [&](long k) { return (size_t)std::min(per, n - k * per); };
     auto slot = [&](int i) { return reinterpret_cast<T*>(ring->mem + (size_t)(2 * w + i) * kSlot); };

@@ -8,11 +8,12 @@ namespace flusi {
 // One pool of pinned staging memory per device, shared by the contexts on it;
 // it is freed with the last of them.
 class HostCopyPool;
-std::shared_ptr<HostCopyPool> host_copy_pool();  // of the current device
+std::shared_ptr<HostCopyPool> host_copy_pool(int device);
 
-// n reals: device element type T (float or double), host doubles.  Ordered
-// after the stream's earlier work; complete on return, with its outcome in
-// `result`.  False: no staging memory, nothing copied (a plain copy needs none).
+// n reals: device element type T (float or double), host doubles; the pool's
+// device holds them, whichever is current for the caller.  Ordered after the
+// stream's earlier work; complete on return, with its outcome in `result`.
+// False: no staging memory, nothing copied (a plain copy needs none).
 bool host_copy_pays(long n, size_t elem);  // else a plain copy is as good
 template <typename T>
 bool host_copy_out(HostCopyPool& pool, const T* dev, double* host, long n, hipStream_t s, hipError_t& result);

@@ -246,6 +246,7 @@ class Solver : public SolverBase {
   using C = typename V2<T>::t;
   static constexpr bool FP64 = sizeof(T) == 8;
   hipStream_t stream = nullptr;
+  int device = 0;           // current when the context was set up: its stream and memory are on it
   // device memory
   void* uk = nullptr;
   void* reg[2] = {nullptr, nullptr};
@@ -376,6 +377,7 @@ class Solver : public SolverBase {
     npts = (long)nx * ny * nz;
     nc = (long)nxh * ny * nz;
     geom = GridGeom{nx, ny, nz, nxh, npts, nc, p.dx(), p.dy(), p.dz(), p.xl, p.yl, p.zl, p.periodic ? 1 : 0};
+    HIPCHECK(hipGetDevice(&device));
     HIPCHECK(hipStreamCreate(&stream));
     noalloc_scratch = scratch_address();  // once per device, with this context's device current
     const size_t cs = sizeof(C) * nc;
@@ -1791,7 +1793,7 @@ class Solver : public SolverBase {
   // ------------------------------------------------------------ host copies
   std::shared_ptr<HostCopyPool> host_pool;  // pinned staging shared by the contexts of this device
   HostCopyPool& pool() {
-    if (!host_pool) host_pool = host_copy_pool();
+    if (!host_pool) host_pool = host_copy_pool(device);
     return *host_pool;
   }
   double* staging(size_t n) {

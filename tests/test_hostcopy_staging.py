@@ -89,7 +89,7 @@ def _run(tmp_path, body):
 def test_round_trips(tmp_path):
     _run(tmp_path, """
   int s = 0;
-  auto pool = host_copy_pool();
+  auto pool = host_copy_pool(0);
   if (round_trip<double>(*pool, &s) || round_trip<float>(*pool, &s)) return 1;
   pool.reset();
   CHECK(allocs == frees);""")
@@ -101,7 +101,7 @@ def test_no_staging_memory_is_not_an_error(tmp_path, what):
     copy plainly; a transfer that fails is an error."""
     _run(tmp_path, f"""
   int s = 0;
-  auto pool = host_copy_pool();
+  auto pool = host_copy_pool(0);
   const long n = 7000000;
   std::vector<double> a(n, 1.0), dev(n, 0.0);
   hipError_t e = hipSuccess;
@@ -114,3 +114,14 @@ def test_no_staging_memory_is_not_an_error(tmp_path, what):
   CHECK(host_copy_in<double>(*pool, a.data(), dev.data(), n, &s, e) && e == hipSuccess && dev[n - 1] == 1.0);
   fail_copies = 1;
   CHECK(host_copy_in<double>(*pool, a.data(), dev.data(), n, &s, e) && e != hipSuccess);""")
+
+
+def test_device_of_the_context(tmp_path):
+    """The events are made and recorded on the pool's device, and the caller's
+    current device is left as it was."""
+    _run(tmp_path, """
+  int s = 1;
+  cur_device = 0;
+  auto pool = host_copy_pool(1);
+  if (round_trip<double>(*pool, &s) || round_trip<float>(*pool, &s)) return 1;
+  CHECK(faults == 0 && cur_device == 0);""")
