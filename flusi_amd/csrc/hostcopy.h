@@ -14,7 +14,7 @@ std::shared_ptr<HostCopyPool> host_copy_pool(int device);
 // device holds them, whichever is current for the caller.  Ordered after the
 // stream's earlier work; complete on return, with its outcome in `result`.
 // False: no staging memory, nothing copied (a plain copy needs none).
-bool host_copy_pays(long n, size_t elem);  // else a plain copy is as good
+bool host_copy_pays(const void* host, long n, size_t elem);  // else a plain copy is as good
 template <typename T>
 bool host_copy_out(HostCopyPool& pool, const T* dev, double* host, long n, hipStream_t s, hipError_t& result);
 template <typename T>

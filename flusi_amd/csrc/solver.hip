@@ -1806,7 +1806,7 @@ class Solver : public SolverBase {
   }
   void copy_real_out(const void* src, double* dst, long n) {
     hipError_t staged = hipSuccess;
-    if (host_copy_pays(n, sizeof(T)) && host_copy_out<T>(pool(), (const T*)src, dst, n, stream, staged)) {
+    if (host_copy_pays(dst, n, sizeof(T)) && host_copy_out<T>(pool(), (const T*)src, dst, n, stream, staged)) {
       HIPCHECK(staged);
       return;
     }
@@ -1820,7 +1820,7 @@ class Solver : public SolverBase {
   }
   void copy_real_in(const double* src, void* dst, long n) {
     hipError_t staged = hipSuccess;
-    if (host_copy_pays(n, sizeof(T)) && host_copy_in<T>(pool(), src, (T*)dst, n, stream, staged)) {
+    if (host_copy_pays(src, n, sizeof(T)) && host_copy_in<T>(pool(), src, (T*)dst, n, stream, staged)) {
       HIPCHECK(staged);
       return;
     }

@@ -46,6 +46,14 @@ inline hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
   if (e->device != *s) ++faults;  // an event of another device
   return hipSuccess;
 }
+enum hipMemoryType { hipMemoryTypeHost, hipMemoryTypeDevice, hipMemoryTypeManaged, hipMemoryTypeUnregistered };
+struct hipPointerAttribute_t { hipMemoryType type; };
+inline int pointer_type = -1;  // -1: the call knows nothing of the address
+inline hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void*) {
+  if (pointer_type < 0) return hip_ret(hipErrorInvalidValue);
+  a->type = (hipMemoryType)pointer_type;
+  return hipSuccess;
+}
 inline hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 inline hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 inline hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
@@ -125,3 +133,22 @@ def test_device_of_the_context(tmp_path):
   auto pool = host_copy_pool(1);
   if (round_trip<double>(*pool, &s) || round_trip<float>(*pool, &s)) return 1;
   CHECK(faults == 0 && cur_device == 0);""")
+
+
+def test_memory_the_runtime_knows(tmp_path):
+    """Pinned arrays of FP64 fields, managed and device memory are copied
+    plainly, as everything below the threshold is."""
+    _run(tmp_path, """
+  const void* p = &events;
+  const long n = 7000000, m = 2 * n;
+  for (int t : {-1, (int)hipMemoryTypeUnregistered}) {
+    pointer_type = t;
+    CHECK(host_copy_pays(p, n, 8) && host_copy_pays(p, m, 4) && hipGetLastError() == hipSuccess);
+    CHECK(!host_copy_pays(p, n / 2, 8) && !host_copy_pays(p, n, 4));
+  }
+  pointer_type = hipMemoryTypeHost;
+  CHECK(!host_copy_pays(p, n, 8) && host_copy_pays(p, m, 4));
+  for (int t : {(int)hipMemoryTypeDevice, (int)hipMemoryTypeManaged}) {
+    pointer_type = t;
+    CHECK(!host_copy_pays(p, n, 8) && !host_copy_pays(p, m, 4));
+  }""")
