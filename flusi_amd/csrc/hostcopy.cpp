@@ -16,6 +16,12 @@
 // core after its last parallel loop, a thread of this copy can wait a time
 // slice of a few milliseconds for a core (three 19 MB copies of a host
 // program between conversions of its own: 3.1 -> 6.4 ms with threads).
+//
+// The pinned slots cost 4 ms (64 MB) when they are made, once while contexts of
+// a device live.  Copies out regain that at once.  Copies in do only from some
+// size on (kMakeIn): a smaller one that finds no slots is left to the plain
+// copy once, for a program that sets one state and steps on (50 MB of FP64: in
+// 1.8 ms plain, 5.1 ms with the slots to be made, 1.4 ms with slots there).
 #include "hostcopy.h"
 #include <algorithm>
 #include <atomic>
@@ -34,7 +40,11 @@ namespace {
 
 constexpr int kMaxThreads = 8;
 constexpr size_t kStagedBytes = 48u << 20;  // transfers from which the threads pay
-constexpr size_t kSlot = 4u << 20;
+constexpr size_t kMakeIn[2] = {96u << 20, 320u << 20};  // FP32, FP64 transfers in that regain the slots' making
+// bytes of a slot: half the slots' cost for the smaller transfers, which run as
+// fast with 2 MB (50 MB of FP64: out 1.6 / 1.9 ms, in 1.42 / 1.36); larger ones
+// do not (403 MB: 35 / 21 ms)
+size_t slot_bytes(size_t transfer) { return transfer < (96u << 20) ? 2u << 20 : 4u << 20; }
 
 // makes a device current for this thread while alive
 struct DeviceScope {
@@ -49,8 +59,10 @@ struct DeviceScope {
 
 // pinned slots and their events, two per thread
 struct Ring {
+  const size_t slot;
   char* mem = nullptr;
   hipEvent_t ev[2 * kMaxThreads] = {};
+  explicit Ring(size_t bytes) : slot(bytes) {}
   ~Ring() {
     for (hipEvent_t e : ev) if (e) (void)hipEventDestroy(e);
     if (mem) (void)hipHostFree(mem);
@@ -58,7 +70,7 @@ struct Ring {
   hipError_t init() {
     for (hipEvent_t& e : ev)
       if (hipError_t r = hipEventCreateWithFlags(&e, hipEventDisableTiming)) return r;
-    return hipHostMalloc((void**)&mem, kSlot * 2 * kMaxThreads, hipHostMallocDefault);
+    return hipHostMalloc((void**)&mem, slot * 2 * kMaxThreads, hipHostMallocDefault);
   }
 };
 
@@ -75,13 +87,23 @@ class HostCopyPool {
  public:
   explicit HostCopyPool(int d) : device(d) {}
   const int device;
-  // null: no pinned memory or events to be had
-  std::unique_ptr<Ring> take() {
+  // A ring for `transfer` bytes.  make: one is made where there is none or only
+  // one of smaller slots; else a smaller one serves, and where there is none
+  // the first call gets none.  Null also: no pinned memory or events to be had.
+  std::unique_ptr<Ring> take(size_t transfer, bool make) {
+    const size_t slot = slot_bytes(transfer);
+    std::unique_ptr<Ring> r;
     {
       std::lock_guard<std::mutex> g(mu_);
-      if (idle_) return std::move(idle_);
+      r = std::move(idle_);
+      if (!r && !make && !declined_) {
+        declined_ = true;
+        return r;
+      }
     }
-    std::unique_ptr<Ring> r(new Ring());
+    if (r && (!make || r->slot >= slot)) return r;
+    r.reset();  // (its memory first)
+    r.reset(new Ring(slot));
     if (r->init() != hipSuccess) {
       (void)hipGetLastError();  // not the next call's error
       r.reset();
@@ -90,12 +112,13 @@ class HostCopyPool {
   }
   void give(std::unique_ptr<Ring> r) {
     std::lock_guard<std::mutex> g(mu_);
-    if (!idle_) idle_ = std::move(r);
+    if (!idle_ || idle_->slot < r->slot) std::swap(idle_, r);
   }
 
  private:
   std::mutex mu_;
   std::unique_ptr<Ring> idle_;
+  bool declined_ = false;  // a copy has been left to the plain copy for want of a ring
 };
 
 std::shared_ptr<HostCopyPool> host_copy_pool(int d) {
@@ -134,9 +157,10 @@ template <typename F> void run_workers(int threads, F&& work) {
 template <typename T, bool OUT>
 bool staged(HostCopyPool& pool, T* dev, double* host, long n, hipStream_t s, hipError_t& result) {
   const DeviceScope scope(pool.device);  // the ring's events are the stream's device's
-  std::unique_ptr<Ring> ring = pool.take();
+  const size_t bytes = (size_t)n * sizeof(T);
+  std::unique_ptr<Ring> ring = pool.take(bytes, OUT || bytes >= kMakeIn[sizeof(T) == 8]);
   if (!ring) return false;
-  const long per = (long)(kSlot / sizeof(T)), chunks = (n + per - 1) / per;
+  const long per = (long)(ring->slot / sizeof(T)), chunks = (n + per - 1) / per;
   const int threads = (int)std::min<long>({(long)kMaxThreads, (long)cpus(), (chunks + 1) / 2});
   std::atomic<long> next{0};
   std::atomic<int> err{(int)hipSuccess};
@@ -150,7 +174,7 @@ bool staged(HostCopyPool& pool, T* dev, double* host, long n, hipStream_t s, hip
     if (!check(on.status)) return;
     long c[2] = {-1, -1};  // the chunk in each slot
     auto len = [&](long k) { return (size_t)std::min(per, n - k * per); };
-    auto slot = [&](int i) { return reinterpret_cast<T*>(ring->mem + (size_t)(2 * w + i) * kSlot); };
+    auto slot = [&](int i) { return reinterpret_cast<T*>(ring->mem + (size_t)(2 * w + i) * ring->slot); };
     auto fetch = [&](int i) {  // the next chunk into slot i
       const long k = next.fetch_add(1);
       if (k >= chunks || err.load() != (int)hipSuccess) return false;

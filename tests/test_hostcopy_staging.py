@@ -68,12 +68,15 @@ MAIN = r"""
 #include <vector>
 using namespace flusi;
 #define CHECK(x) do { if (!(x)) { std::printf("line %d: %s\n", __LINE__, #x); return 1; } } while (0)
+// with slots made by a copy out: a pool's first small copy in makes none
 template <typename T> int round_trip(HostCopyPool& pool, int* stream) {
   const long n = 13000003;  // 48 MB on the wire and a remainder
   std::vector<double> a(n), b(n);
   std::vector<T> dev(n);
   for (long i = 0; i < n; ++i) a[i] = 1.0 / (double)(i + 1);
   hipError_t e = hipErrorInvalidValue;
+  CHECK(host_copy_out<T>(pool, dev.data(), b.data(), n, stream, e) && e == hipSuccess);
+  e = hipErrorInvalidValue;
   CHECK(host_copy_in<T>(pool, a.data(), dev.data(), n, stream, e) && e == hipSuccess);
   CHECK(host_copy_out<T>(pool, dev.data(), b.data(), n, stream, e) && e == hipSuccess);
   for (long i = 0; i < n; ++i) CHECK(dev[i] == (T)a[i] && b[i] == (double)dev[i]);
@@ -152,3 +155,26 @@ def test_memory_the_runtime_knows(tmp_path):
     pointer_type = t;
     CHECK(!host_copy_pays(p, n, 8) && !host_copy_pays(p, m, 4));
   }""")
+
+
+def test_when_slots_are_made(tmp_path):
+    """A small copy in makes none at first; a copy out, a second one in and a
+    large one in do, and a larger copy's replace smaller slots."""
+    _run(tmp_path, """
+  int s = 0;
+  const long n = 7000000, big = 45000000;  // 56 and 360 MB of FP64
+  std::vector<double> a(big, 2.0), dev(big, 0.0);
+  hipError_t e = hipSuccess;
+  auto pool = host_copy_pool(0);
+  CHECK(!host_copy_in<double>(*pool, a.data(), dev.data(), n, &s, e) && allocs == 0 && dev[0] == 0.0);
+  CHECK(host_copy_in<double>(*pool, a.data(), dev.data(), n, &s, e) && allocs == 1 && dev[n - 1] == 2.0);
+  CHECK(host_copy_in<double>(*pool, a.data(), dev.data(), big / 2, &s, e) && allocs == 1 && dev[big / 2 - 1] == 2.0);
+  CHECK(host_copy_in<double>(*pool, a.data(), dev.data(), big, &s, e) && allocs == 2 && frees == 1 && dev[big - 1] == 2.0);
+  CHECK(host_copy_out<double>(*pool, dev.data(), a.data(), n, &s, e) && allocs == 2);
+  pool.reset();
+  CHECK(frees == 2);
+  pool = host_copy_pool(0);
+  CHECK(host_copy_out<double>(*pool, dev.data(), a.data(), n, &s, e) && allocs == 3);
+  pool.reset();
+  pool = host_copy_pool(0);
+  CHECK(host_copy_in<double>(*pool, a.data(), dev.data(), big, &s, e) && allocs == 4);""")
