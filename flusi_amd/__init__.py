@@ -388,8 +388,8 @@ class Flusi:
         return g
 
     def autotune(self, reps: int = 3):
-        """Picks the fastest kernel variant for this grid (cached per grid,
-        precision and batch size); returns (variant[6], ms per right-hand side)."""
+        """Picks the fastest kernel variant for this grid and method (cached per
+        grid, precision, batch size and method); returns (variant[6], ms per right-hand side)."""
         v = (_I * 6)()
         ms = ctypes.c_double()
         self._check(self._lib.flusi_autotune(self._ctx, int(reps), v, ctypes.byref(ms)))

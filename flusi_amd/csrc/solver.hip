@@ -848,20 +848,28 @@ class Solver : public SolverBase {
   // y/z passes, operand prefetch in the block passes, the in-wave (line pairs)
   // or the block x pass, and the in-wave or block z
   // step.  autotune() runs `reps` right-hand sides of the current state (the
-  // whole batch when one is active) for every variant the grid allows and
-  // keeps the fastest; results are cached per grid, precision, sponge and
-  // batch size for the life of the process.
+  // whole batch when one is active), pruned as the method's steps are, for
+  // every variant the grid allows and keeps the fastest; results are cached
+  // per grid, precision, sponge, batch size, method and pruning for the life
+  // of the process.
   struct Variant { int twave, tpf, xwave, xwpe, zwave, zeu; };
   Variant variant() const { return Variant{twave, tpf, xwave, xwpe, zwave, zeu}; }
   void apply(const Variant& v) {
     twave = v.twave != 0; tpf = v.tpf != 0; xwave = v.xwave != 0; xwpe = v.xwpe; zwave = v.zwave != 0; zeu = v.zeu;
   }
   double time_rhs(int reps) {
-    auto rhs = [&] {
-      pre_rhs(uk, time, false);
+    auto one = [&](bool in, bool out, bool first) {
+      pre_rhs(uk, time, false, in, out, first);
       ZStepArgs z = zargs(SM_RHS_ONLY);
       z.rhs_out = P; z.udiff = uk;
+      z.prune = (in ? 1 : 0) | (out ? 2 : 0);
       post_rhs(z);
+    };
+    // (see fluid_timestep; RK4: its stages after the first)
+    const bool dea = prunes(), rk2 = p.method == "RK2";
+    auto rhs = [&] {
+      if (rk2) { one(false, dea, true); one(dea, false, false); }
+      else one(dea, dea, p.method == "AB2");
     };
     rhs();  // first launches of a variant set its LDS limits
     hipEvent_t e0, e1;
@@ -873,7 +881,7 @@ class Solver : public SolverBase {
     float ms = 0.f;
     HIPCHECK(hipEventElapsedTime(&ms, e0, e1));
     (void)hipEventDestroy(e0); (void)hipEventDestroy(e1);
-    return ms / std::max(reps, 1);
+    return ms / (std::max(reps, 1) * (rk2 ? 2 : 1));
   }
   std::vector<Variant> candidates() const {
     const bool tw_any = tile_wave_supported(ny) || tile_wave_supported(nz);
@@ -905,7 +913,8 @@ class Solver : public SolverBase {
   static std::mutex& tune_mutex() { static std::mutex mu; return mu; }
   std::string tune_key() const {
     return std::to_string(nx) + "x" + std::to_string(ny) + "x" + std::to_string(nz) + (FP64 ? ":f64" : ":f32") +
-           ":sp" + std::to_string(sponge_code()) + ":m" + std::to_string(batch_n(bat));
+           ":sp" + std::to_string(sponge_code()) + ":m" + std::to_string(batch_n(bat)) + ":" + p.method +
+           (prunes() ? ":p" : "") + (p.dt_fixed <= 0.0 ? ":a" : "");
   }
   static constexpr int kVariantInts = 6;
   // v: the chosen variant (6 ints: twave, tpf, xwave, xwpe, zwave, zeu); ms: its

@@ -164,9 +164,10 @@ int flusi_timers(flusi_ctx* ctx, int enable, double* ms, const char** names);
 
 /* Kernel-variant autotuner (no counterpart in the reference, which has one
  * FFT library plan per transform, cof_p3dfft.f90:160-180 p3dfft_setup).
- * Runs `reps` right-hand sides of the current state for every variant the
- * grid allows and keeps the fastest for this context; results are cached per
- * grid, precision and batch size for the life of the process.
+ * Runs `reps` right-hand sides of the current state, as the .ini's method makes
+ * them, for every variant the grid allows and keeps the fastest for this
+ * context; results are cached per grid, precision, batch size and method for
+ * the life of the process.
  * variant[6] (may be NULL): in-wave y/z passes, block-pass prefetch, one-wave
  * x pass, its waves-per-SIMD register budget, in-wave z step, epilogue
  * positions the block z step schedules together (0 = all).  ms: time of one
