@@ -1053,6 +1053,14 @@ class Solver : public SolverBase {
     });
   }
 
+  // the same for the registers of the next step, before it is captured: a
+  // recorded clearing would run in every replay
+  void prune_step_regs() {
+    if (!prunes()) return;
+    if (p.method == "RK2") prune_reg(0);
+    else if (p.method == "RK4" && state_pruned()) { prune_reg(0); prune_reg(1); }
+  }
+
   void cal_nlk(double t, double* nlk, double* u) override {
     need_fft();
     if (!fields_initialized) throw FlusiError(900004, "fields not initialised (call flusi_init_fields)");
@@ -2594,6 +2602,10 @@ class Ensemble : public EnsembleBase {
       g.nstage = mask_updates(*g.lead);
       Solver<T>& L = *g.lead;
       L.timers(0, nullptr);  // no event timing inside the graph
+      {
+        BatchScope bs(L, g.idx.size(), g.stride);
+        L.prune_step_regs();
+      }
       if (g.nstage && !L.ins_cap)
         L.ins_cap = (InsectArgs*)L.dalloc(sizeof(InsectArgs) * Solver<T>::INS_SLOTS * g.idx.size());
     }
