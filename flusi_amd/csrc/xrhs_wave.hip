@@ -539,9 +539,8 @@ __global__ __launch_bounds__(XW_NT) __attribute__((amdgpu_waves_per_eu(pair_wpe<
 // pass, four / eight a lane: FP32 64^3 11.4 / 12.8 us, 128^3 29.0 / 26.4 us;
 // FP32 96x64x64, four / twelve: 14.1 / 19.6 us).  FP64 keeps four up to nx = 256: eight
 // positions of six fields leave no room for a second wave per SIMD without
-// spills (64^3 13.2 / 13.9 us, 256x128x128 76 / 82 us).  The plan and the
-// waves of a block (the statistics' order of summation) do not depend on the
-// batch: a member's results are those of its own run.
+// spills (64^3 13.2 / 13.9 us, 256x128x128 76 / 82 us).  The plan does not
+// depend on the batch: a member's results are those of its own run.
 int pair_e(int nx, long nlines, bool fp64) {
   const bool small = nlines * nx < (1L << 20);
   if (nx % 3 == 0) return nx == 96 && small ? 4 : 12;
@@ -558,7 +557,10 @@ int pair_waves(int nx, long nlines, int e) {
 template <typename T, int N, int E, int VAR, int PR, int NF = 6>
 void run_pair(const XPassArgs& a, hipStream_t s) {
   using PP = PairPlan<N, E>;
-  const int w = pair_waves(N, a.nlines, E), ppb = w * PP::PPW;
+  // with statistics one member's lines decide: the waves of a block are their
+  // order of summation, which must not depend on the batch
+  const bool stats = VAR == 1 || (VAR == 2 && a.want_stats);
+  const int w = pair_waves(N, (long)a.nlines * (stats ? 1 : batch_n(a.bat)), E), ppb = w * PP::PPW;
   static_assert(pair_smem<T, PP>(XW_NT / 64) + sizeof(double) * XW_NT / 16 <= 65536, "LDS of a block");
   const int blocks = (a.nlines / 2 + ppb - 1) / ppb;
   const size_t smem = pair_smem<T, PP>(w);
@@ -663,6 +665,7 @@ bool x_rhs_wave_supported(int nx) {
   return nx == 32 || nx == 48 || nx == 64 || nx == 96 || nx == 128 || nx == 192 || nx == 256 || nx == 384 || nx == 512;
 }
 
+// with statistics: the rows of `partial` per member
 int x_rhs_wave_blocks(int nx, int nlines, bool fp64) {
   const int e = pair_e(nx, nlines, fp64);
   const int ppb = pair_waves(nx, nlines, e) * (64 / (nx / e));
