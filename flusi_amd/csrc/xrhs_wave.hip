@@ -248,10 +248,6 @@ __global__ __launch_bounds__(XW_NT) __attribute__((amdgpu_waves_per_eu(pair_wpe<
     const gptr<const cplx<T>> t = (gptr<const cplx<T>>)a.twX;
     for (int i = threadIdx.x; i < N; i += blockDim.x) twl[i] = gld<T>(t + i);
   }
-  if constexpr (PP::IDLE > 0) {  // the idle lanes' row (see PairPlan)
-    if (lane >= PPW * G)
-      for (int i = l; i < LS; i += PP::IDLE) ln[i] = mk<T>(T(0), T(0));
-  }
 
   // ---- loads: the two lines' spectra at k = l + qG in X[f][q] and
   // X[f][E - QL + q], and (not PIN) at k = N/2 on lane 0
@@ -283,6 +279,10 @@ __global__ __launch_bounds__(XW_NT) __attribute__((amdgpu_waves_per_eu(pair_wpe<
         nyq[f] = f == 4 ? mk<T>(xa.x + kx * va.y, xb.x + kx * vb.y) : mk<T>(-kx * va.y - xa.x, -kx * vb.y - xb.x);
       }
     }
+  }
+  if constexpr (PP::IDLE > 0) {  // the idle lanes' row (see PairPlan)
+    if (lane >= PPW * G)
+      for (int i = l; i < LS; i += PP::IDLE) ln[i] = mk<T>(T(0), T(0));
   }
   // Whether any line of the wave meets the mask.  The mask and us are read
   // through buffers, whose out-of-range offset stands for "not needed"; a line
