@@ -103,8 +103,7 @@ struct XPassArgs {
   // RHS extras
   const void* mask;    // N reals (element type of the pass)
   const void* us;      // 3N reals, component stride N
-  const uint8_t* mflag;  // per x line (ny*nz): 0 where the line's mask is all zero; null: read every line
-  const void* mzero;   // nx zeros of the element type, read instead of a line whose flag is 0
+  const uint8_t* mflag;  // per x line (ny*nz): 0 where the line's mask is all zero (not read); null: read every line
   long npts;           // N
   double eps_inv;      // 1/eta
   int sponge;          // 0 none, 1 cavity, 2 outlet_x

@@ -258,9 +258,8 @@ class Solver : public SolverBase {
   uint8_t* color = nullptr;
   // per x line: may the mask be nonzero (the x pass reads only those lines'
   // mask); valid after an unbatched, uncaptured insect mask update, which
-  // recomputes the lines it redrew
+  // recomputes the lines it redrew, and for a mask that no step redraws
   uint8_t* mflag = nullptr;
-  void* mzero = nullptr;
   bool mflag_valid = false;
   bool mflag_on = true;     // FLUSI_MASK_FLAGS=0: every line's mask is read
   void* phys = nullptr;     // 7 real fields for diagnostics (u, w, div)
@@ -584,7 +583,6 @@ class Solver : public SolverBase {
   // kernel variants (chosen by autotune(), or by the FLUSI_* environment overrides)
   bool twave = true;        // y/z passes with the line transform inside one wavefront
   bool tpf = true;          // block y/z passes: prefetch the next job's operand
-  int xwpe = FP64 ? 0 : 3;  // reported with the variant; the x pass fixes its register budgets itself
   void tile(const TilePassArgs& a0, int L, int dir, bool contig_in) {
     TilePassArgs a = a0;
     a.pf = tpf ? 1 : 0;
@@ -712,7 +710,7 @@ class Solver : public SolverBase {
     if (out) a.kout = (int)std::min<long>(prowc, nxh);
     a.in = P; a.out = P; a.fstride_in = pc; a.fstride_out = pc; a.nf = 6;
     a.mask = mask; a.us = us; a.eps_inv = 1.0 / p.eps;
-    a.mflag = mflag_valid && batch_n(bat) == 1 ? mflag : nullptr; a.mzero = mzero;
+    a.mflag = mflag_valid && batch_n(bat) == 1 ? mflag : nullptr;
     a.sponge = sponge_code();
     a.sponge_thickness = p.sponge_thickness;
     a.sponge_eps_inv = a.sponge ? 1.0 / p.eps_sponge : 0.0;
@@ -852,10 +850,10 @@ class Solver : public SolverBase {
   // every variant the grid allows and keeps the fastest; results are cached
   // per grid, precision, sponge, batch size, method and pruning for the life
   // of the process.
-  struct Variant { int twave, tpf, xwave, xwpe, zwave, zeu; };
-  Variant variant() const { return Variant{twave, tpf, xwave, xwpe, zwave, zeu}; }
+  struct Variant { int twave, tpf, xwave, zwave, zeu; };
+  Variant variant() const { return Variant{twave, tpf, xwave, zwave, zeu}; }
   void apply(const Variant& v) {
-    twave = v.twave != 0; tpf = v.tpf != 0; xwave = v.xwave != 0; xwpe = v.xwpe; zwave = v.zwave != 0; zeu = v.zeu;
+    twave = v.twave != 0; tpf = v.tpf != 0; xwave = v.xwave != 0; zwave = v.zwave != 0; zeu = v.zeu;
   }
   double time_rhs(int reps) {
     auto one = [&](bool in, bool out, bool first) {
@@ -898,7 +896,7 @@ class Solver : public SolverBase {
             if (zv && !zw) continue;
             for (int eu : {0, 2, 4}) {
               if (eu && (zv || nz < 256)) continue;  // grouping acts in the block z step at nz >= 256
-              c.push_back(Variant{tw, pf, xv, xwpe, zv, eu});
+              c.push_back(Variant{tw, pf, xv, zv, eu});
             }
           }
         }
@@ -917,7 +915,7 @@ class Solver : public SolverBase {
            (prunes() ? ":p" : "") + (p.dt_fixed <= 0.0 ? ":a" : "");
   }
   static constexpr int kVariantInts = 6;
-  // v: the chosen variant (6 ints: twave, tpf, xwave, xwpe, zwave, zeu); ms: its
+  // v: the chosen variant (6 ints: twave, tpf, xwave, 0, zwave, zeu); ms: its
   // time per right-hand side; force: tune again even when cached
   void autotune(int reps, int* v, double* ms, bool force) {
     need_fft();
@@ -944,7 +942,7 @@ class Solver : public SolverBase {
     apply(best.first);
     if (v) {
       const Variant& b = best.first;
-      const int o[6] = {b.twave, b.tpf, b.xwave, b.xwpe, b.zwave, b.zeu};
+      const int o[6] = {b.twave, b.tpf, b.xwave, 0, b.zwave, b.zeu};
       for (int i = 0; i < kVariantInts; ++i) v[i] = o[i];
     }
     if (ms) *ms = best.second;
@@ -1586,14 +1584,7 @@ class Solver : public SolverBase {
     launch_mask_flags<T>(mask, mflag, nx, ny, 0, ny - 1, 0, nz - 1, stream);
     mflag_valid = true;
   }
-  void alloc_mask_flags() {
-    if (!mflag) {
-      const size_t zb = (sizeof(T) * nx + 255) / 256 * 256;
-      mzero = dalloc(zb + (size_t)ny * nz);
-      mflag = (uint8_t*)mzero + zb;
-      launch_zero(mzero, zb, stream);
-    }
-  }
+  void alloc_mask_flags() { if (!mflag) mflag = (uint8_t*)dalloc((size_t)ny * nz); }
   // Line flags after an insect update: insect_k writes only inside its region
   // box, so lines outside it keep their flags; the lines crossing the box
   // (or every line, when the flags were not valid before) are recomputed

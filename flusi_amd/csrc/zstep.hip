@@ -16,6 +16,10 @@
 #include <stdexcept>
 #include <string>
 
+#ifndef FLUSI_PART
+#error "FLUSI_PART (0..3) selects the instantiations"
+#endif
+
 namespace flusi {
 
 __device__ __forceinline__ double vis_factor(double dtv, double nu, double k2, bool alias) {
@@ -697,7 +701,7 @@ __global__ __launch_bounds__(NT, zb_wpe<T>(L)) void zstep_k(ZStepArgs a) {
 }
 
 // The same pass with each z line transformed inside one wavefront (nz = 64,
-// 128, 256, 512): per field, TL lines' 128-byte ky segments are staged
+// 128, 256): per field, TL lines' 128-byte ky segments are staged
 // through the LDS tile (one block-wide wait each way), every wave transforms
 // its own line in registers, and the next field's loads are in flight
 // meanwhile.  A lane ends with positions kz = l + qG of all fields of its
@@ -965,9 +969,6 @@ static void run_z_sp(const ZStepArgs& a, hipStream_t s) {
 
 // The instantiations are compiled in four parts (build.py), by element type
 // and line length: 0, 1 - FP32, 2, 3 - FP64; the even parts up to nz = 128.
-#ifndef FLUSI_PART
-#error "FLUSI_PART (0..3) selects the instantiations"
-#endif
 template <typename T> void launch_zstep_short(const ZStepArgs& a, hipStream_t s);  // nz <= 128
 template <typename T> void launch_zstep_long(const ZStepArgs& a, hipStream_t s);
 using PartT = std::conditional_t<(FLUSI_PART < 2), float, double>;

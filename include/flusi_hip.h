@@ -168,9 +168,9 @@ int flusi_timers(flusi_ctx* ctx, int enable, double* ms, const char** names);
  * them, for every variant the grid allows and keeps the fastest for this
  * context; results are cached per grid, precision, batch size and method for
  * the life of the process.
- * variant[6] (may be NULL): in-wave y/z passes, block-pass prefetch, one-wave
- * x pass, its waves-per-SIMD register budget, in-wave z step, epilogue
- * positions the block z step schedules together (0 = all).  ms: time of one
+ * variant[6] (may be NULL): in-wave y/z passes, block-pass prefetch, in-wave x
+ * pass, 0 (unused), in-wave z step, epilogue positions the block z step
+ * schedules together (0 = all).  ms: time of one
  * right-hand side with the chosen variant. */
 int flusi_autotune(flusi_ctx* ctx, int reps, int* variant, double* ms);
 
