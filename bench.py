@@ -287,6 +287,7 @@ def run_ensemble(args):
     best = max(per_pass, key=lambda k: per_pass[k])
     nlaunch = 2 * k_eager * len(leads)
     ach = per_bytes[best] / (per_pass[best] / 1e3)
+    step_bytes = sum(per_size * n ** 3 * step_bytes_per_point(n, 4, "RK2") for n in sizes)  # of all members
     out = {
         "metric": ENS_METRIC, "value": value, "unit": "grid-pt·steps/s", "n_gpus": 1,
         "steps": args.steps, "warmup": args.warmup, "ms_per_step": 1e3 * dt / args.steps,
@@ -299,7 +300,7 @@ def run_ensemble(args):
                      "frac": ach / HBM_PEAK, "traffic": None, "kernel": best,
                      "algorithmic_bytes_per_launch": per_bytes[best] / nlaunch,
                      "avg_launch_ms": per_pass[best] / nlaunch},
-        "step_roofline_frac": step_bytes_per_point(128, 4, "RK2") * value / HBM_PEAK,
+        "step_roofline_frac": step_bytes * args.steps / dt / HBM_PEAK,
         "batched_eager_gps": pts * k_eager / dt_eager,
         "members_alone_gps": pts / dt_members,
         "pass_ms_per_step": {k: v / k_eager for k, v in per_pass.items()},
