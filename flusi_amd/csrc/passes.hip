@@ -35,7 +35,11 @@ namespace flusi {
 // transforms (e.g. u and i k u).  The next job's loads are issued as soon as
 // the current operands have been consumed, so they are in flight while the
 // LDS stages of the current transform run.
-template <typename T, int L, int TL, int NT, int S, bool CONTIG_IN, bool PF>
+//
+// PR: the pass is pruned (a.prune).  Full passes have kernels of their own: on
+// the small grids that run them the region's tests were 4-6 % of a step (RK2,
+// FP32 32^3 75.4 / 71.0 us, FP64 48^3 131 / 125, FP32 64x32x96 110 / 105).
+template <typename T, int L, int TL, int NT, int S, bool CONTIG_IN, bool PF, bool PR>
 __global__ __launch_bounds__(NT) void tile_pass_k(TilePassArgs a) {
   constexpr int NSTG = plan_count_k(PLAN_TILE, L);
   static_assert(NSTG >= 2, "tile pass needs at least two stages");
@@ -49,7 +53,7 @@ __global__ __launch_bounds__(NT) void tile_pass_k(TilePassArgs a) {
   cplx<T>* buf = reinterpret_cast<cplx<T>*>(smem_raw);
   const int tid = threadIdx.x;
   int b0 = blockIdx.x * TL, c = blockIdx.y;
-  if (a.tiles) {  // the tiles that meet the dealiased region
+  if (PR && a.tiles) {  // the tiles that meet the dealiased region
     const uint32_t t = ((gptr<const uint32_t>)a.tiles)[blockIdx.x];
     b0 = (int)(t & 0xffffu) * TL;
     c = (int)(t >> 16);
@@ -76,24 +80,28 @@ __global__ __launch_bounds__(NT) void tile_pass_k(TilePassArgs a) {
         const int b = b0 + bb;
         int lim = b < a.nb ? L : -1, row = b;
         unsigned lo = 0, hi = 0;
-        if (CONTIG_IN && a.prune == PR_ZINV) {
+        if (PR && CONTIG_IN && a.prune == PR_ZINV) {
           lim = ((gptr<const int16_t>)a.pr.zlim)[c * a.pr.nyp + b];
           row = b - a.pr.ym0;
           if (row < 0) row += a.nb;
-        } else if (CONTIG_IN && a.prune == PR_YINV) {
+        } else if (PR && CONTIG_IN && a.prune == PR_YINV) {
           lim = b < a.nb ? ((gptr<const int16_t>)a.pr.ylim)[b] : -1;
           lo = a.pr.ym0;
           hi = (unsigned)(a.pr.ym0 - L);
         }
         const unsigned base = CONTIG_IN ? (unsigned)c * (unsigned)a.sin.c + (unsigned)row * (unsigned)a.sin.b
                                         : (unsigned)c * (unsigned)a.sin.c + (unsigned)b;
+        // byte offset of position 0 on the contiguous side of a full pass (kOob + a line is out of range, too)
+        const unsigned line0 = lim >= 0 ? (base + (unsigned)j) * ES : kOob;
 #pragma unroll
         for (int q = 0; q < R0; ++q) {
           const int aa = j + q * (L / R0);
           unsigned off;
-          if (CONTIG_IN) {
+          if (CONTIG_IN && PR) {
             const bool up = aa >= L / 2;
             off = (up ? L - aa : aa) <= lim ? (base + aa + (up ? hi : lo)) * ES : kOob;
+          } else if (CONTIG_IN) {
+            off = line0 + q * (L / R0) * ES;
           } else {
             off = lim >= 0 ? (base + (unsigned)aa * (unsigned)a.sin.a) * ES : kOob;
           }
@@ -172,7 +180,7 @@ __global__ __launch_bounds__(NT) void tile_pass_k(TilePassArgs a) {
           const unsigned base = !CONTIG_IN ? (unsigned)c * (unsigned)a.sout.c + (unsigned)b * (unsigned)a.sout.b
                                            : (unsigned)c * (unsigned)a.sout.c + (unsigned)b;
           int plo = 0, phi = 0;  // PR_YFWD: compact positions written (see tile_wave_k)
-          if (!CONTIG_IN && a.prune == PR_YFWD) {
+          if (PR && !CONTIG_IN && a.prune == PR_YFWD) {
             constexpr int SEG = 128 / ES;
             const int ym = ok ? ((gptr<const int16_t>)a.pr.ylim)[b] : -1;
             plo = (a.pr.ym0 - ym) & ~(SEG - 1);
@@ -182,7 +190,7 @@ __global__ __launch_bounds__(NT) void tile_pass_k(TilePassArgs a) {
           for (int q = 0; q < RL; ++q) {
             const int aa = j + q * (L / RL);
             unsigned off;
-            if (!CONTIG_IN && a.prune == PR_YFWD) {
+            if (PR && !CONTIG_IN && a.prune == PR_YFWD) {
               const int pp = a.pr.ym0 + (aa < L / 2 ? aa : aa - L);
               off = pp >= plo && pp < phi ? (base + (unsigned)pp) * ES : kOob;
             } else {
@@ -197,15 +205,22 @@ __global__ __launch_bounds__(NT) void tile_pass_k(TilePassArgs a) {
   }
 }
 
-template <typename T, int L, int S, bool CI, bool PF>
-static void run_tile_pf(const TilePassArgs& a, hipStream_t s) {
+template <typename T, int L, int S, bool CI, bool PF, bool PR>
+static void run_tile_pr(const TilePassArgs& a, hipStream_t s) {
   constexpr int TL = Tile<T>::TL;
   constexpr int NT = pick_nt(TL * L);
   const size_t smem = sizeof(cplx<T>) * TL * line_stride<T>(L);
   static bool init = false;
-  if (!init) { set_smem(tile_pass_k<T, L, TL, NT, S, CI, PF>, smem); init = true; }
-  const dim3 grid = a.tiles ? dim3(a.ntiles, 1, batch_n(a.bat)) : dim3((a.nb + TL - 1) / TL, a.nc, batch_n(a.bat));
-  hipLaunchKernelGGL((tile_pass_k<T, L, TL, NT, S, CI, PF>), grid, dim3(NT), smem, s, a);
+  if (!init) { set_smem(tile_pass_k<T, L, TL, NT, S, CI, PF, PR>, smem); init = true; }
+  const dim3 grid = PR && a.tiles ? dim3(a.ntiles, 1, batch_n(a.bat)) : dim3((a.nb + TL - 1) / TL, a.nc, batch_n(a.bat));
+  hipLaunchKernelGGL((tile_pass_k<T, L, TL, NT, S, CI, PF, PR>), grid, dim3(NT), smem, s, a);
+}
+template <typename T, int L, int S, bool CI, bool PF>
+static void run_tile_pf(const TilePassArgs& a, hipStream_t s) {
+  if constexpr (CI == (S > 0)) {  // the pruned passes: inverse from lines, forward to lines
+    if (a.prune) { run_tile_pr<T, L, S, CI, PF, true>(a, s); return; }
+  }
+  run_tile_pr<T, L, S, CI, PF, false>(a, s);
 }
 template <typename T, int L, int S, bool CI>
 static void run_tile(const TilePassArgs& a, hipStream_t s) {
@@ -240,6 +255,7 @@ void launch_tile_pass(const TilePassArgs& a, int L, int dir, bool ci, hipStream_
   const bool unit = ci ? (a.sin.a == 1 && a.sout.b == 1) : (a.sin.b == 1 && a.sout.a == 1);
   if (!unit) throw std::runtime_error("tile pass: the contiguous axes must have unit stride");
   if (a.njobs < 1 || a.njobs > 6) throw std::runtime_error("tile pass: 1..6 jobs");
+  if (a.prune && ci != (dir > 0)) throw std::runtime_error("tile pass: no such pruned pass");
   if (a.ibytes >= kOob || a.obytes >= kOob) throw std::runtime_error("tile pass: field too large for 32-bit offsets");
   switch (L) {
     case 16: run_tile_dir<T, 16>(a, dir, ci, s); break;
