@@ -294,7 +294,12 @@ __host__ __device__ constexpr int x_threads(int nb) { return nb >= 256 ? 256 : (
 //   D  inverse last stage -> u x w - chi (u - us) [+ sponge] -> forward
 //      stage 0, all in registers (PLAN_XI ends with the radix PLAN_XF starts with)
 //   E  forward remaining stages (LDS), split into nx/2+1 entries, store
-template <typename T, int M, int TLX, int NT, int MODE, int NFI, int NFO, bool SPONGE>
+//
+// PR: kin or kout may leave entries out.  The forward transforms never do, and
+// nx = 16, which this pass alone serves, mostly does not: kernels without
+// those tests (16x512x512 FP32 right-hand side 146 / 137 us, FP64 16x64x64 80 / 74
+// per RK4 step).
+template <typename T, int M, int TLX, int NT, int MODE, int NFI, int NFO, bool SPONGE, bool PR>
 __global__ __launch_bounds__(NT) void x_pass_k(XPassArgs a) {
   to_member(a, blockIdx.y);
   constexpr int NST = plan_count_k(PLAN_XF, M);
@@ -324,7 +329,7 @@ __global__ __launch_bounds__(NT) void x_pass_k(XPassArgs a) {
         const int line = e / nxh, k = e - line * nxh;
         const int gl = l0 + line;
         cplx<T> v = mk<T>(T(0), T(0));
-        if (gl < a.nlines && k < a.kin) v = gld<T>(in + f * a.fstride_in + (long)gl * a.prow + k);
+        if (gl < a.nlines && (!PR || k < a.kin)) v = gld<T>(in + f * a.fstride_in + (long)gl * a.prow + k);
         L_(f, line)[lp<T>(k)] = v;
       }
     __syncthreads();
@@ -558,8 +563,8 @@ __global__ __launch_bounds__(NT) void x_pass_k(XPassArgs a) {
       const cplx<T> zm = L_(f, line)[lp<T>(k2 == M ? 0 : k2)];
       const cplx<T> s1 = add(zk, conj_(zm)), d1 = sub(zk, conj_(zm));
       const gptr<cplx<T>> o = out + f * a.fstride_out + (long)gl * a.prow;
-      if (k < a.kout) gst<T>(o + k, scl(sub(s1, ik_<T>(T(1), cmul(wa, d1))), half));
-      if (k2 != k && k2 < a.kout) {
+      if (!PR || k < a.kout) gst<T>(o + k, scl(sub(s1, ik_<T>(T(1), cmul(wa, d1))), half));
+      if (k2 != k && (!PR || k2 < a.kout)) {
         const cplx<T> s2 = add(zm, conj_(zk)), d2 = sub(zm, conj_(zk));
         gst<T>(o + k2, scl(sub(s2, ik_<T>(T(1), cmul(wb, d2))), half));
       }
@@ -573,16 +578,25 @@ int x_pass_blocks(int nx, int nlines, bool fp64) {
   return (nlines + t - 1) / t;
 }
 
-template <typename T, int M, int MODE, int NFI, int NFO, bool SP>
-static void run_x(const XPassArgs& a, hipStream_t s) {
+template <typename T, int M, int MODE, int NFI, int NFO, bool SP, bool PR>
+static void run_x_pr(const XPassArgs& a, hipStream_t s) {
   constexpr int TLX = xtlx(M, XTile<T>::W);
   constexpr int NT = x_threads(TLX * (M / plan_radix_k(PLAN_XF, M, 0)));
   constexpr int NF = NFI > NFO ? NFI : NFO;
   const size_t smem = sizeof(cplx<T>) * (size_t)NF * TLX * line_stride<T>(M + 1);
   static bool init = false;
-  if (!init) { set_smem(x_pass_k<T, M, TLX, NT, MODE, NFI, NFO, SP>, smem); init = true; }
+  if (!init) { set_smem(x_pass_k<T, M, TLX, NT, MODE, NFI, NFO, SP, PR>, smem); init = true; }
   const int blocks = (a.nlines + TLX - 1) / TLX;
-  hipLaunchKernelGGL((x_pass_k<T, M, TLX, NT, MODE, NFI, NFO, SP>), dim3(blocks, batch_n(a.bat)), dim3(NT), smem, s, a);
+  hipLaunchKernelGGL((x_pass_k<T, M, TLX, NT, MODE, NFI, NFO, SP, PR>), dim3(blocks, batch_n(a.bat)), dim3(NT), smem, s, a);
+}
+
+template <typename T, int M, int MODE, int NFI, int NFO, bool SP>
+static void run_x(const XPassArgs& a, hipStream_t s) {
+  if constexpr (MODE == XM_FWD || M == 8) {
+    if (a.kin == M + 1 && a.kout == M + 1) { run_x_pr<T, M, MODE, NFI, NFO, SP, false>(a, s); return; }
+    if constexpr (MODE == XM_FWD) throw std::runtime_error("x forward pass: writes every entry");
+  }
+  if constexpr (MODE != XM_FWD) run_x_pr<T, M, MODE, NFI, NFO, SP, true>(a, s);
 }
 
 template <typename T, int M>
