@@ -40,8 +40,13 @@ template <typename T, int L> struct TWShape {
   static constexpr int NT = NW * 64;
   static constexpr int LS = line_stride<T>(L);
   static constexpr int K = TL * L / NT;              // tile elements per thread (E)
-  // twiddles in LDS when two blocks still fit in 160 KB
-  static constexpr bool TWL = 2 * (TL * LS + L) * (int)sizeof(cplx<T>) <= 160 * 1024;
+  // twiddles in LDS when two blocks still fit in 160 KB, and where the
+  // registers hold one block to a compute unit anyway (FP64, L = 512: eight
+  // waves of 168): from global memory each of the 14 a lane needs was waited
+  // for by itself, and every such wait also covered the prefetched operands
+  // (128x512x512 FP64 RK4 step, z / y inverse / y forward 685 / 1693 / 974 us,
+  // from LDS 527 / 1303 / 743)
+  static constexpr bool TWL = (sizeof(T) == 8 && L == 512) || 2 * (TL * LS + L) * (int)sizeof(cplx<T>) <= 160 * 1024;
   static constexpr size_t smem = (size_t)(TL * LS + (TWL ? L : 0)) * sizeof(cplx<T>);
 };
 
