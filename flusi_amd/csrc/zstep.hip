@@ -118,9 +118,9 @@ struct ZLim {
   __device__ __forceinline__ bool in(int kzi, int nz) const { return (kzi < (nz >> 1) ? kzi : nz - kzi) <= zm; }
   __device__ __forceinline__ bool out(int kzi) const { return kzi < up || kzi >= dn; }
 };
-template <typename T> __device__ __forceinline__ ZLim zlim_at(const ZStepArgs& a, int kx, int p) {
+template <typename T, bool PR> __device__ __forceinline__ ZLim zlim_at(const ZStepArgs& a, int kx, int p) {
   ZLim z{a.nz, a.nz, 0};
-  if (a.prune) {
+  if (PR && a.prune) {
     z.zm = (kx < a.pr.nkx && p >= 0 && p < a.pr.nyp) ? a.pr.zlim[kx * a.pr.nyp + p] : -1;
     if (a.prune & 2) {
       constexpr int SEG = 128 / (int)sizeof(cplx<T>);
@@ -131,8 +131,8 @@ template <typename T> __device__ __forceinline__ ZLim zlim_at(const ZStepArgs& a
   return z;
 }
 // the ky index of tile line b: compact Q rows hold ky = b - ym0
-__device__ __forceinline__ int zrow(const ZStepArgs& a, int b) {
-  if (!(a.prune & 2)) return b;
+template <bool PR> __device__ __forceinline__ int zrow(const ZStepArgs& a, int b) {
+  if (!PR || !(a.prune & 2)) return b;
   const int ky = b - a.pr.ym0;
   return ky < 0 ? ky + a.ny : ky;
 }
@@ -141,7 +141,7 @@ __device__ __forceinline__ int zpos(const ZStepArgs& a, int row) {
   return a.pr.ym0 + (row < (a.ny + 1) / 2 ? row : row - a.ny);
 }
 // row length of Q and number of lines of the tile axis
-__device__ __forceinline__ int zq_lines(const ZStepArgs& a) { return (a.prune & 2) ? a.pr.nyp : a.ny; }
+template <bool PR> __device__ __forceinline__ int zq_lines(const ZStepArgs& a) { return (PR && (a.prune & 2)) ? a.pr.nyp : a.ny; }
 
 // Epilogue at one spectral point (kx, ky, kz): rv[f] is field f of the
 // z-transformed right-hand side (unscaled).  Sponge curl (sponge.f90:22-83),
@@ -441,7 +441,8 @@ template <typename T, int L, int TL> struct ZBShape {
 // EU > 0: the epilogue of at most EU positions is scheduled together (a
 // scheduling barrier after every EU positions keeps the compiler from
 // hoisting all positions' state loads)
-template <typename T, int L, int TL, int NT, bool SPONGE, int MG, int EU>
+// PR: the launch may be pruned (a.prune); see run_zb.
+template <typename T, int L, int TL, int NT, bool SPONGE, int MG, int EU, bool PR>
 __global__ __launch_bounds__(NT, zb_wpe<T>(L)) void zstep_k(ZStepArgs a) {
   const MOff mo = member_off<T>(a);
   constexpr int NSTG = plan_count_k(PLAN_TILE, L);
@@ -460,14 +461,14 @@ __global__ __launch_bounds__(NT, zb_wpe<T>(L)) void zstep_k(ZStepArgs a) {
   // workgroups x and x + 8 of a row run on one XCD one after the other; they
   // take neighbouring ky tiles, whose Q segments share 128-byte lines.
   int bx = blockIdx.x;
-  if (TL * sizeof(cplx<T>) < 128 && gridDim.x % 8 == 0 && !a.tiles) bx = (bx % 8) * (gridDim.x / 8) + bx / 8;
+  if (TL * sizeof(cplx<T>) < 128 && gridDim.x % 8 == 0 && !(PR && a.tiles)) bx = (bx % 8) * (gridDim.x / 8) + bx / 8;
   int b0 = bx * TL, kx = blockIdx.y;
-  if (a.tiles) {  // the tiles that meet the dealiased region, in the same order
+  if (PR && a.tiles) {  // the tiles that meet the dealiased region, in the same order
     const uint32_t t = a.tiles[blockIdx.x];
     b0 = (int)(t & 0xffffu) * TL;
     kx = (int)(t >> 16);
   }
-  const int nyq = zq_lines(a);
+  const int nyq = zq_lines<PR>(a);
   constexpr bool PARK = ZBShape<T, L, TL>::park;
   // fixed-mode kernels load each epilogue position's operands one position
   // ahead (ZPre); without the sponge, field 2 then waits in the transform tile
@@ -624,7 +625,7 @@ __global__ __launch_bounds__(NT, zb_wpe<T>(L)) void zstep_k(ZStepArgs a) {
 #pragma unroll
             for (int q = 0; q < RL; ++q) {
               cplx<T> s0 = PARK ? pk[lp<T>(j + q * (L / RL))] : r[0][p][q];
-              sponge_term<T>(a, mo, kxs, b0 + bb < nyq ? zrow(a, b0 + bb) : a.ny, j + q * (L / RL), s0, r[1][p][q], r[2][p][q]);
+              sponge_term<T>(a, mo, kxs, b0 + bb < nyq ? zrow<PR>(a, b0 + bb) : a.ny, j + q * (L / RL), s0, r[1][p][q], r[2][p][q]);
               if constexpr (PARK) pk[lp<T>(j + q * (L / RL))] = s0;
               else r[0][p][q] = s0;
               __builtin_amdgcn_sched_barrier(0);  // one position at a time
@@ -664,8 +665,8 @@ __global__ __launch_bounds__(NT, zb_wpe<T>(L)) void zstep_k(ZStepArgs a) {
   for (int p = 0; p < PERL; ++p) {
     int bb, kzi;
     const bool ok = at(p * RL, bb, kzi);
-    row[p] = ok ? zrow(a, b0 + bb) : 0;
-    zl[p] = zlim_at<T>(a, kx, (a.prune & 2) ? b0 + bb : zpos(a, row[p]));
+    row[p] = ok ? zrow<PR>(a, b0 + bb) : 0;
+    zl[p] = zlim_at<T, PR>(a, kx, (a.prune & 2) ? b0 + bb : zpos(a, row[p]));
     if (!ok) zl[p] = ZLim{-1, 0, a.nz};
   }
   // operands of position k
@@ -673,7 +674,7 @@ __global__ __launch_bounds__(NT, zb_wpe<T>(L)) void zstep_k(ZStepArgs a) {
   auto preload = [&](int k, ZPre<T>& pr) {
     int bb, kzi;
     const int p = k / RL;
-    const bool ok = at(k, bb, kzi) && zl[p].in(kzi, a.nz);
+    const bool ok = at(k, bb, kzi) && (!PR || zl[p].in(kzi, a.nz));
     const unsigned off = ok ? (((unsigned)kx * a.ny + row[p]) * a.nz + kzi) * (unsigned)sizeof(cplx<T>) : kOob;
     zpreload<T, MG>(a, mo, off, row[p], kzi, pr);
   };
@@ -684,13 +685,13 @@ __global__ __launch_bounds__(NT, zb_wpe<T>(L)) void zstep_k(ZStepArgs a) {
       if (k + 1 < NPOS) preload(k + 1, pre[(k + 1) & 1]);
     int bb, kzi;
     const int p = k / RL, q = k % RL;
-    if (!at(k, bb, kzi) || !zl[p].out(kzi)) continue;
+    if (!at(k, bb, kzi) || (PR && !zl[p].out(kzi))) continue;
     cplx<T> rv[3];
 #pragma unroll
     for (int f = 0; f < 3; ++f)
       rv[f] = (PARK && f == 0) ? park[bb * LSP + lp<T>(kzi)] : ((TILE2 && f == 2) ? buf[bb * LSP + lp<T>(kzi)] : r[f][p][q]);
     zepilogue<T, false, MG, SPONGE>(a, mo, kx, row[p], kzi, rv, kxv, kxt2, wE, final_stage, esum, ecomp,
-                                    zl[p].in(kzi, a.nz), &pre[k & 1]);
+                                    !PR || zl[p].in(kzi, a.nz), &pre[k & 1]);
     if constexpr (EU > 0)
       if ((k + 1) % EU == 0) __builtin_amdgcn_sched_barrier(0);
   }
@@ -701,7 +702,7 @@ __global__ __launch_bounds__(NT, zb_wpe<T>(L)) void zstep_k(ZStepArgs a) {
     if (tid == 0) {
       double s = 0.0;
       for (int w = 0; w < NT / 64; ++w) s += red[w];
-      a.energy_partial[mo.md + (a.tiles ? (long)blockIdx.x : (long)blockIdx.y * gridDim.x + bx)] = s;
+      a.energy_partial[mo.md + (PR && a.tiles ? (long)blockIdx.x : (long)blockIdx.y * gridDim.x + bx)] = s;
     }
   }
 }
@@ -742,7 +743,7 @@ __global__ __launch_bounds__((ZWShape<T, L>::NT)) void zstep_wave_k(ZStepArgs a)
     b0 = (int)(t & 0xffffu) * TL;
     kx = (int)(t >> 16);
   }
-  const int nyq = zq_lines(a);
+  const int nyq = zq_lines<true>(a);
   // twiddles: the block's LDS copy (made after the first field's loads are
   // issued, so that the two memory latencies overlap; first read after the
   // first block barrier), or global memory where it does not fit
@@ -820,7 +821,7 @@ __global__ __launch_bounds__((ZWShape<T, L>::NT)) void zstep_wave_k(ZStepArgs a)
         if constexpr (i == 2) {
           const double kxs = a.kx[kx + mo.md];
 #pragma unroll
-          for (int q = 0; q < 8; ++q) sponge_term<T>(a, mo, kxs, b0 + line < nyq ? zrow(a, b0 + line) : a.ny, l + q * G, r[0][q], r[1][q], r[2][q]);
+          for (int q = 0; q < 8; ++q) sponge_term<T>(a, mo, kxs, b0 + line < nyq ? zrow<true>(a, b0 + line) : a.ny, l + q * G, r[0][q], r[1][q], r[2][q]);
         }
       } else {
 #pragma unroll
@@ -842,8 +843,8 @@ __global__ __launch_bounds__((ZWShape<T, L>::NT)) void zstep_wave_k(ZStepArgs a)
   double esum = 0.0, ecomp = 0.0;
   const bool final_stage = mg_final_stage<MG>(a);
   if (b0 + line < nyq) {
-    const int ky = zrow(a, b0 + line);
-    const ZLim zl = zlim_at<T>(a, kx, (a.prune & 2) ? b0 + line : zpos(a, ky));
+    const int ky = zrow<true>(a, b0 + line);
+    const ZLim zl = zlim_at<T, true>(a, kx, (a.prune & 2) ? b0 + line : zpos(a, ky));
     // fixed-mode kernels: operands loaded one position ahead (ZPre)
     constexpr bool AHEAD = MG >= MG_FIXED;
     ZPre<T> pre[2];
@@ -895,15 +896,26 @@ int zstep_blocks(int nz, int ny, int nxh, bool fp64, bool wave) {
 
 #endif
 
-template <typename T, int L, bool SP, int MG, int EU>
-static void run_zb(const ZStepArgs& a, hipStream_t s) {
+template <typename T, int L, bool SP, int MG, int EU, bool PR>
+static void run_zb_pr(const ZStepArgs& a, hipStream_t s) {
   constexpr int TL = zb_tl<T>(L);
   constexpr int NT = pick_nt(TL * L);
   const size_t smem = ZBShape<T, L, TL>::smem;
   static bool init = false;
-  if (!init) { set_smem(zstep_k<T, L, TL, NT, SP, MG, EU>, smem); init = true; }
-  const dim3 grid = a.tiles ? dim3(a.ntiles, 1, batch_n(a.bat)) : dim3((a.ny + TL - 1) / TL, a.nxh, batch_n(a.bat));
-  hipLaunchKernelGGL((zstep_k<T, L, TL, NT, SP, MG, EU>), grid, dim3(NT), smem, s, a);
+  if (!init) { set_smem(zstep_k<T, L, TL, NT, SP, MG, EU, PR>, smem); init = true; }
+  const dim3 grid = PR && a.tiles ? dim3(a.ntiles, 1, batch_n(a.bat)) : dim3((a.ny + TL - 1) / TL, a.nxh, batch_n(a.bat));
+  hipLaunchKernelGGL((zstep_k<T, L, TL, NT, SP, MG, EU, PR>), grid, dim3(NT), smem, s, a);
+}
+
+// One kernel serves pruned and full launches, except in FP32 at nz = 512, held
+// to 128 registers: there the steppers' full launches have kernels without
+// the region's limits (AB2: with them it spills; 16x512x512 73 us, 66 without).
+template <typename T, int L, bool SP, int MG, int EU>
+static void run_zb(const ZStepArgs& a, hipStream_t s) {
+  if constexpr (sizeof(T) == 4 && L == 512 && MG >= MG_FIXED) {
+    if (!a.prune) { run_zb_pr<T, L, SP, MG, EU, false>(a, s); return; }
+  }
+  run_zb_pr<T, L, SP, MG, EU, true>(a, s);
 }
 
 template <typename T, int L, bool SP, int MG>
