@@ -1505,7 +1505,7 @@ class Solver : public SolverBase {
     // the mask changes below; the line flags are brought up to date only by
     // the unbatched, uncaptured insect update
     const bool flags_were_valid = mflag_valid;
-    mflag_valid = false;
+    mflag_valid = mflag_valid && p.iPenalization != 1;  // (nothing is drawn then)
     timed(TM_MASK, [&] {
       if (p.iPenalization == 1) {
         if (p.iMask == "sphere" || p.iMask == "Sphere") {
