@@ -15,7 +15,8 @@
 // -> 0.8 ms), but beside a program whose own thread pool still spins on every
 // core after its last parallel loop, a thread of this copy can wait a time
 // slice of a few milliseconds for a core (three 19 MB copies of a host
-// program between conversions of its own: 3.1 -> 6.4 ms with threads).
+// program between conversions of its own: 3.1 -> 6.4 ms with threads).  Slots
+// driven by the calling thread alone were not measured.
 //
 // The pinned slots cost 4 ms (64 MB) when they are made, once while contexts of
 // a device live.  Copies out regain that at once.  Copies in do only from some
