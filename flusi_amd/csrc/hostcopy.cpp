@@ -18,10 +18,12 @@
 // program between conversions of its own: 3.1 -> 6.4 ms with threads).  Slots
 // driven by the calling thread alone were not measured.
 //
-// The pinned slots cost 4 ms (64 MB) when they are made, once while contexts of
-// a device live.  Copies out regain that at once.  Copies in do only from some
-// size on (kMakeIn): a smaller one that finds no slots is left to the plain
-// copy once, for a program that sets one state and steps on (50 MB of FP64: in
+// The pinned slots cost 4 ms (64 MB) when they are made and first touched, once
+// while contexts of a device live.  Copies out into fresh arrays regain that at
+// once (into arrays touched before they do not: 115 MB of an FP32 field, whose
+// first copy took 2 ms more than a plain one).  Copies in do only from some size
+// on (kMakeIn): a smaller one that finds no slots is left to the plain copy
+// once, for a program that sets one state and steps on (50 MB of FP64: in
 // 1.8 ms plain, 5.1 ms with the slots to be made, 1.4 ms with slots there).
 #include "hostcopy.h"
 #include <algorithm>
