@@ -1031,10 +1031,12 @@ class Solver : public SolverBase {
   // Whether steps are pruned: RK4 dealiases always, AB2 and RK2 with iDealias.
   // The smallest grids are bound by their launches and the latency of each
   // pass, which the region's tables add a load to (us per step, full/pruned:
-  // 32^3 FP64 AB2 51.5/52.4, RK2 102/109, FP32 RK2 111/123; 48^3 AB2 81/73,
-  // RK2 158/160, FP32 AB2 69/68, RK2 133/147; 64^3 AB2 57/51, RK2 107/101,
-  // FP32 51/49, 99/97): AB2 and RK4 gain from 48^3 on, RK2, pruned on one
-  // side of each right-hand side, from 64^3.
+  // 32^3 FP64 AB2 34/36, RK2 67/70, FP32 RK2 71/76; 48^3 FP64 AB2 64/63, RK2
+  // 125/125, FP32 AB2 53/55, RK2 105/108; 64^3 FP64 AB2 52/47, RK2 101/97, FP32
+  // AB2 44/44, RK2 85/87; 96^3 FP32 AB2 85/73, RK2 159/156).  A batch gains
+  // earlier (eight members, FP32: 48^3 RK2 219/214, RK4 407/375; 64^3 RK2
+  // 260/237, RK4 512/393), and a member takes the passes of its own run: AB2 and
+  // RK4 from 48^3 on, RK2, pruned on one side of each right-hand side, from 64^3.
   bool prunes() const {
     if (!prune_ok || !(p.method == "RK4" || p.iDealias == 1)) return false;
     return prune_any_size || npts >= (p.method == "RK2" ? 1L << 18 : 100000L);
